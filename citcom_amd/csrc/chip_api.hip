@@ -167,11 +167,6 @@ void do_gs(chip_ctx *c, int lev, V *d, const V *F, V *Ad, int sweeps, int guess,
         gs_xcd(S(c), L, BI, d, F, Ad, rhs, res, sweeps, guess, c->dots + D_XST, pg.a, pg.b);
         return;
     }
-    if (c->small_levels && c->gs_wg && gs_wg_ok<V>(L)) {
-        ProfGuard pg(c, 3, gs_bytes<V>(L) * L.g.nno * sweeps + mv_bytes<V>(L) * L.g.nno, lev);
-        gs_wg(S(c), L, BI, d, F, Ad, rhs, res, sweeps, guess, pg.a, pg.b);
-        return;
-    }
     if constexpr (sizeof(V) == 4) {
         if (c->box_gs && L.Kbox && sweeps > 0) {
             // sweeps alternate between d and the level's scratch; a sweep
@@ -187,6 +182,26 @@ void do_gs(chip_ctx *c, int lev, V *d, const V *F, V *Ad, int sweeps, int guess,
             do_matvec(c, lev, (const V *)src, Ad, rhs, res, src == d ? nullptr : d);
             return;
         }
+    }
+    const bool small = L.g.nno <= SMALL_NNO;
+    if (c->small_levels && L.planes.shape && (c->gs_wg || !small) && sweeps > 0) {
+        // joined colour passes: two launches a sweep; sweeps alternate between d and the level's scratch, as the boxes'
+        V *t;
+        if constexpr (sizeof(V) == sizeof(double)) t = L.tmp;
+        else t = L.tmpf;
+        const V *src = guess == 1 ? d : nullptr;
+        V *dst = guess == 1 ? t : d;
+        for (int cyc = 0; cyc < sweeps; cyc++) {
+            for (int jpar = 0; jpar < 2; jpar++) {
+                const int *cn = L.g.cn + 4 * jpar;
+                ProfGuard pg(c, small ? 3 : 1, gs_bytes<V>(L) * (cn[0] + cn[1] + cn[2] + cn[3]), lev);
+                gs_rect(S(c), L, BI, F, jpar, src, jpar ? (const V *)dst : src, dst, pg.a, pg.b);
+            }
+            src = dst;
+            dst = dst == d ? t : d;
+        }
+        do_matvec(c, lev, src, Ad, rhs, res, src == d ? nullptr : d);
+        return;
     }
     if (guess == 0) fill(S(c), d, V(0), 3L * L.g.nno);
     for (int cyc = 0; cyc < sweeps; cyc++)

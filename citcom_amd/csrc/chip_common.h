@@ -23,6 +23,8 @@ constexpr int KROW = 243;   // 3 rows x 27 neighbour nodes x 3 columns
 // inverse is 3 nno x 3 nno FP32 (243 MB at 8192), applied a few times per
 // multigrid call, factored in FP64 at every rebuild
 constexpr long DIRECT_MAX_DOF = 8192;
+// levels the option "gs_wg" is about, and below those of "xcd_gs"
+constexpr int SMALL_NNO = 1024;
 constexpr int GNX_SZ = 216; // Shape_function_dx: vpt[3*8*8] + ppt[3*8]
 constexpr int GDA_SZ = 11;  // Shape_function_dA: vpt[9] + ppt[2]
 constexpr int ECO_SZ = 13;  // COORD: centre[4] size[4] recip_size[4] area
@@ -54,6 +56,13 @@ constexpr int BOX_MAXSEG = 40;
 struct BoxPart {
     int n[3];
     unsigned short s[3][BOX_MAXSEG + 1];
+};
+
+// How a level's planes are cut into the workgroups of k_gs_rect: the
+// workgroup's shape (0: not for this level), strips of lines, segments of Wz
+// nodes along k (ns of them)
+struct RectPart {
+    int shape, Wz, nstrip, ns;
 };
 
 // arrival counter and XCD mask of a level's one-XCD smoother launches
@@ -97,6 +106,7 @@ struct Level {
     // FP32 copies for the mixed-precision cycle
     float *velf = nullptr, *resf = nullptr, *flf = nullptr, *delf = nullptr, *AUf = nullptr;
     float *BIf = nullptr;
+    RectPart planes{};       // joined colour passes (k_gs_rect)
     // one-XCD smoother state (levels gs_xcd_ok accepts)
     XcdBar *xbar = nullptr;
     // box smoother of the FP32 cycles: the partition, and the cycle's
@@ -157,8 +167,8 @@ struct chip_ctx {
     int solution_cycles = 0;
     bool built = false;      // operators constructed at least once
     bool use_graphs = true;  // replay multi_grid as a captured HIP graph
-    bool small_levels = true;  // single-workgroup smoother on small levels
-    bool gs_wg = true;         // ... including levels whose stiffness is read through L2
+    bool small_levels = true;  // small levels' own smoother kernels (k_gs_lds, k_gs_rect)
+    bool gs_wg = true;         // joined colour passes on levels of at most SMALL_NNO nodes
     bool xcd_gs = false;       // whole smoother calls of mid-size levels on one XCD (k_gs_xcd)
     // FP32 cycles: the levels between the exact (or affine) level and the
     // finest smoothed by boxes, one launch per sweep (option "box_gs")

@@ -31,19 +31,17 @@ void matvec(hipStream_t s, const Level &L, const V *u, V *Au, const V *rhs, V *r
 template <typename V>
 void gs_colour(hipStream_t s, const Level &L, const V *BI, int colour, V *d, const V *F, hipEvent_t e0 = nullptr,
                hipEvent_t e1 = nullptr);
+// the four colours of the planes of parity jpar, from dself (their nodes) and
+// dside (the planes between; null: zero) to dout
+RectPart rect_planes(const Geo &g);
+template <typename V>
+void gs_rect(hipStream_t s, const Level &L, const V *BI, const V *F, int jpar, const V *dself, const V *dside, V *dout,
+             hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // every sweep of a small level in one workgroup, then Ad = K d
 void gs_small(hipStream_t s, const Level &L, double *d, const double *F, double *Ad, int sweeps, int guess);
 // 1: the level's stiffness and vectors fit in LDS (gs_small), 0: one launch
 // per colour pass
 int gs_small_kind(const Level &L);
-// a whole gauss_seidel call in one workgroup with d in LDS and the FP32
-// stiffness read through L2, then Ad = K d (and res = rhs - Ad if res):
-// for levels gs_wg_ok accepts (small enough, no FP16 stiffness)
-template <typename V>
-bool gs_wg_ok(const Level &L);
-template <typename V>
-void gs_wg(hipStream_t s, const Level &L, const V *BI, V *d, const V *F, V *Ad, const V *rhs, V *res, int sweeps,
-           int guess, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // a whole gauss_seidel call as one launch of a few workgroups on one XCD,
 // colour passes separated by barriers through that XCD's L2 (k_gs_xcd), then
 // Ad = K d (and res = rhs - Ad); a nonzero *status after the launch means it

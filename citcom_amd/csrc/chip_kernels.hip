@@ -88,6 +88,11 @@ __device__ __forceinline__ void colour_kij(const Geo &g, int c, int q, int &k, i
     j = 2 * (t / nx) + ((c >> 2) & 1);
 }
 
+// colour-ordered index of node (k, i, j) of colour c (inverse of colour_kij)
+__device__ __forceinline__ int colour_index(const Geo &g, int c, int k, int i, int j) {
+    return g.cs[c] + (k >> 1) + g.cz[c] * ((i >> 1) + g.cx[c] * (j >> 1));
+}
+
 __device__ __forceinline__ int colour_of(const Geo &g, int q) {
     int c = 0;
 #pragma unroll
@@ -357,7 +362,7 @@ template <typename V, typename KT>
 __global__ void __launch_bounds__(192) k_matvec3(Geo g, const KT *__restrict__ K, const unsigned *__restrict__ NODE,
                                                  const V *__restrict__ u, V *__restrict__ Au,
                                                  const V *__restrict__ rhs, V *__restrict__ res,
-                                                 const V *__restrict__ BIs) {
+                                                 const V *__restrict__ BIs, V *__restrict__ ucopy) {
     __shared__ V Ts[2][27][64];   // [plane - 1][block * 3 + row][lane]
     const int lane = threadIdx.x & 63, P = threadIdx.x >> 6;
     const int q = xcd_tile(blockIdx.x, gridDim.x) * 64 + lane;
@@ -398,6 +403,11 @@ __global__ void __launch_bounds__(192) k_matvec3(Geo g, const KT *__restrict__ K
             for (int t = 0; t < 27; t++) Ts[P - 1][t][lane] = T[t];
     }
     __syncthreads();
+    if (P == 1 && col >= 0 && ucopy) {   // u copied to ucopy in the same launch
+        ucopy[3 * self] = u[3 * self];
+        ucopy[3 * self + 1] = u[3 * self + 1];
+        ucopy[3 * self + 2] = u[3 * self + 2];
+    }
     if (P != 0 || col < 0) return;
     V out[3] = {V(0), V(0), V(0)};
 #pragma unroll
@@ -517,12 +527,6 @@ void matvec(hipStream_t s, const Level &L, const V *u, V *Au, const V *rhs, V *r
                                ucopy);
         return;
     }
-    if (ucopy) {   // large levels: a copy launch of its own
-        if constexpr (sizeof(V) == 8)
-            copy(s, (double *)ucopy, (const double *)u, 3L * L.g.nno);
-        else
-            fcopy(s, (float *)ucopy, (const float *)u, 3L * L.g.nno);
-    }
     const int tiles = L.g.pitch / 64;   // the colour index space is whole 64-node tiles
     if constexpr (sizeof(V) == 4) {
         if (L.Kh) {
@@ -531,9 +535,9 @@ void matvec(hipStream_t s, const Level &L, const V *u, V *Au, const V *rhs, V *r
             auto kern = k_matvec3<V, _Float16>;
             if (e0)
                 hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, Kh, L.NODE, u, Au, rhs, res,
-                                      BIs);
+                                      BIs, ucopy);
             else
-                hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, Kh, L.NODE, u, Au, rhs, res, BIs);
+                hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, Kh, L.NODE, u, Au, rhs, res, BIs, ucopy);
             return;
         }
     }
@@ -541,9 +545,10 @@ void matvec(hipStream_t s, const Level &L, const V *u, V *Au, const V *rhs, V *r
     const float *K = L.K;
     auto kern = k_matvec3<V, float>;
     if (e0)
-        hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, K, L.NODE, u, Au, rhs, res, none);
+        hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, K, L.NODE, u, Au, rhs, res, none,
+                              ucopy);
     else
-        hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, K, L.NODE, u, Au, rhs, res, none);
+        hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, K, L.NODE, u, Au, rhs, res, none, ucopy);
 }
 template void matvec<double>(hipStream_t, const Level &, const double *, double *, const double *, double *,
                              hipEvent_t, hipEvent_t, double *);
@@ -624,6 +629,240 @@ template void gs_colour<double>(hipStream_t, const Level &, const double *, int,
                                 hipEvent_t);
 template void gs_colour<float>(hipStream_t, const Level &, const float *, int, float *, const float *, hipEvent_t,
                                hipEvent_t);
+
+// ---------------------------------------------------------------------------
+// Colour passes of one sweep joined into two launches, with the bits of the
+// 8-colour order.  Colour = (k&1) | (i&1) << 1 | (j&1) << 2 and a node couples
+// to its 26 neighbours only, so nodes two apart along any axis are
+// independent: all of colours 0-3 lie on even y-planes, where a plane sees
+// its two neighbours as they were before the sweep, and colours 4-7 on odd
+// ones; within a plane, colours 0-1 (4-5) lie on even x-lines and 2-3 (6-7)
+// on odd ones.
+//
+// A workgroup of k_gs_rect takes a strip of W lines of one plane, cut along k
+// into segments of Wz nodes, through the plane's four colours.  The odd lines
+// need the even line on either side updated, so it also updates the even line
+// past its strip and, at a cut, the nodes that later colours read, from the
+// sweep's input (din); it writes its own nodes only, to dout.
+//
+// A lane forms one row of one node.  Its 81 coefficients are requested at the
+// start; the sums of the planes dy = -1 and +1, whose entries no colour of the
+// launch changes, are formed by all wavefronts at once; only the plane dy = 0
+// is left for the chain of colours, one workgroup barrier each.  A node's own
+// entries are kept in registers, so its three rows need no barrier between
+// reading and writing them.
+//
+// Bound by the chain: launch, one load, four colours of LDS reads and sums.
+// FP64 vectors, a half sweep (four colours) against four launches of
+// k_gs_colour, without the gaps between launches: 4913 nodes (17x17x17) 8.1 us
+// against 18.4, 18513 (33x33x17) 9.8 against 18.5, 35937 (33x33x33) 11.0
+// against 18.9, 139425 (65x65x33) 31 against 30, 274625 (65x65x65) 73 against
+// 46: past one workgroup per CU the nodes computed twice and the LDS reads
+// cost more than the launches saved, and the level stays with k_gs_colour.
+// Shapes: narrow, a colour's 21 nodes in one wavefront, three lanes each
+// (four wavefronts, one a SIMD: 7.9 us where the wide shape takes 9.3); wide,
+// a colour's 64 nodes in three wavefronts, one a row (18513 nodes: 9.8 us
+// where narrow strips, two workgroups to some CUs, take 11.5).
+
+// row r of one plane's tree (absent neighbours have zero coefficients and
+// zero entries; adding the tree's empty slots changes no bit but a zero's sign)
+template <typename V>
+__device__ __forceinline__ V plane_sum_row(const float kv[27], const V uv[27]) {
+    V t[9];
+#pragma unroll
+    for (int b = 0; b < 9; b++) t[b] = kv[3 * b] * uv[3 * b] + kv[3 * b + 1] * uv[3 * b + 1] + kv[3 * b + 2] * uv[3 * b + 2];
+    return (((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) + t[8];
+}
+
+// the shape of a workgroup: nodes of a colour, W lines, HZ entries of one k
+// parity in the staged region
+template <bool WIDE_, int W_, int HZ_>
+struct RectShape {
+    static constexpr bool WIDE = WIDE_;
+    static constexpr int W = W_, HZ = HZ_, NL = W + 3, NODES = WIDE ? 64 : 21, WAVES = WIDE ? 12 : 4;
+    static constexpr int CH = (2 * HZ + 20) / 21;           // chunks of a staged line, 21 nodes each
+    static constexpr int BATCH = (3 * NL + WAVES - 1) / WAVES * CH;
+    static constexpr int LINE = 3 * 2 * HZ;                 // [component][k parity][k/2]
+};
+
+template <typename V, typename KT, class S>
+__global__ void __launch_bounds__(S::WAVES * 64, sizeof(V) == 8 || sizeof(KT) == 2 ? 3 : 4) k_gs_rect(Geo g, RectPart rp, int jpar, const KT *__restrict__ K,
+                                                           const V *__restrict__ BI, const V *__restrict__ F,
+                                                           const V *__restrict__ dself, const V *__restrict__ dside,
+                                                           V *__restrict__ dout) {
+    constexpr int W = S::W, HZ = S::HZ, NL = S::NL, LINE = S::LINE;
+    __shared__ __align__(16) V sd[3 * NL * LINE];   // [plane][line]
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ph = S::WIDE ? w / 3 : w;
+    const int seg = blockIdx.x, strip = blockIdx.y, j = 2 * blockIdx.z + jpar;
+    const int i0 = strip * W, k0 = seg * rp.Wz, k1 = k0 + rp.Wz;
+    // this wavefront's colour: its lines and nodes (step 2 each way)
+    const int kp = ph & 1, ip = ph >> 1, grow = 2 - ph;   // nodes past the segment that later colours read
+    const int klo = max(kp, k0 - grow), khi = min(g.noz - 1, k1 + grow);
+    const int ilo = i0 + ip, ihi = min(g.nox - 1, i0 + W - ip);
+    const int nk = khi >= klo ? ((khi - klo) >> 1) + 1 : 0, ni = ihi >= ilo ? ((ihi - ilo) >> 1) + 1 : 0;
+    const int r = S::WIDE ? w - 3 * ph : lane / 21, t = S::WIDE ? lane : lane - 21 * r;
+    const bool act = r < 3 && t < nk * ni;
+    int ii = 0;   // t / nk, of at most W/2 + 1 lines
+#pragma unroll
+    for (int m = 1; m <= W / 2; m++) ii += t >= m * nk;
+    const int k = klo + 2 * (t - ii * nk), i = ilo + 2 * ii;
+    const int c = kp | (ip << 1) | (jpar << 2);
+    const int fself = act ? 3 * nid(g, k, i, j) + r : 0;
+    // staged region: lines i0-1 .. i0+W+1 of three planes, nodes kr0 .. (kr0
+    // even), zero outside the mesh.  A wavefront takes whole lines, 21 nodes
+    // at a time (a lane keeps its component), all requested before the first
+    // is stored; past its last line it repeats it.
+    const int l3 = min(lane, 62) / 3, comp = min(lane, 62) - 3 * l3;
+    const int kr0 = max(k0 - 4, -2);
+    V stage[S::BATCH];
+    const V *side = dside ? dside : F, *same = dself ? dself : F;
+#pragma unroll
+    for (int q = 0; q < S::BATCH; q++) {
+        const int ln = min(w + q / S::CH * S::WAVES, 3 * NL - 1), pl = ln / NL;
+        const int gi = min(max(i0 - 1 + ln - pl * NL, 0), g.nox - 1), gj = min(max(j + pl - 1, 0), g.noy - 1);
+        const int gk = min(max(kr0 + q % S::CH * 21 + l3, 0), g.noz - 1);
+        stage[q] = (pl == 1 ? same : side)[3 * nid(g, gk, gi, gj) + comp];
+    }
+    const V Fr = F[fself], Br = BI[fself];
+    float kv[3][27];
+    {
+        const KT *kq = K + ktile(act ? colour_index(g, c, k, i, j) : g.cs[c]) + (r < 3 ? 3 * 64 * r : 0);
+#pragma unroll
+        for (int pp = 0; pp < 3; pp++) {   // in the order of their use
+            const int P = pp == 0 ? 0 : pp == 1 ? 2 : 1;
+#pragma unroll
+            for (int bb = 0; bb < 9; bb++)
+#pragma unroll
+                for (int cc = 0; cc < 3; cc++) kv[P][3 * bb + cc] = (float)kq[(81 * P + 9 * bb + cc) * 64];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < S::BATCH; q++) {
+        const int ln = min(w + q / S::CH * S::WAVES, 3 * NL - 1), kq = q % S::CH * 21 + l3, pl = ln / NL;
+        const bool in = (pl == 1 ? dself : dside) && (unsigned)(i0 - 1 + ln - pl * NL) < (unsigned)g.nox &&
+                        (unsigned)(j + pl - 1) < (unsigned)g.noy && (unsigned)(kr0 + kq) < (unsigned)g.noz;
+        if (kq < 2 * HZ) sd[ln * LINE + comp * 2 * HZ + (kq & 1) * HZ + (kq >> 1)] = in ? stage[q] : V(0);
+    }
+    __syncthreads();
+    // this node's component 0 on its own plane (an idle lane's: any inner
+    // one), and its neighbours along k, which lie in the other parity's run
+    const int own = act ? (NL + i - i0 + 1) * LINE + kp * HZ + ((k - kr0) >> 1) : (NL + 1) * LINE + kp * HZ + 1;
+    const V *u0 = sd + own, *um = u0 + (kp ? -HZ : HZ - 1), *up = u0 + (kp ? 1 - HZ : HZ);
+    // the coefficients stay as loaded until here: widened earlier they would
+    // not fit the registers
+    auto hold = [](float kv[27]) {
+#pragma unroll
+        for (int e = 0; e < 27; e++) asm volatile("" : "+v"(kv[e]));
+    };
+    auto gather = [&](int pl, V uv[27]) {
+#pragma unroll
+        for (int dx = -1; dx <= 1; dx++)
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                const int p = (pl * NL + dx) * LINE + e * 2 * HZ;
+                uv[9 * (dx + 1) + e] = um[p];
+                uv[9 * (dx + 1) + 3 + e] = u0[p];
+                uv[9 * (dx + 1) + 6 + e] = up[p];
+            }
+    };
+    V uv[27];
+    hold(kv[0]);
+    gather(-1, uv);
+    const V s0 = plane_sum_row<V>(kv[0], uv);
+    __builtin_amdgcn_sched_barrier(0);   // one plane's entries live at a time
+    hold(kv[2]);
+    gather(1, uv);
+    const V s2 = plane_sum_row<V>(kv[2], uv);
+    __builtin_amdgcn_sched_barrier(0);
+    const V m0 = u0[0], m1 = u0[2 * HZ], m2 = u0[4 * HZ];
+#pragma unroll 1
+    for (int p = 0; p < 4; p++) {
+        __syncthreads();
+        if (ph == p) {
+            gather(0, uv);
+            uv[12] = m0;
+            uv[13] = m1;
+            uv[14] = m2;
+            const V o = (s0 + plane_sum_row<V>(kv[1], uv)) + s2;
+            // FP16 rows are stored scaled by BI: t = BI F - (BI K) d
+            const float tt = sizeof(KT) == 2 ? (float)(Fr * Br - o) : (float)((Fr - o) * Br);
+            const V dr = r == 0 ? m0 : r == 1 ? m1 : m2;
+            if (act) sd[own + r * 2 * HZ] = dr + tt;
+        }
+    }
+    __syncthreads();
+    // the workgroup's own nodes, a line to a wavefront
+    const int ie = strip == rp.nstrip - 1 ? g.nox : i0 + W;
+    const int onk = (seg == rp.ns - 1 ? g.noz : k1) - k0, rel = (k0 - kr0) >> 1;   // k0 - kr0 is even
+    for (int gi = i0 + w; gi < ie; gi += S::WAVES) {
+        V *out = dout + 3L * nid(g, k0, gi, j) + comp;
+        const V *row = sd + (NL + gi - i0 + 1) * LINE + comp * 2 * HZ + rel;
+        for (int kq = lane < 63 ? l3 : onk; kq < onk; kq += 21) out[3 * kq] = row[(kq & 1) * HZ + (kq >> 1)];
+    }
+}
+
+using RectNarrow = RectShape<false, 2, 10>;
+using RectWide = RectShape<true, 4, 23>;
+
+template <class S>
+static RectPart rect_part(const Geo &g, int shape) {
+    const int most = S::NODES / (S::W / 2 + 1);   // nodes of a colour along k
+    for (int ns = 1; ns <= (g.noz + 1) / 2; ns++) {
+        RectPart rp{};
+        rp.shape = shape;
+        rp.Wz = std::max(2, ((g.noz - 1 + ns - 1) / ns + 1) / 2 * 2);
+        rp.ns = std::max(1, (g.noz - 1 + rp.Wz - 1) / rp.Wz);
+        if (rp.ns != ns) continue;
+        const int nk = ns == 1 ? (g.noz + 1) / 2 : std::min((g.noz + 1) / 2, rp.Wz / 2 + 3);
+        if (nk > most || std::min(rp.Wz + 7, g.noz + 2) + 1 > 2 * S::HZ) continue;
+        rp.nstrip = std::max(1, (g.nox - 1 + S::W - 1) / S::W);
+        return rp;
+    }
+    return RectPart{};
+}
+
+// the narrow shape, else the wide one, while there is at most one workgroup
+// per CU (measured above); larger levels pass colour by colour
+RectPart rect_planes(const Geo &g) {
+    constexpr long CUS = 256;
+    for (const RectPart &rp : {rect_part<RectNarrow>(g, 1), rect_part<RectWide>(g, 2)})
+        if (rp.shape && (long)(g.noy + 1) / 2 * rp.nstrip * rp.ns <= CUS) return rp;
+    return RectPart{};
+}
+
+template <typename V, typename KT>
+static void rect_launch(hipStream_t s, const Level &L, const KT *K, const V *BI, const V *F, int jpar, const V *dself,
+                        const V *dside, V *dout, hipEvent_t e0, hipEvent_t e1) {
+    const RectPart &rp = L.planes;
+    const dim3 grid(rp.ns, rp.nstrip, (L.g.noy - jpar + 1) / 2);
+    if (grid.z == 0) return;
+    auto launch = [&](auto kern, int waves) {
+        if (e0)
+            hipExtLaunchKernelGGL(kern, grid, dim3(64 * waves), 0, s, e0, e1, 0, L.g, rp, jpar, K, BI, F, dself, dside, dout);
+        else
+            hipLaunchKernelGGL(kern, grid, dim3(64 * waves), 0, s, L.g, rp, jpar, K, BI, F, dself, dside, dout);
+    };
+    if (rp.shape == 1) launch(k_gs_rect<V, KT, RectNarrow>, RectNarrow::WAVES);
+    else launch(k_gs_rect<V, KT, RectWide>, RectWide::WAVES);
+}
+
+template <typename V>
+void gs_rect(hipStream_t s, const Level &L, const V *BI, const V *F, int jpar, const V *dself, const V *dside, V *dout,
+             hipEvent_t e0, hipEvent_t e1) {
+    if constexpr (sizeof(V) == 4) {
+        if (L.Kh) {
+            rect_launch<V, _Float16>(s, L, (const _Float16 *)L.Kh, BI, F, jpar, dself, dside, dout, e0, e1);
+            return;
+        }
+    }
+    rect_launch<V, float>(s, L, (const float *)L.K, BI, F, jpar, dself, dside, dout, e0, e1);
+}
+template void gs_rect<double>(hipStream_t, const Level &, const double *, const double *, int, const double *,
+                              const double *, double *, hipEvent_t, hipEvent_t);
+template void gs_rect<float>(hipStream_t, const Level &, const float *, const float *, int, const float *, const float *,
+                             float *, hipEvent_t, hipEvent_t);
 
 // the FP16 stiffness of the mixed = 2 form: each row scaled by its BI, so
 // the coefficients are O(1) (the diagonal block's diagonal is 1) whatever the
@@ -770,24 +1009,11 @@ constexpr long AFFINE_MAX_DOF = 1500;
 
 bool affine_ok(const Level &L) { return 3L * L.g.nno <= AFFINE_MAX_DOF; }
 
-// one-workgroup smoother call (k_gs_wg, below): tiles in flight, threads,
-// and the largest level it takes.  One CU reads the stiffness through L2 at
-// 50-70 GB/s, so at 2601 nodes a call takes 156 us against 111 us as
-// per-colour launches of 4.3 us each; below about 1500 nodes it is faster.
-constexpr int WG_SLOTS = 4;
-constexpr int WG_TPB = WG_SLOTS * 3 * 64;
-constexpr int WG_MAX_NNO = 1024;
 // largest level of the one-XCD smoother (k_gs_xcd, below): its FP32
 // stiffness (972 B a node) stays within about one XCD's 4 MB L2; polls per
 // barrier before a launch gives up
 constexpr int XCD_MAX_NNO = 6000;
 constexpr unsigned XCD_SPIN = 1u << 20;
-template <typename V>
-__global__ void __launch_bounds__(WG_TPB) k_gs_wg(Geo g, const float *__restrict__ K,
-                                                  const unsigned *__restrict__ NODE, const V *__restrict__ BI, V *d,
-                                                  const V *__restrict__ F, V *__restrict__ Ad,
-                                                  const V *__restrict__ rhs, V *__restrict__ res, int sweeps,
-                                                  int guess);
 
 size_t lds_limit() {
     static size_t lim = 0;
@@ -800,11 +1026,6 @@ size_t lds_limit() {
             lim = 65536;
         if (lim > 65536) {
             (void)hipFuncSetAttribute((const void *)k_gs_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lim);
-            const size_t ps = (size_t)WG_SLOTS * 9 * 64;   // k_gs_wg's static partial sums
-            (void)hipFuncSetAttribute((const void *)k_gs_wg<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)(lim - ps * sizeof(double)));
-            (void)hipFuncSetAttribute((const void *)k_gs_wg<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)(lim - ps * sizeof(float)));
         }
     }
     return lim;
@@ -820,119 +1041,6 @@ void gs_small(hipStream_t s, const Level &L, double *d, const double *F, double 
     hipLaunchKernelGGL(k_gs_lds, dim3(1), dim3(SMALL_TPB), kstage_bytes(nno) + vstage_bytes(nno), s, L.g, L.K, L.BI,
                        L.NODE, d, F, Ad, sweeps, guess, 0);
 }
-
-// ---------------------------------------------------------------------------
-// A small level whose stiffness does not fit in LDS (8x8x8 elements, 729
-// nodes, 708 KB of stiffness) runs a whole gauss_seidel call in one
-// workgroup: d in LDS, the stiffness read through L2 (resident in the one
-// XCD's L2 after the first sweep).  Each colour pass is
-// k_gs_colour's, with workgroup barriers in place of kernel boundaries:
-// three wavefronts per 64-node tile form the three y-planes (same trees,
-// same update expression), WG_SLOTS tiles at a time; then Ad = K d in
-// row_product's order, BC rows stripped, and res = rhs - Ad when asked.
-// A colour pass of such a level is latency-bound as a kernel of its own.
-
-template <typename V>
-__global__ void __launch_bounds__(WG_TPB) k_gs_wg(Geo g, const float *__restrict__ K,
-                                                  const unsigned *__restrict__ NODE, const V *__restrict__ BI, V *d,
-                                                  const V *__restrict__ F, V *__restrict__ Ad,
-                                                  const V *__restrict__ rhs, V *__restrict__ res, int sweeps,
-                                                  int guess) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    V *ds = (V *)smem;   // [3 nno]
-    __shared__ V Ps[WG_SLOTS][3][3][64];   // [slot][plane][row][node]
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, slot = w / 3, pl = w - 3 * slot;
-    const int n3 = 3 * g.nno;
-    for (int idx = tid; idx < n3; idx += blockDim.x) ds[idx] = guess ? d[idx] : V(0);
-    __syncthreads();
-    for (int cyc = 0; cyc < sweeps; cyc++)
-        for (int c = 0; c < 8; c++) {
-            const int tiles = (g.cn[c] + 63) >> 6;
-            for (int t0 = 0; t0 < tiles; t0 += WG_SLOTS) {   // uniform over the workgroup
-                const int q = g.cs[c] + (t0 + slot) * 64 + lane;
-                const bool act = t0 + slot < tiles && q < g.cs[c] + g.cn[c];
-                int k = 0, i = 0, j = 0;
-                if (act) colour_kij(g, c, q, k, i, j);
-                const int self = nid(g, k, i, j);
-                V Fr = V(0), Br = V(0);
-                if (act) {
-                    Fr = F[3 * self + pl];
-                    Br = BI[3 * self + pl];
-                    V out[3];
-                    const float *kp = K + ktile(q);
-                    if (pl == 0)
-                        plane_rows<0>(g, kp, k, i, j, self, (const V *)ds, out);
-                    else if (pl == 1)
-                        plane_rows<1>(g, kp, k, i, j, self, (const V *)ds, out);
-                    else
-                        plane_rows<2>(g, kp, k, i, j, self, (const V *)ds, out);
-                    Ps[slot][pl][0][lane] = out[0];
-                    Ps[slot][pl][1][lane] = out[1];
-                    Ps[slot][pl][2][lane] = out[2];
-                }
-                __syncthreads();
-                if (act) {
-                    const int r = pl;
-                    const V o = (Ps[slot][0][r][lane] + Ps[slot][1][r][lane]) + Ps[slot][2][r][lane];
-                    const float t = (float)((Fr - o) * Br);
-                    ds[3 * self + r] = ds[3 * self + r] + t;
-                }
-                __syncthreads();
-            }
-        }
-    for (int q = tid; q < g.pitch; q += blockDim.x) {
-        const int col = colour_valid(g, q);
-        if (col < 0) continue;
-        int k, i, j;
-        colour_kij(g, col, q, k, i, j);
-        const float *kp = K + ktile(q);
-        const V *u = ds;
-        V out[3];
-        row_product_t<V>(
-            g, [kp](int ci) { return kp[ci * 64]; }, k, i, j, [u](int idx) { return u[idx]; }, out);
-        const int n = nid(g, k, i, j);
-        strip3(NODE[n], out);
-        Ad[3 * n] = out[0];
-        Ad[3 * n + 1] = out[1];
-        Ad[3 * n + 2] = out[2];
-        if (res) {
-            res[3 * n] = rhs[3 * n] - out[0];
-            res[3 * n + 1] = rhs[3 * n + 1] - out[1];
-            res[3 * n + 2] = rhs[3 * n + 2] - out[2];
-        }
-    }
-    for (int idx = tid; idx < n3; idx += blockDim.x) d[idx] = ds[idx];
-}
-
-template <typename V>
-size_t wg_stage_bytes(const Level &L) {
-    return (size_t)3 * L.g.nno * sizeof(V);
-}
-
-template <typename V>
-bool gs_wg_ok(const Level &L) {
-    return !L.Kh && L.g.nno <= WG_MAX_NNO &&
-           wg_stage_bytes<V>(L) + sizeof(V) * WG_SLOTS * 9 * 64 <= lds_limit();
-}
-template bool gs_wg_ok<double>(const Level &);
-template bool gs_wg_ok<float>(const Level &);
-
-template <typename V>
-void gs_wg(hipStream_t s, const Level &L, const V *BI, V *d, const V *F, V *Ad, const V *rhs, V *res, int sweeps,
-           int guess, hipEvent_t e0, hipEvent_t e1) {
-    auto kern = k_gs_wg<V>;
-    const float *K = L.K;
-    if (e0)
-        hipExtLaunchKernelGGL(kern, dim3(1), dim3(WG_TPB), wg_stage_bytes<V>(L), s, e0, e1, 0, L.g, K, L.NODE, BI, d,
-                              F, Ad, rhs, res, sweeps, guess);
-    else
-        hipLaunchKernelGGL(kern, dim3(1), dim3(WG_TPB), wg_stage_bytes<V>(L), s, L.g, K, L.NODE, BI, d, F, Ad, rhs,
-                           res, sweeps, guess);
-}
-template void gs_wg<double>(hipStream_t, const Level &, const double *, double *, const double *, double *,
-                            const double *, double *, int, int, hipEvent_t, hipEvent_t);
-template void gs_wg<float>(hipStream_t, const Level &, const float *, float *, const float *, float *, const float *,
-                           float *, int, int, hipEvent_t, hipEvent_t);
 
 // ---------------------------------------------------------------------------
 // A mid-size level (a few thousand nodes, a few MB of stiffness) runs a
@@ -1094,7 +1202,7 @@ int xcd_groups(const Level &L) {
 bool gs_xcd_ok(const Level &L) {
     int t = 1;
     for (int c = 0; c < 8; c++) t = std::max(t, (L.g.cn[c] + 63) / 64);
-    return !L.Kh && L.xbar && L.g.nno > WG_MAX_NNO && L.g.nno <= XCD_MAX_NNO && t <= 16;
+    return !L.Kh && L.xbar && L.g.nno > SMALL_NNO && L.g.nno <= XCD_MAX_NNO && t <= 16;
 }
 
 template <typename V>
@@ -1181,11 +1289,6 @@ __device__ __forceinline__ BoxColour box_colour(const BoxPart &bp, int bz, int b
     r.nx = max(0, (x1 - r.i0 + 1) >> 1);
     r.ny = max(0, (y1 - r.j0 + 1) >> 1);
     return r;
-}
-
-// colour-ordered index of node (k, i, j) of colour c (inverse of colour_kij)
-__device__ __forceinline__ int colour_index(const Geo &g, int c, int k, int i, int j) {
-    return g.cs[c] + (k >> 1) + g.cz[c] * ((i >> 1) + g.cx[c] * (j >> 1));
 }
 
 // Box tiles: for the (box, colour) tile b 8 + c and y-plane P, each node's

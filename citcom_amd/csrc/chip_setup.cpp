@@ -473,6 +473,14 @@ int build_mesh(chip_ctx *c) {
             if (L.Kbox_half ? dev_alloc(c, (uint16_t **)&L.Kbox, n) : dev_alloc(c, (float **)&L.Kbox, n)) return -1;
             if (!L.tmpf && dev_alloc(c, &L.tmpf, 3 * (size_t)L.g.nno)) return -1;
         }
+    // joined colour passes, and the vector their sweeps alternate with
+    for (int lev = c->levmin; lev <= c->levmax; lev++) {
+        Level &L = c->L[lev];
+        L.planes = rect_planes(L.g);
+        if (!L.planes.shape) continue;
+        if (!L.tmp && dev_alloc(c, &L.tmp, 3 * (size_t)L.g.nno)) return -1;
+        if (p.mixed && !L.tmpf && dev_alloc(c, &L.tmpf, 3 * (size_t)L.g.nno)) return -1;
+    }
     const Geo &g = c->L[c->levmax].g;
     const size_t nno = g.nno, nel = g.nel, neq = 3 * nno;
     if (dev_alloc(c, &c->U, neq) || dev_alloc(c, &c->P, nel) || dev_alloc(c, &c->F, neq) ||

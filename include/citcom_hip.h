@@ -182,8 +182,9 @@ int chip_timestep(chip_ctx *c, chip_pg_stats *pg, chip_stokes_stats *st, float *
 int chip_general_stokes_solver(chip_ctx *c, chip_stokes_stats *st);
 
 /* ---- measurement ---------------------------------------------------------- */
-/* kernel: "gs_colour", "matvec", "gs_wg" (the one-workgroup smoother call
- * of small levels), "gs_xcd" (the one-XCD smoother call of mid-size
+/* kernel: "gs_colour" (the launches of one colour, or of four where a level
+ * joins them), "matvec", "gs_wg" (the joined colour passes of levels of at
+ * most 1024 nodes), "gs_xcd" (the one-XCD smoother call of mid-size
  * levels) or "gs_box" (one sweep of the box smoother of the FP32
  * cycles).  While enabled, every launch of that kernel
  * is bracketed by HIP events on the work stream; read returns the number of
@@ -195,11 +196,13 @@ long chip_device_bytes(chip_ctx *c);
 /* "graphs": 1 (default) replays each multigrid call as one captured HIP
  * graph, 0 launches its kernels one by one; results are identical.
  * "small_levels": 1 (default) smooths levels whose stiffness fits in LDS in
- * one single-workgroup kernel per gauss_seidel call, 0 launches one kernel
- * per colour pass on every level; results are identical.
- * "gs_wg": 1 (default) also runs a whole gauss_seidel call in one workgroup
- * on levels of at most 1024 nodes whose stiffness does not fit in LDS;
- * 0 launches one kernel per colour pass there; results are identical.
+ * one single-workgroup kernel per gauss_seidel call, and other levels of at
+ * most about 36000 nodes in two launches per sweep (four colours each);
+ * 0 launches one kernel per colour pass on every level; results are
+ * identical.
+ * "gs_wg": 1 (default) joins the colour passes also on levels of at most
+ * 1024 nodes; 0 launches one kernel per colour pass there; results are
+ * identical.
  * "coarse_direct": 1 (default) lets the FP32 cycles of the mixed forms
  * stop at the largest level below the finest with at most 8192 unknowns
  * and at least two levels below it (17x17x9 nodes at 128x128x64 elements)

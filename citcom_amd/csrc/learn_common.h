@@ -51,4 +51,11 @@ __device__ __forceinline__ bf16x4 load4(const uint16_t *p) {
     return a;
 }
 
+// 3x3x3 convolution of X[nb][nv][ci] with W[co][27][ci] (wtrans: W[ci][27][co]),
+// the tap's offset mirrored if asked (unet_kernels.hip); for operands that
+// conv_block_ok accepts, 0 or -1
+bool conv_block_ok(int ci, const uint16_t *x, const uint16_t *w, const uint16_t *res, const uint16_t *y, const float *yf);
+int conv_fwd(const Vol &g, int nb, int ci, int co, const uint16_t *x, const uint16_t *w, int wtrans, const float *bias,
+             const uint16_t *res, int relu, int mirror, uint16_t *y, float *yf, hipStream_t s);
+
 }  // namespace learn

@@ -15,90 +15,17 @@
 #include <string>
 
 #include "../../include/citcom_learn.h"
+#include "learn_common.h"
+
+using namespace learn;
 
 namespace {
 
 constexpr int CH = 16;   // channels (padded)
 constexpr int TAPS = 27;
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-// round to nearest even (finite values)
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    const uint32_t u = __float_as_uint(f);
-    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
-
-struct Vol {
-    int nx, ny, nz, nv;
-};
-
-__device__ __forceinline__ int nbr(const Vol &g, int v, int t) {
-    const int k = v % g.nz, i = (v / g.nz) % g.nx, j = v / (g.nz * g.nx);
-    const int dz = t % 3 - 1, dx = (t / 3) % 3 - 1, dy = t / 9 - 1;
-    const int kk = k + dz, ii = i + dx, jj = j + dy;
-    if ((unsigned)kk >= (unsigned)g.nz || (unsigned)ii >= (unsigned)g.nx || (unsigned)jj >= (unsigned)g.ny) return -1;
-    return kk + g.nz * (ii + g.nx * jj);
-}
-
-// the same with v's (k, i, j) formed once: in a loop over the taps, which
-// is then unrolled, no division is left per tap
-struct Cell {
-    int v, k, i, j;
-    bool in;
-};
-__device__ __forceinline__ Cell cell(const Vol &g, int v) {
-    return {v, v % g.nz, (v / g.nz) % g.nx, v / (g.nz * g.nx), v < g.nv};
-}
-__device__ __forceinline__ int nbr(const Vol &g, const Cell &c, int t) {
-    const int dz = t % 3 - 1, dx = (t / 3) % 3 - 1, dy = t / 9 - 1;
-    const bool ok = c.in && (unsigned)(c.k + dz) < (unsigned)g.nz && (unsigned)(c.i + dx) < (unsigned)g.nx &&
-                    (unsigned)(c.j + dy) < (unsigned)g.ny;
-    return ok ? c.v + dz + g.nz * (dx + g.nx * dy) : -1;
-}
-
-__device__ __forceinline__ bf16x4 load4(const uint16_t *p) {
-    const uint2 r = *reinterpret_cast<const uint2 *>(p);
-    bf16x4 a;
-    a[0] = (short)(r.x & 0xFFFF);
-    a[1] = (short)(r.x >> 16);
-    a[2] = (short)(r.y & 0xFFFF);
-    a[3] = (short)(r.y >> 16);
-    return a;
-}
-
-// ---- forward: Y[v][o] = act(sum_t sum_c X[v+off_t][c] W[o][t][c] + bias[o])
-// one wavefront per 16 voxels; the 27 taps are the K loop (16 channels each)
-__global__ void __launch_bounds__(256) k_conv_fwd(Vol g, const uint16_t *__restrict__ X, const uint16_t *__restrict__ W,
-                                                  const float *__restrict__ bias, int relu, uint16_t *__restrict__ Y,
-                                                  float *__restrict__ Yf) {
-    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, b = blockIdx.y;
-    const int v0 = (blockIdx.x * 4 + wv) * 16;
-    if (v0 >= g.nv) return;
-    const uint16_t *Xb = X + (size_t)b * g.nv * CH;
-    const int m = v0 + (l & 15), kq = 4 * (l >> 4);
-    const Cell cm = cell(g, m);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < TAPS; t++) {
-        const int vn = nbr(g, cm, t);
-        bf16x4 a = {0, 0, 0, 0};
-        if (vn >= 0) a = load4(Xb + (size_t)vn * CH + kq);
-        const bf16x4 w = load4(W + ((size_t)(l & 15) * TAPS + t) * CH + kq);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, w, acc, 0, 0, 0);
-    }
-    const int o = l & 15;
-    for (int i = 0; i < 4; i++) {
-        const int v = v0 + kq + i;
-        if (v >= g.nv) continue;
-        float y = acc[i] + bias[o];
-        if (relu) y = y > 0.f ? y : 0.f;
-        Y[((size_t)b * g.nv + v) * CH + o] = f2bf(y);
-        if (Yf) Yf[((size_t)b * g.nv + v) * CH + o] = y;
-    }
-}
+// neighbour of voxel v at tap t, -1 outside the grid
+__device__ __forceinline__ int nbr(const Vol &g, int v, int t) { return learn::nbr(g, learn::cell(g, v), t); }
 
 // ---- backward through the activation: dYp = dY * (Y > 0)
 __global__ void k_relu_bwd(const uint16_t *__restrict__ Y, uint16_t *__restrict__ dY, long n) {
@@ -106,7 +33,7 @@ __global__ void k_relu_bwd(const uint16_t *__restrict__ Y, uint16_t *__restrict_
     if (i < n && !(bf2f(Y[i]) > 0.f)) dY[i] = 0;
 }
 
-// ---- backward data: dX[v][c] = sum_t sum_o dY[v-off_t][o] W[o][t][c]
+// ---- backward data, less aligned operands: dX[v][c] = sum_t sum_o dY[v-off_t][o] W[o][t][c]
 __global__ void __launch_bounds__(256) k_conv_bwd_data(Vol g, const uint16_t *__restrict__ dY,
                                                        const uint16_t *__restrict__ W, uint16_t *__restrict__ dX) {
     __shared__ __align__(16) uint16_t Wt[TAPS][CH][CH];   // [t][c][o]
@@ -273,10 +200,7 @@ extern "C" {
 
 int cl_conv3d_fwd(const uint16_t *x, int nb, int nx, int ny, int nz, const uint16_t *w, const float *bias, int relu,
                   uint16_t *y, float *yf, void *stream) {
-    const Vol g{nx, ny, nz, nx * ny * nz};
-    if (nb <= 0 || g.nv <= 0) return -1;
-    hipLaunchKernelGGL(k_conv_fwd, dim3((g.nv + 63) / 64, nb), dim3(256), 0, st(stream), g, x, w, bias, relu, y, yf);
-    return ret();
+    return cl_conv3d_fwd_c(x, nb, nx, ny, nz, CH, CH, w, bias, nullptr, relu, 0, y, yf, stream);
 }
 
 int cl_relu_bwd(const uint16_t *y, uint16_t *dy, long n, void *stream) {
@@ -287,6 +211,11 @@ int cl_relu_bwd(const uint16_t *y, uint16_t *dy, long n, void *stream) {
 int cl_conv3d_bwd_data(const uint16_t *dy, int nb, int nx, int ny, int nz, const uint16_t *w, uint16_t *dx,
                        void *stream) {
     const Vol g{nx, ny, nz, nx * ny * nz};
+    // the forward convolution of dy with the weights read transposed and the
+    // taps mirrored
+    if (nb > 0 && g.nv > 0 && conv_block_ok(CH, dy, w, nullptr, dx, nullptr) &&
+        conv_fwd(g, nb, CH, CH, dy, w, 1, nullptr, nullptr, 0, 1, dx, nullptr, st(stream)) == 0)
+        return ret();
     hipLaunchKernelGGL(k_conv_bwd_data, dim3((g.nv + 63) / 64, nb), dim3(256), 0, st(stream), g, dy, w, dx);
     return ret();
 }

@@ -58,4 +58,9 @@ bool conv_block_ok(int ci, const uint16_t *x, const uint16_t *w, const uint16_t 
 int conv_fwd(const Vol &g, int nb, int ci, int co, const uint16_t *x, const uint16_t *w, int wtrans, const float *bias,
              const uint16_t *res, int relu, int mirror, uint16_t *y, float *yf, hipStream_t s);
 
+// weight and bias gradient, partial sums in at most `slots` slots of
+// co*27*ci + co floats; for 16-byte aligned operands, 0 or -1
+int conv_wgrad(const Vol &g, int nb, int ci, int co, const uint16_t *x, const uint16_t *dy, float *part, long slots,
+               float *grad, hipStream_t s);
+
 }  // namespace learn

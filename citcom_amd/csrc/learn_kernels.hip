@@ -24,9 +24,6 @@ namespace {
 constexpr int CH = 16;   // channels (padded)
 constexpr int TAPS = 27;
 
-// neighbour of voxel v at tap t, -1 outside the grid
-__device__ __forceinline__ int nbr(const Vol &g, int v, int t) { return learn::nbr(g, learn::cell(g, v), t); }
-
 // ---- backward through the activation: dYp = dY * (Y > 0)
 __global__ void k_relu_bwd(const uint16_t *__restrict__ Y, uint16_t *__restrict__ dY, long n) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -66,57 +63,8 @@ __global__ void __launch_bounds__(256) k_conv_bwd_data(Vol g, const uint16_t *__
     }
 }
 
-// ---- backward weights: dW[o][t][c] = sum_v dY[v][o] X[v+off_t][c], per
-// wavefront over its voxel chunk (K = 16 voxels per MFMA), partial sums per
-// wavefront; db[o] partials likewise
-constexpr int WCHUNK = 256;   // voxels per wavefront
-__global__ void __launch_bounds__(256) k_conv_bwd_weight(Vol g, int nb, const uint16_t *__restrict__ X,
-                                                         const uint16_t *__restrict__ dY, float *__restrict__ part) {
-    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const long chunk = (long)blockIdx.x * 4 + wv;   // over nb * ceil(nv / WCHUNK)
-    const int per = (g.nv + WCHUNK - 1) / WCHUNK;
-    float *P = part + (size_t)chunk * (TAPS * CH * CH + CH);
-    if (chunk >= (long)nb * per) return;
-    const int b = (int)(chunk / per), vbeg = (int)(chunk % per) * WCHUNK;
-    const int vend = min(g.nv, vbeg + WCHUNK);
-    const uint16_t *Xb = X + (size_t)b * g.nv * CH, *dYb = dY + (size_t)b * g.nv * CH;
-    const int o = l & 15, kq = 4 * (l >> 4);
-    float dbias = 0.f;
-    for (int t = 0; t < TAPS; t++) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int v0 = vbeg; v0 < vend; v0 += 16) {
-            bf16x4 a, bb;
-            for (int i = 0; i < 4; i++) {
-                const int v = v0 + kq + i;
-                uint16_t av = 0, bv = 0;
-                if (v < vend) {
-                    av = dYb[(size_t)v * CH + o];
-                    const int vn = nbr(g, v, t);
-                    if (vn >= 0) bv = Xb[(size_t)vn * CH + o];
-                    if (t == 0) dbias += bf2f(av);
-                }
-                a[i] = (short)av;
-                bb[i] = (short)bv;
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, acc, 0, 0, 0);
-        }
-        // D[4(l/16)+i][l%16] = dW[o' = kq+i][t][c = l%16]
-        for (int i = 0; i < 4; i++) P[((size_t)(kq + i) * TAPS + t) * CH + (l & 15)] = acc[i];
-    }
-    // bias: lanes sharing o = l%16 hold disjoint voxel quarters
-    dbias += __shfl_xor(dbias, 16, 64);
-    dbias += __shfl_xor(dbias, 32, 64);
-    if (l < 16) P[TAPS * CH * CH + l] = dbias;
-}
-
-// dW (and db) = sum of the partials in chunk order
-__global__ void k_sum_partials(const float *__restrict__ part, long nchunks, float *__restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= TAPS * CH * CH + CH) return;
-    float s = 0.f;
-    for (long k = 0; k < nchunks; k++) s += part[(size_t)k * (TAPS * CH * CH + CH) + i];
-    out[i] = s;
-}
+// chunks of voxels whose partial sums a caller's workspace has slots for
+constexpr int WCHUNK = 256;
 
 // mean squared error over the first nout channels; dY = d loss / d Y in bf16
 __global__ void k_mse(const float *__restrict__ Y, const float *__restrict__ T, long nvox, int nout,
@@ -227,13 +175,8 @@ long cl_conv3d_bwd_weight_workspace(int nb, int nx, int ny, int nz) {
 
 int cl_conv3d_bwd_weight(const uint16_t *x, const uint16_t *dy, int nb, int nx, int ny, int nz, float *grad,
                          float *workspace, void *stream) {
-    const Vol g{nx, ny, nz, nx * ny * nz};
-    const long chunks = (long)nb * ((g.nv + WCHUNK - 1) / WCHUNK);
-    hipLaunchKernelGGL(k_conv_bwd_weight, dim3((unsigned)((chunks + 3) / 4)), dim3(256), 0, st(stream), g, nb, x, dy,
-                       workspace);
-    hipLaunchKernelGGL(k_sum_partials, dim3((TAPS * CH * CH + CH + 255) / 256), dim3(256), 0, st(stream), workspace,
-                       chunks, grad);
-    return ret();
+    // (a slot for 256 voxels holds at least as many as the general call's for 512)
+    return cl_conv3d_bwd_weight_c(x, dy, nb, nx, ny, nz, CH, CH, grad, workspace, stream);
 }
 
 long cl_scratch_bytes(void) { return SCRATCH_FLOATS * (long)sizeof(float); }
@@ -260,19 +203,12 @@ int cl_conv3d_bwd_weight_noalloc(const uint16_t *x, const uint16_t *dy, int nb, 
         g_learn_err = std::string("cl_conv3d_bwd_weight_noalloc: ") + why;
         return -1;
     }
-    // every chunk's slot of partial sums is written in full by
-    // k_conv_bwd_weight before k_sum_partials reads it, so nothing is cleared
-    const long chunks = (long)nb * ((g.nv + WCHUNK - 1) / WCHUNK);
-    hipLaunchKernelGGL(k_conv_bwd_weight, dim3((unsigned)((chunks + 3) / 4)), dim3(256), 0, st(stream), g, nb, x, dy,
-                       part);
-    hipLaunchKernelGGL(k_sum_partials, dim3((TAPS * CH * CH + CH + 255) / 256), dim3(256), 0, st(stream), part, chunks,
-                       grad);
+    // every slot of partial sums that is summed is written in full before, so
+    // nothing is cleared
+    if (cl_conv3d_bwd_weight(x, dy, nb, nx, ny, nz, grad, part, stream) == 0) return 0;
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        g_learn_err = std::string("cl_conv3d_bwd_weight_noalloc: ") + hipGetErrorString(e);
-        return -1;
-    }
-    return 0;
+    g_learn_err = std::string("cl_conv3d_bwd_weight_noalloc: ") + hipGetErrorString(e);
+    return -1;
 }
 
 int cl_mse(const float *y, const float *target, long nvox, int nout, uint16_t *dy, float *partial, void *stream) {

@@ -59,13 +59,46 @@ struct ConvBlock {
     int region;                       // staged voxels and pad
 };
 
+// A block's region of NCB 16-channel blocks into LDS: 64 units of 16 bytes of a
+// line to a wavefront at a time, CONV_BATCH of them requested before the first
+// is stored (no branch: off the grid the nearest voxel is read and zero
+// stored).  X: the batch's first voxel and channel, ci its voxels' stride.
+template <int NCB>
+__device__ __forceinline__ void stage_region(const Vol &g, const ConvBlock &cb, const uint16_t *__restrict__ X, int ci,
+                                             int k0, int i0, int j0, unsigned char *smem, int lane, int w) {
+    constexpr int UPV = 2 * NCB;   // 16-byte units of a voxel
+    const int nlines = cb.LX * cb.LY, upl = cb.LZ * UPV, nch = (upl + 63) >> 6, total = nlines * nch;
+    const unsigned mch = 65536u / nch + 1, mlx = 65536u / cb.LX + 1;   // exact for the few hundred chunks here
+    for (int ch = w; ch < total; ch += CONV_WAVES * CONV_BATCH) {
+        uint4 v[CONV_BATCH];
+        int at[CONV_BATCH];
+#pragma unroll
+        for (int q = 0; q < CONV_BATCH; q++) {
+            const int cq = min(ch + q * CONV_WAVES, total - 1), ln = (int)(cq * mch >> 16);
+            const int ly = (int)(ln * mlx >> 16), lx = ln - ly * cb.LX;
+            const int gi = i0 - 1 + lx, gj = j0 - 1 + ly;
+            const int u = min((cq - ln * nch) * 64 + lane, upl - 1), z = u / UPV, c = u - z * UPV, gk = k0 - 1 + z;
+            const int gic = min(max(gi, 0), g.nx - 1), gjc = min(max(gj, 0), g.ny - 1), gkc = min(max(gk, 0), g.nz - 1);
+            v[q] = *reinterpret_cast<const uint4 *>(X + (size_t)(gkc + g.nz * (gic + g.nx * gjc)) * ci + c * 8);
+            const bool in = gi == gic && gj == gjc && gk == gkc;
+            at[q] = (((c >> 1) * cb.region + 1 + ln * cb.LZ + z) * 32 + (c & 1) * 16) | (in ? 0 : 1);
+        }
+#pragma unroll
+        for (int q = 0; q < CONV_BATCH; q++) {
+            const unsigned keep = at[q] & 1 ? 0u : ~0u;
+            *reinterpret_cast<uint4 *>(smem + (at[q] & ~1)) =
+                make_uint4(v[q].x & keep, v[q].y & keep, v[q].z & keep, v[q].w & keep);
+        }
+    }
+}
+
 template <int NCB, int NBO, bool WREG>
 __global__ void __launch_bounds__(CONV_TPB) k_conv_block(Vol g, ConvBlock cb, int co, const uint16_t *__restrict__ X,
                                                          const uint16_t *__restrict__ W, int wtrans,
                                                          const float *__restrict__ bias, const uint16_t *__restrict__ R,
                                                          int relu, int mirror, uint16_t *__restrict__ Y,
                                                          float *__restrict__ Yf) {
-    constexpr int CI = 16 * NCB, UPV = 2 * NCB;   // 16-byte units of a voxel
+    constexpr int CI = 16 * NCB;
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned char *ws = smem + (size_t)NCB * cb.region * 32;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -103,32 +136,7 @@ __global__ void __launch_bounds__(CONV_TPB) k_conv_block(Vol g, ConvBlock cb, in
     else
         fetch_w(0);
     __builtin_amdgcn_sched_barrier(0);
-    // the region: 64 units of 16 bytes of a line to a wavefront at a time,
-    // CONV_BATCH of them requested before the first is stored (no branch: off
-    // the grid the nearest voxel is read and zero stored)
-    const int nlines = cb.LX * cb.LY, upl = cb.LZ * UPV, nch = (upl + 63) >> 6, total = nlines * nch;
-    const unsigned mch = 65536u / nch + 1, mlx = 65536u / cb.LX + 1;   // exact for the few hundred chunks here
-    for (int ch = w; ch < total; ch += CONV_WAVES * CONV_BATCH) {
-        uint4 v[CONV_BATCH];
-        int at[CONV_BATCH];
-#pragma unroll
-        for (int q = 0; q < CONV_BATCH; q++) {
-            const int cq = min(ch + q * CONV_WAVES, total - 1), ln = (int)(cq * mch >> 16);
-            const int ly = (int)(ln * mlx >> 16), lx = ln - ly * cb.LX;
-            const int gi = i0 - 1 + lx, gj = j0 - 1 + ly;
-            const int u = min((cq - ln * nch) * 64 + lane, upl - 1), z = u / UPV, c = u - z * UPV, gk = k0 - 1 + z;
-            const int gic = min(max(gi, 0), g.nx - 1), gjc = min(max(gj, 0), g.ny - 1), gkc = min(max(gk, 0), g.nz - 1);
-            v[q] = *reinterpret_cast<const uint4 *>(Xb + (size_t)(gkc + g.nz * (gic + g.nx * gjc)) * CI + c * 8);
-            const bool in = gi == gic && gj == gjc && gk == gkc;
-            at[q] = (((c >> 1) * cb.region + 1 + ln * cb.LZ + z) * 32 + (c & 1) * 16) | (in ? 0 : 1);
-        }
-#pragma unroll
-        for (int q = 0; q < CONV_BATCH; q++) {
-            const unsigned keep = at[q] & 1 ? 0u : ~0u;
-            *reinterpret_cast<uint4 *>(smem + (at[q] & ~1)) =
-                make_uint4(v[q].x & keep, v[q].y & keep, v[q].z & keep, v[q].w & keep);
-        }
-    }
+    stage_region<NCB>(g, cb, Xb, CI, k0, i0, j0, smem, lane, w);
     float bo[NBO][4];
 #pragma unroll
     for (int ob = 0; ob < NBO; ob++)
@@ -243,18 +251,23 @@ ConvBlock conv_block(const Vol &g, int nb, int groups, int ncb, int most, long l
 
 constexpr long CONV_LDS = 80 << 10;       // two workgroups to a CU
 
+// a kernel's dynamic LDS limit raised to CONV_LDS, once per device (a bit of `raised`)
+int raise_lds(const void *kern, std::atomic<uint64_t> &raised) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev > 63) return -1;
+    if (!(raised.load() >> dev & 1)) {
+        if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CONV_LDS) != hipSuccess) return -1;
+        raised.fetch_or(1ull << dev);
+    }
+    return 0;
+}
+
 template <int NCB, int NBO, bool WREG>
 int conv_launch(const Vol &g, int nb, int co, const uint16_t *x, const uint16_t *w, int wtrans, const float *bias,
                 const uint16_t *res, int relu, int mirror, uint16_t *y, float *yf, hipStream_t s) {
     auto kern = k_conv_block<NCB, NBO, WREG>;
-    static std::atomic<uint64_t> raised{0};   // a bit per device
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev > 63) return -1;
-    if (!(raised.load() >> dev & 1)) {
-        if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CONV_LDS) != hipSuccess)
-            return -1;
-        raised.fetch_or(1ull << dev);
-    }
+    static std::atomic<uint64_t> raised{0};
+    if (raise_lds((const void *)kern, raised)) return -1;
     const long wlds = WREG ? 0 : 9L * NCB * NBO * 512;
     const int groups = co / (16 * NBO);
     const ConvBlock cb = conv_block(g, nb, groups, NCB, WREG ? 1 << 20 : CONV_WAVES * CONV_M, (NCB * NBO == 1 ? CONV_LDS / 2 : CONV_LDS) - wlds);
@@ -361,10 +374,187 @@ __global__ void k_transpose_w(const uint16_t *__restrict__ W, int ci, int co, ui
 }
 
 // ---- weight gradient: dW[o][t][c] = sum_b sum_v dY[b][v][o] X[b][v+off_t][c],
-// db[o] = sum dY[b][v][o].  One wavefront per (voxel chunk, 16 output
-// channels, 16 input channels): 27 tap tiles, K = 16 voxels per MFMA, its
-// partial sums in its own slot; a second kernel sums the slots in chunk
-// order (a fixed order: the result does not depend on scheduling).
+// db[o] = sum dY[b][v][o].
+//
+// A workgroup takes NOB*16 output and NCB*16 input channels and every
+// nslots-th block of voxels: the block of X with its halo and the block of dY
+// are staged in LDS voxel by voxel, and the MFMA operands, which need four
+// voxels of one channel to a lane, are read with the transposing LDS read.  K
+// runs over the block's voxels inside the grid, 16 at a time (a table in LDS
+// holds each one's place in the region, so a tap is one offset); a wavefront
+// keeps the sums of seven taps in registers over all its blocks, the last one
+// the bias as a tap of ones, and writes them once into its slot.  A second
+// kernel sums the slots in a fixed order.
+//
+// Bound by the LDS reads (a tap's operand per MFMA, shared by the NOB output
+// blocks) and the staging.  65^3 nodes, batch 4: 16 x 16 channels 83 us and
+// its slots' sum 8; with 2-byte loads of single voxels and a slot for 512
+// voxels these took 1715 and 502 us.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ bf16x4 lds_read_tr(const unsigned char *p) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p);
+}
+
+constexpr int WG_TAPS = 7;   // taps of a wavefront: 0-6, 7-13, 14-20, 21-26 and the bias
+
+template <int NCB, int NOB>
+__global__ void __launch_bounds__(CONV_TPB) k_wgrad_block(Vol g, ConvBlock cb, int nblocks, int ci, int co,
+                                                          const uint16_t *__restrict__ X, const uint16_t *__restrict__ dY,
+                                                          float *__restrict__ part) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int most = (cb.TZ * cb.TX * cb.TY + 15) & ~15;
+    unsigned char *ys = smem + (size_t)NCB * cb.region * 32;                     // [NOB][voxel][16]
+    int *table = reinterpret_cast<int *>(ys + (size_t)NOB * most * 32);          // [voxel] byte of its place
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ngc = ci / (16 * NCB), c0 = (blockIdx.y % ngc) * NCB * 16, o0 = (blockIdx.y / ngc) * NOB * 16;
+    const int t0 = w * WG_TAPS;
+    int off[WG_TAPS];
+#pragma unroll
+    for (int n = 0; n < WG_TAPS; n++) {
+        const int t = min(t0 + n, TAPS - 1);
+        off[n] = 32 * ((t % 3 - 1) + cb.LZ * (((t / 3) % 3 - 1) + cb.LX * (t / 9 - 1)));
+    }
+    f32x4 acc[WG_TAPS][NCB][NOB];
+#pragma unroll
+    for (int n = 0; n < WG_TAPS; n++)
+#pragma unroll
+        for (int c = 0; c < NCB; c++)
+#pragma unroll
+            for (int o = 0; o < NOB; o++) acc[n][c][o] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
+        int b = blk;
+        const int k0 = (b % cb.nbz) * cb.TZ;
+        b /= cb.nbz;
+        const int i0 = (b % cb.nbx) * cb.TX;
+        b /= cb.nbx;
+        const int j0 = (b % cb.nby) * cb.TY, batch = b / cb.nby;
+        const int tz = min(cb.TZ, g.nz - k0), tx = min(cb.TX, g.nx - i0), ty = min(cb.TY, g.ny - j0);
+        const int count = tz * tx * ty;   // the block's voxels inside the grid, z fastest
+        if (blk != (int)blockIdx.x) __syncthreads();   // the last block's reads
+        stage_region<NCB>(g, cb, X + (size_t)batch * g.nv * ci + c0, ci, k0, i0, j0, smem, lane, w);
+        for (int v = threadIdx.x; v < ((count + 15) & ~15); v += CONV_TPB) {
+            const int vc = min(v, count - 1), z = vc % tz, x = (vc / tz) % tx, y = vc / (tz * tx);
+            table[v] = (1 + ((y + 1) * cb.LX + x + 1) * cb.LZ + z + 1) * 32;
+            const uint16_t *src = dY + ((size_t)batch * g.nv + k0 + z + (size_t)g.nz * (i0 + x + (size_t)g.nx * (j0 + y))) * co + o0;
+#pragma unroll
+            for (int o = 0; o < NOB; o++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    uint4 q = *reinterpret_cast<const uint4 *>(src + o * 16 + h * 8);
+                    if (v >= count) q = make_uint4(0, 0, 0, 0);
+                    *reinterpret_cast<uint4 *>(ys + ((size_t)o * most + v) * 32 + h * 16) = q;
+                }
+        }
+        __syncthreads();
+        const int row = 4 * (lane >> 4) + ((lane & 15) >> 2), quad = (lane & 3) * 8;   // what this lane reads of 16 voxels
+        const bf16x4 one = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
+        for (int v0 = 0; v0 < count; v0 += 16) {
+            const unsigned char *xp = smem + table[v0 + row] + quad;
+            bf16x4 y[NOB];
+#pragma unroll
+            for (int o = 0; o < NOB; o++) y[o] = lds_read_tr(ys + ((size_t)o * most + v0 + row) * 32 + quad);
+            const bool whole = v0 + 16 <= count;
+#pragma unroll
+            for (int n = 0; n < WG_TAPS; n++) {
+                const bool bias = t0 + n == TAPS;   // uniform; more taps than that are not there
+#pragma unroll
+                for (int c = 0; c < NCB; c++) {
+                    bf16x4 x = lds_read_tr(xp + off[n] + (size_t)c * cb.region * 32);
+                    if (bias) x = one;
+                    if (!whole)   // past the block: neither operand counts, whatever the region holds there
+#pragma unroll
+                        for (int e = 0; e < 4; e++) x[e] = v0 + 4 * (lane >> 4) + e < count ? x[e] : (short)0;
+#pragma unroll
+                    for (int o = 0; o < NOB; o++)
+                        acc[n][c][o] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(y[o], x, acc[n][c][o], 0, 0, 0);
+                }
+            }
+        }
+    }
+    // D[4(l/16)+i][l%16] = dW[o0 + 16 o + 4(l/16)+i][t][c0 + 16 c + l%16]
+    const int r = lane & 15, kq = 4 * (lane >> 4);
+    float *P = part + (size_t)blockIdx.x * ((size_t)co * TAPS * ci + co);
+#pragma unroll
+    for (int n = 0; n < WG_TAPS; n++) {
+        const int t = t0 + n;
+#pragma unroll
+        for (int o = 0; o < NOB; o++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const size_t oc = o0 + o * 16 + kq + i;
+                if (t < TAPS)
+#pragma unroll
+                    for (int c = 0; c < NCB; c++) P[(oc * TAPS + t) * ci + c0 + c * 16 + r] = acc[n][c][o][i];
+                else if (t == TAPS && c0 == 0 && r == 0)
+                    P[(size_t)co * TAPS * ci + oc] = acc[n][0][o][i];
+            }
+    }
+}
+
+// out[i] = sum of the slots' i: 64 entries to a workgroup, a quarter of the slots to a wavefront
+__global__ void __launch_bounds__(256) k_sum_slots(const float *__restrict__ part, int nslots, long slot,
+                                                   float *__restrict__ out) {
+    __shared__ float sh[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const long i = (long)blockIdx.x * 64 + lane;
+    const int per = (nslots + 3) / 4, k1 = min(nslots, (w + 1) * per);
+    float s = 0.f;
+    if (i < slot)
+#pragma unroll 8
+        for (int k = w * per; k < k1; k++) s += part[(size_t)k * slot + i];
+    sh[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && i < slot) out[i] = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
+}
+
+template <int NCB, int NOB>
+int wgrad_launch(const Vol &g, int nb, int ci, int co, const uint16_t *x, const uint16_t *dy, float *part, long slots,
+                 hipStream_t s) {
+    auto kern = k_wgrad_block<NCB, NOB>;
+    static std::atomic<uint64_t> raised{0};
+    if (raise_lds((const void *)kern, raised)) return -1;
+    const int groups = (ci / (16 * NCB)) * (co / (16 * NOB));
+    // dY and the table take less than NOB + 1/8 blocks' regions
+    const ConvBlock cb = conv_block(g, nb, groups, NCB + NOB, 1 << 20, CONV_LDS * 8 / 9);
+    if (!cb.TZ) return -1;
+    const long blocks = (long)nb * cb.nbz * cb.nbx * cb.nby;
+    if (blocks >= 1L << 31) return -1;
+    // two workgroups to a CU; no more slots than the workspace has
+    const long nslots = std::min(std::min(blocks, slots), std::max(1L, 512L / groups));
+    const long most = ((long)cb.TZ * cb.TX * cb.TY + 15) & ~15L;
+    hipLaunchKernelGGL(kern, dim3((unsigned)nslots, groups), dim3(CONV_TPB),
+                       (size_t)NCB * cb.region * 32 + NOB * most * 32 + most * 4, s, g, cb, (int)blocks, ci, co, x, dy, part);
+    return (int)nslots;
+}
+
+}  // namespace
+
+namespace learn {
+
+// partial sums of at most `slots` slots of co*27*ci + co floats, then their
+// sum; for 16-byte aligned operands, 0 or -1
+int conv_wgrad(const Vol &g, int nb, int ci, int co, const uint16_t *x, const uint16_t *dy, float *part, long slots,
+               float *grad, hipStream_t s) {
+    if (!aligned(x, 16) || !aligned(dy, 16) || slots < 1) return -1;
+    const int ncb = ci / 16, nob = co / 16;
+    int n;
+#define WGRAD_CASE(NCB, NOB) wgrad_launch<NCB, NOB>(g, nb, ci, co, x, dy, part, slots, s)
+    if (ncb % 2 == 0) n = nob % 2 == 0 ? WGRAD_CASE(2, 2) : WGRAD_CASE(2, 1);
+    else if (ncb % 3 == 0) n = WGRAD_CASE(3, 1);
+    else n = nob % 2 == 0 ? WGRAD_CASE(1, 2) : WGRAD_CASE(1, 1);
+#undef WGRAD_CASE
+    if (n < 1) return -1;
+    const long slot = (long)co * TAPS * ci + co;
+    hipLaunchKernelGGL(k_sum_slots, dim3((unsigned)((slot + 63) / 64)), dim3(256), 0, s, part, n, slot, grad);
+    return 0;
+}
+
+}  // namespace learn
+
+namespace {
+
+// the same for less aligned operands: one wavefront per (voxel chunk, 16 output
+// channels, 16 input channels), its partial sums in its own slot
 constexpr int WCH = 512;   // voxels per chunk
 __global__ void __launch_bounds__(256) k_conv_bwd_weight_c(Vol g, int nb, int ci, int co,
                                                            const uint16_t *__restrict__ X,
@@ -412,14 +602,6 @@ __global__ void __launch_bounds__(256) k_conv_bwd_weight_c(Vol g, int nb, int ci
         dbias += __shfl_xor(dbias, 32, 64);
         if (l < 16) P[(size_t)co * TAPS * ci + o] = dbias;
     }
-}
-
-__global__ void k_sum_slots(const float *__restrict__ part, long nslots, long slot, float *__restrict__ out) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= slot) return;
-    float s = 0.f;
-    for (long k = 0; k < nslots; k++) s += part[k * slot + i];
-    out[i] = s;
 }
 
 // ---- grid transfers.  Coarse node c of a level lies on fine node 2c per
@@ -659,11 +841,14 @@ int cl_conv3d_bwd_weight_c(const uint16_t *x, const uint16_t *dy, int nb, int nx
     const Vol g{nx, ny, nz, nx * ny * nz};
     if (nb <= 0 || g.nv <= 0 || !chan_ok(ci) || !chan_ok(co)) return -1;
     const long chunks = (long)nb * ((g.nv + WCH - 1) / WCH);
+    if (conv_wgrad(g, nb, ci, co, x, dy, workspace, chunks, grad, st(stream)) == 0) return ret();
     const long waves = chunks * (co / 16) * (ci / 16);
     const long slot = (long)co * TAPS * ci + co;
+    if (chunks >= 1L << 31) return -1;
     hipLaunchKernelGGL(k_conv_bwd_weight_c, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st(stream), g, nb, ci,
                        co, x, dy, workspace);
-    hipLaunchKernelGGL(k_sum_slots, dim3(nblk(slot)), dim3(256), 0, st(stream), workspace, chunks, slot, grad);
+    hipLaunchKernelGGL(k_sum_slots, dim3((unsigned)((slot + 63) / 64)), dim3(256), 0, st(stream), workspace, (int)chunks,
+                       slot, grad);
     return ret();
 }
 

@@ -79,3 +79,35 @@ def test_eight_channel_transfers_same_bits(dims, ch):
         assert L.cl_interp(_p(shifted(coarse, by)), 2, *dims, ch, 0.125, _p(f2), None) == 0
         out.append((c2, f2))
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("dims", DIMS)
+def test_block_weight_gradient(dims):
+    """against the general kernel's (FP32 sums of the same products in another
+    order; the chunks' and the blocks' sums differ by rounding: 1e-5, as the
+    kernels are held to the restatement); values that are not finite spread to
+    the same entries"""
+    import torch
+    from citcom_amd import unet
+    from citcom_amd.learn import _p
+    L = unet._lib()
+    g = torch.Generator(device="cuda").manual_seed(7)
+    nv = dims[0] * dims[1] * dims[2]
+    for ci, co in CHANNELS + [(80, 16), (96, 48)]:
+        for nb, wild in ((1, False), (3, False), (2, True)):
+            x = torch.randn((nb, nv, ci), generator=g, device="cuda").bfloat16()
+            dy = torch.randn((nb, nv, co), generator=g, device="cuda").bfloat16()
+            if wild:
+                x[0, 0, 1] = float("inf")
+                x[1, nv // 2, ci - 1] = float("nan")
+                dy[0, nv - 1, 2] = float("-inf")
+            ws = torch.empty(L.cl_conv3d_bwd_weight_c_workspace(nb, *dims, ci, co) // 4, device="cuda")
+            out = []
+            for xx in (x, shifted(x, 1)):
+                gr = torch.full((co * 27 * ci + co,), 7.0, device="cuda")
+                assert L.cl_conv3d_bwd_weight_c(_p(xx), _p(dy), nb, *dims, ci, co, _p(gr), _p(ws), None) == 0
+                out.append(gr)
+            a, b = out
+            fine = torch.isfinite(b)
+            assert torch.equal(torch.isfinite(a), fine) and torch.equal(torch.isnan(a), torch.isnan(b)), (dims, ci, co)
+            assert float((a - b)[fine].norm()) <= 1e-5 * float(b[fine].norm()) + 1e-30, (dims, ci, co, nb)

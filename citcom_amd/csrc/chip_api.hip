@@ -657,7 +657,12 @@ int rebuild(chip_ctx *c) {
     // before the stiffness is rebuilt
     if (c->fact_pending) CHIP_CHECK(hipStreamWaitEvent(q, c->ev_fact, 0));
     for (int lev = c->levmax; lev > c->levmin; lev--) project_viscosity(q, c->L[lev], c->L[lev - 1]);
-    for (int lev = c->levmin; lev <= c->levmax; lev++) elt_g(q, c->L[lev]);
+    for (int lev = c->levmin; lev <= c->levmax; lev++) {
+        Level &L = c->L[lev];
+        if (L.eg_brick) continue;   // geometry only: as the last rebuild left it
+        elt_g(q, L);
+        L.eg_brick = L.brick;
+    }
     for (int lev = c->levmax; lev >= c->levmin; lev--) node_ks(q, c->L[lev], c->p);
     for (int lev = c->levmax; lev >= c->levmin; lev--) build_bpi(q, c->L[lev], c->p.precond);
     if (c->cnet_w) cnet_logeta(q, c->L[c->levmin], c->cnet_logeta);
@@ -983,6 +988,10 @@ int chip_upload(chip_ctx *c, const char *which, int lev, const void *host, long 
     }
     CHIP_CHECK(hipMemcpyAsync(ptr, host, n * elem, hipMemcpyHostToDevice, c->stream));
     CHIP_CHECK(hipStreamSynchronize(c->stream));
+    // element arrays that the compact geometry stands for
+    Level &L = c->L[lev < 0 ? c->levmax : lev];
+    if (ptr == L.GNX || ptr == L.GDA || ptr == L.ECO) return check_brick(c, L);
+    if (ptr == L.EG) L.eg_brick = false;
     return 0;
 }
 

@@ -30,6 +30,7 @@ constexpr int GDA_SZ = 11;  // Shape_function_dA: vpt[9] + ppt[2]
 constexpr int ECO_SZ = 13;  // COORD: centre[4] size[4] recip_size[4] area
 constexpr int TWW_SZ = 9;   // FNODE: node[9]
 constexpr int EG_SZ = 24;   // EG: g[24][1]
+constexpr int BRICK_SZ = 20; // compact geometry of a brick element
 
 // node flag bits (global_defs.h:65-89)
 constexpr unsigned VBX = 0x2, VBZ = 0x4, VBY = 0x8;
@@ -87,6 +88,10 @@ struct Level {
     float *GDA = nullptr;    // [nel][11]
     float *ECO = nullptr;    // [nel][13]
     float *TWW = nullptr;    // [nel][9]
+    // the same for brick elements, [BRICK_SZ][nel] (k_brick); whether GNX, GDA
+    // and ECO, and whether EG, are what it holds
+    float *GB = nullptr;
+    bool brick = false, eg_brick = false;
     float *MASS = nullptr;   // [nno]
     unsigned *NODE = nullptr;// [nno]
     float *iw = nullptr;     // interpolation weights n1,n2 per fine index: x[2*nox], z[2*noz], y[2*noy]
@@ -197,6 +202,7 @@ struct chip_ctx {
     bool fact_pending = false;
     bool direct_async = true;  // option "direct_async": 0 factors every time on the work stream
     unsigned *xcd_ids = nullptr;   // [16] set-up check of the XCD dispatch
+    int *brick_bad = nullptr;      // [1] check_brick's count
     // learned coarse-level correction (chip_set_coarse_net): a 3-D CNN on the
     // coarsest level in place of its smoother call; BF16 weights
     // [layers][16][27][16], FP32 biases [layers][16], output scales [3],
@@ -245,6 +251,8 @@ struct chip_ctx {
 namespace chip {
 // setup (chip_setup.cpp)
 int build_mesh(chip_ctx *c);
+// L.GB from the level's element arrays, and whether it stands for them
+int check_brick(chip_ctx *c, Level &L);
 // device buffers of the learned coarse-level correction (once per context)
 constexpr int CNET_MAX_LAYERS = 8;
 int alloc_coarse_net(chip_ctx *c);

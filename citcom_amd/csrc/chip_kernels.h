@@ -15,6 +15,8 @@ size_t lds_limit();
 // ---- stiffness rebuild --------------------------------------------------
 void visc_from_T(hipStream_t s, const chip_ctx *c, const float *T, float *evi);
 void project_viscosity(hipStream_t s, const Level &fine, const Level &coarse);
+// L.GB from the element arrays; *bad counts elements they do not reduce to
+void brick(hipStream_t s, const Level &L, int *bad);
 void elt_g(hipStream_t s, const Level &L);
 void node_ks(hipStream_t s, const Level &L, const chip_problem &p);
 void build_bpi(hipStream_t s, const Level &L, int precond);

@@ -13,6 +13,7 @@
 
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
 
 #include "chip_kernels.h"
 
@@ -2511,6 +2512,248 @@ __device__ void elt_block(const float *__restrict__ gnx, const float *__restrict
     }
 }
 
+// ---------------------------------------------------------------------------
+// Compact geometry of brick elements.  On a mesh given by one coordinate array
+// per axis every element is a brick, and its 192 shape-function derivatives
+// are twelve numbers: the derivative along an axis of node a at Gauss point q
+// depends on whether a and q lie on the same side along the other two axes,
+// and its sign on a's side along this one; the eight Jacobians are one, and
+// the 24 entries of elt_del three.  k_brick gathers them, entry by entry of
+// the arrays as the reference computes them, [BRICK_SZ][nel] so that elements
+// side by side are read side by side, and counts the elements whose arrays are
+// not reproduced bit for bit (those levels keep the arrays).  The kernels that
+// read the derivatives are bound by these bytes: 908 B an element as arrays
+// (a cache line per lane and entry), 80 B so.
+constexpr int CORNER_X[8] = {0, 1, 1, 0, 0, 1, 1, 0}, CORNER_Y[8] = {0, 0, 1, 1, 0, 0, 1, 1},
+              CORNER_Z[8] = {0, 0, 0, 0, 1, 1, 1, 1};
+constexpr int BRICK_B = 0, BRICK_J = 12, BRICK_E = 13, BRICK_SIZE = 16, BRICK_AREA = 19;
+
+// which of the four values of axis d: sides of a and q along the other axes
+__device__ constexpr int brick_idx(int d, int a, int q) {
+    const int x = CORNER_X[a] ^ CORNER_X[q], y = CORNER_Y[a] ^ CORNER_Y[q], z = CORNER_Z[a] ^ CORNER_Z[q];
+    return d == 0 ? y + 2 * z : d == 1 ? x + 2 * z : x + 2 * y;
+}
+__device__ constexpr bool brick_up(int d, int a) {
+    return (d == 0 ? CORNER_X[a] : d == 1 ? CORNER_Y[a] : CORNER_Z[a]) != 0;
+}
+
+__global__ void __launch_bounds__(64) k_brick(Geo g, const float *__restrict__ GNX, const float *__restrict__ GDA,
+                                              const float *__restrict__ ECO, float *__restrict__ GB, int *bad) {
+    const int e = blockIdx.x * 64 + threadIdx.x;
+    if (e >= g.nel) return;
+    const float *gnx = GNX + (size_t)e * GNX_SZ, *gda = GDA + (size_t)e * GDA_SZ, *eco = ECO + (size_t)e * ECO_SZ;
+    bool ok = true;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        float b[4];
+#pragma unroll
+        for (int q = 0; q < 8; q++) b[brick_idx(d, 6, q)] = gnx[64 * d + 8 * 6 + q];   // node 6: the far corner
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const float v = b[brick_idx(d, a, q)];
+                ok = ok && __float_as_uint(gnx[64 * d + 8 * a + q]) == __float_as_uint(brick_up(d, a) ? v : -v);
+            }
+            const float c = gnx[192 + 8 * d + 6];
+            ok = ok && __float_as_uint(gnx[192 + 8 * d + a]) == __float_as_uint(brick_up(d, a) ? c : -c);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) GB[(size_t)(BRICK_B + 4 * d + q) * g.nel + e] = b[q];
+        // get_elt_g: -(derivative at the centre) x weight, rounded once
+        GB[(size_t)(BRICK_E + d) * g.nel + e] = (float)(gnx[192 + 8 * d + 6] * (double)(8.0f * gda[10]));
+        GB[(size_t)(BRICK_SIZE + d) * g.nel + e] = eco[5 + d];
+    }
+#pragma unroll
+    for (int q = 2; q <= 8; q++) ok = ok && __float_as_uint(gda[q]) == __float_as_uint(gda[1]);
+    GB[(size_t)BRICK_J * g.nel + e] = gda[1];
+    GB[(size_t)BRICK_AREA * g.nel + e] = eco[12];
+    if (!ok) atomicAdd(bad, 1);
+}
+
+void brick(hipStream_t s, const Level &L, int *bad) {
+    hipLaunchKernelGGL(k_brick, dim3(nblk(L.g.nel, 64)), dim3(64), 0, s, L.g, L.GNX, L.GDA, L.ECO, L.GB, bad);
+}
+
+// k_node_ks (below) from the compact geometry: three wavefronts per 64-node
+// tile, wavefront P the 81 coefficients of y-plane dy = P - 1 in registers,
+// through the two or four elements times two planes of elements that hold them
+// in ascending element order.  The same products and sums: with self the
+// node, m its neighbour, row r, column c, an element adds
+//   sum over the Gauss points of (W lo) hi, lo and hi the derivatives (self
+//   along c, m along r) of the node with the smaller and the larger local
+//   number, + the Laplacian term on the diagonal, + visc aug e e
+// (the reference forms one of each pair and transposes; a node's own block is
+// read transposed).  Elements outside the mesh have weight 0.
+// Bound by FP64 arithmetic (about 17000 operations a node); 128x128x64
+// elements, finest level 1.7 ms, from the arrays (one thread a node) 12 to 17.
+__global__ void __launch_bounds__(192, 2) k_node_ks_brick(Geo g, const float *__restrict__ GB, const float *__restrict__ EVI,
+                                                          const unsigned *__restrict__ NODE, int aug_on, double aug,
+                                                          float *__restrict__ K, double *__restrict__ BI) {
+    const int lane = threadIdx.x & 63, P = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = blockIdx.x * 64 + lane;
+    const int col = colour_valid(g, q);
+    int k = 0, i = 0, j = 0;
+    if (col >= 0) colour_kij(g, col, q, k, i, j);
+    const int self = nid(g, k, i, j);
+    float acc[9][3][3];
+    double diag[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int b = 0; b < 9; b++)
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) acc[b][r][c] = 0.0f;
+#pragma unroll 1
+    for (int my = P == 2; my <= (P >= 1); my++) {   // element rows ey = j - 1 + my
+        const int by = P - my, ay = 1 - my;          // sides of m and of the node along y
+#pragma unroll
+        for (int mx = 0; mx < 2; mx++)
+#pragma unroll
+            for (int mz = 0; mz < 2; mz++) {
+                const int ez = k - 1 + mz, ex = i - 1 + mx, ey = j - 1 + my;
+                const bool ok = (unsigned)ez < (unsigned)g.elz && (unsigned)ex < (unsigned)g.elx &&
+                                (unsigned)ey < (unsigned)g.ely;
+                const int e = ok ? ez + g.elz * (ex + g.elx * ey) : 0;
+                const int ax = 1 - mx, az = 1 - mz;
+                const float *gb = GB + e;
+                float B[3][4], E[3];
+#pragma unroll
+                for (int f = 0; f < 12; f++) B[f / 4][f % 4] = gb[(size_t)(BRICK_B + f) * g.nel];
+#pragma unroll
+                for (int d = 0; d < 3; d++) E[d] = gb[(size_t)(BRICK_E + d) * g.nel];
+                const float jv = gb[(size_t)BRICK_J * g.nel];
+                float evi[8];
+                {
+                    const float4 v0 = *reinterpret_cast<const float4 *>(EVI + (size_t)e * 8);
+                    const float4 v1 = *reinterpret_cast<const float4 *>(EVI + (size_t)e * 8 + 4);
+                    evi[0] = v0.x, evi[1] = v0.y, evi[2] = v0.z, evi[3] = v0.w;
+                    evi[4] = v1.x, evi[5] = v1.y, evi[6] = v1.z, evi[7] = v1.w;
+                }
+                double W[8], visc = 0.0;
+#pragma unroll
+                for (int p = 0; p < 8; p++) {
+                    const float wf = (1.0f * jv) * evi[p];
+                    W[p] = ok ? (double)wf : 0.0;
+                    visc += evi[p];
+                }
+                visc = visc / 8;
+                const double va = ok && aug_on ? visc * aug : 0.0;
+                // values of the node (side ay) and of m (side by) along y: x and z
+                // derivatives by the Gauss point's y side, y derivatives' sign
+                float Sx[2][2], Sz[2][2], Sy[4], Mx[2][2], Mz[2][2], My[4];   // [y side][z side], [y side][x side]
+#pragma unroll
+                for (int y = 0; y < 2; y++)
+#pragma unroll
+                    for (int o = 0; o < 2; o++) {
+                        Sx[y][o] = ay ? B[0][(1 - y) + 2 * o] : B[0][y + 2 * o];
+                        Mx[y][o] = by ? B[0][(1 - y) + 2 * o] : B[0][y + 2 * o];
+                        Sz[y][o] = ay ? B[2][o + 2 * (1 - y)] : B[2][o + 2 * y];
+                        Mz[y][o] = by ? B[2][o + 2 * (1 - y)] : B[2][o + 2 * y];
+                    }
+#pragma unroll
+                for (int o = 0; o < 4; o++) {
+                    Sy[o] = ay ? B[1][o] : -B[1][o];
+                    My[o] = by ? B[1][o] : -B[1][o];
+                }
+                float S[3][8];
+#pragma unroll
+                for (int p = 0; p < 8; p++) {
+                    const int qx = CORNER_X[p], qy = CORNER_Y[p], qz = CORNER_Z[p];
+                    const float sx = Sx[qy][az ^ qz], sz = Sz[qy][ax ^ qx];
+                    S[0][p] = ax ? sx : -sx;
+                    S[1][p] = Sy[(ax ^ qx) + 2 * (az ^ qz)];
+                    S[2][p] = az ? sz : -sz;
+                }
+                const double ES[3] = {ax ? -E[0] : E[0], ay ? -E[1] : E[1], az ? -E[2] : E[2]};
+#pragma unroll
+                for (int bx = 0; bx < 2; bx++)
+#pragma unroll
+                    for (int bz = 0; bz < 2; bz++) {
+                        const int b = (mz + bz) + 3 * (mx + bx);
+                        // formed anew in each block: shared over the blocks the
+                        // products would not fit the registers
+#pragma unroll
+                        for (int p = 0; p < 8; p++) {
+                            asm volatile("" : "+v"(W[p]));
+#pragma unroll
+                            for (int d = 0; d < 3; d++) asm volatile("" : "+v"(S[d][p]));
+                        }
+                        double T[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, temp = 0.0;
+                        // local numbers: z first, then (x, y) in the order 00 10 11 01
+                        const int oa = ax ? 1 + ay : 3 * ay, ob = bx ? 1 + by : 3 * by;
+                        const bool self_lo = az != bz ? az == 0 : oa <= ob;
+                        auto sum = [&](auto lo) {
+#pragma unroll
+                            for (int p = 0; p < 8; p++) {
+                                const int qx = CORNER_X[p], qy = CORNER_Y[p], qz = CORNER_Z[p];
+                                const float mxv = Mx[qy][bz ^ qz], mzv = Mz[qy][bx ^ qx];
+                                const float M[3] = {bx ? mxv : -mxv, My[(bx ^ qx) + 2 * (bz ^ qz)], bz ? mzv : -mzv};
+                                double wl[3];   // W times the lower node's derivatives
+#pragma unroll
+                                for (int d = 0; d < 3; d++) wl[d] = W[p] * (lo.value ? S[d][p] : M[d]);
+#pragma unroll
+                                for (int r = 0; r < 3; r++)
+#pragma unroll
+                                    for (int c = 0; c < 3; c++) T[r][c] += lo.value ? wl[c] * M[r] : wl[r] * S[c][p];
+                                const float s = S[0][p] * M[0] + S[1][p] * M[1] + S[2][p] * M[2];
+                                temp += W[p] * s;
+                            }
+                        };
+                        if (self_lo) sum(std::true_type{});
+                        else sum(std::false_type{});
+                        T[0][0] += temp;
+                        T[1][1] += temp;
+                        T[2][2] += temp;
+                        if (aug_on) {
+                            const double EM[3] = {bx ? -E[0] : E[0], by ? -E[1] : E[1], bz ? -E[2] : E[2]};
+                            // m <= the node (in node order): the node's rows are the larger node's
+                            const int dx = mx + bx - 1, dz = mz + bz - 1;
+                            const bool nbig = P == 0 || (P == 1 && (dx < 0 || (dx == 0 && dz <= 0)));
+#pragma unroll
+                            for (int r = 0; r < 3; r++)
+#pragma unroll
+                                for (int c = 0; c < 3; c++) T[r][c] += nbig ? va * ES[r] * EM[c] : va * EM[c] * ES[r];
+                        }
+                        if (b == 4 && P == 1) {
+                            diag[0] += T[0][0];
+                            diag[1] += T[1][1];
+                            diag[2] += T[2][2];
+                        }
+#pragma unroll
+                        for (int r = 0; r < 3; r++)
+#pragma unroll
+                            for (int c = 0; c < 3; c++) {
+                                acc[b][r][c] = (float)(acc[b][r][c] + T[r][c]);
+                                asm volatile("" : "+v"(acc[b][r][c]));   // added here, not kept for the loop's end
+                            }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+    }
+    if (col < 0) return;
+    float *kq = K + ktile(q) + (size_t)(81 * P) * 64;
+    const unsigned fs = NODE[self];
+    const float wr[3] = {(fs & VBX) ? 0.0f : 1.0f, (fs & VBY) ? 0.0f : 1.0f, (fs & VBZ) ? 0.0f : 1.0f};
+#pragma unroll
+    for (int b = 0; b < 9; b++) {
+        const int km = k + b % 3 - 1, im = i + b / 3 - 1, jm = j + P - 1;
+        const bool ok = (unsigned)km < (unsigned)g.noz && (unsigned)im < (unsigned)g.nox && (unsigned)jm < (unsigned)g.noy;
+        const unsigned fm = NODE[ok ? nid(g, km, im, jm) : self];
+        const float wc[3] = {(fm & VBX) ? 0.0f : 1.0f, (fm & VBY) ? 0.0f : 1.0f, (fm & VBZ) ? 0.0f : 1.0f};
+        const bool own = b == 4 && P == 1;
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) kq[(b * 9 + r * 3 + c) * 64] = (own ? acc[b][c][r] : acc[b][r][c]) * (wr[r] * wc[c]) + 0.0f;
+    }
+    if (P == 1) {
+        BI[3 * self] = (float)1.0 / diag[0];
+        BI[3 * self + 1] = (float)1.0 / diag[1];
+        BI[3 * self + 2] = (float)1.0 / diag[2];
+    }
+}
+
 // construct_node_ks (Construct_arrays.c:359-535) restated per node: the block
 // coupling node n with neighbour m is the float accumulation, in element
 // order, of w_r ww_c elt_k[rows of max(n,m)][cols of min(n,m)] (BC weights
@@ -2599,6 +2842,11 @@ __global__ void __launch_bounds__(128) k_node_ks(Geo g, const float *__restrict_
 }
 
 void node_ks(hipStream_t s, const Level &L, const chip_problem &p) {
+    if (L.brick && L.eg_brick) {
+        hipLaunchKernelGGL(k_node_ks_brick, dim3(L.g.pitch / 64), dim3(192), 0, s, L.g, L.GB, L.EVI, L.NODE, p.aug_lagr,
+                           p.aug_number, L.K, L.BI);
+        return;
+    }
     hipLaunchKernelGGL(k_node_ks, dim3(nblk(L.g.pitch, 128)), dim3(128), 0, s, L.g, L.GNX, L.GDA, L.EVI, L.EG, L.NODE,
                        p.aug_lagr, p.aug_number, L.K, L.BI);
 }

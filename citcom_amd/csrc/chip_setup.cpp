@@ -287,6 +287,18 @@ int alloc_warm_net(chip_ctx *c) {
     return 0;
 }
 
+int check_brick(chip_ctx *c, Level &L) {
+    if (!c->brick_bad && dev_alloc(c, &c->brick_bad, 1)) return -1;
+    int bad = 0;
+    CHIP_CHECK(hipMemcpyAsync(c->brick_bad, &bad, sizeof bad, hipMemcpyHostToDevice, c->stream));
+    brick(c->stream, L, c->brick_bad);
+    CHIP_CHECK(hipMemcpyAsync(&bad, c->brick_bad, sizeof bad, hipMemcpyDeviceToHost, c->stream));
+    CHIP_CHECK(hipStreamSynchronize(c->stream));
+    L.brick = bad == 0;
+    L.eg_brick = false;   // until elt_g forms EG from it
+    return 0;
+}
+
 int build_mesh(chip_ctx *c) {
     const chip_problem &p = c->p;
     Master m;
@@ -406,6 +418,7 @@ int build_mesh(chip_ctx *c) {
             dev_upload(c, &L.ECO, h.ECO) || dev_upload(c, &L.TWW, h.TWW) || dev_upload(c, &L.MASS, h.MASS) ||
             dev_upload(c, &L.iw, h.iw))
             return -1;
+        if (dev_alloc(c, &L.GB, (size_t)g.nel * BRICK_SZ) || check_brick(c, L)) return -1;
         if (dev_alloc(c, &L.K, (size_t)KROW * g.pitch) || dev_alloc(c, &L.BI, 3 * (size_t)g.nno) ||
             dev_alloc(c, &L.BPI, g.nel) || dev_alloc(c, &L.EG, (size_t)g.nel * EG_SZ) ||
             dev_alloc(c, &L.EVI, (size_t)g.nel * 8) || dev_alloc(c, &L.VN, g.nno) ||

@@ -146,13 +146,12 @@ struct chip_ctx {
     double *U = nullptr, *P = nullptr, *F = nullptr;
     float *T = nullptr, *Tdot = nullptr, *V = nullptr, *buoy = nullptr;
     float *T1 = nullptr, *Tdot1 = nullptr;
-    double *Eres = nullptr;  // [nel][8] element residual / element force scratch
+    double *Eres = nullptr;  // [8][nel] element residual / element force scratch, and what lies between
     float *TB = nullptr;     // [nno] boundary temperature (TB[3])
     float *expansivity = nullptr, *diffusivity = nullptr; // [noz]
     float *xc_d = nullptr, *yc_d = nullptr;               // finest coordinates per axis
     int *mat = nullptr;      // [nel] material group (1-based ids)
     float *H = nullptr;      // [noz] horizontal average
-    float *hf = nullptr;     // [nno] nodal heat flux
     float *Have = nullptr;   // [3 noz] layer averages of T, |V|^2, viscosity (chip_averages)
     float *ave_scratch = nullptr;  // [nno]
     // Uzawa vectors

@@ -2553,7 +2553,7 @@ __global__ void __launch_bounds__(64) k_brick(Geo g, const float *__restrict__ G
 #pragma unroll
             for (int q = 0; q < 8; q++) {
                 const float v = b[brick_idx(d, a, q)];
-                ok = ok && __float_as_uint(gnx[64 * d + 8 * a + q]) == __float_as_uint(brick_up(d, a) ? v : -v);
+                ok = ok && isfinite(v) && __float_as_uint(gnx[64 * d + 8 * a + q]) == __float_as_uint(brick_up(d, a) ? v : -v);
             }
             const float c = gnx[192 + 8 * d + 6];
             ok = ok && __float_as_uint(gnx[192 + 8 * d + a]) == __float_as_uint(brick_up(d, a) ? c : -c);
@@ -2566,6 +2566,7 @@ __global__ void __launch_bounds__(64) k_brick(Geo g, const float *__restrict__ G
     }
 #pragma unroll
     for (int q = 2; q <= 8; q++) ok = ok && __float_as_uint(gda[q]) == __float_as_uint(gda[1]);
+    ok = ok && isfinite(gda[1]);   // elements outside the mesh count as 0 times these
     GB[(size_t)BRICK_J * g.nel + e] = gda[1];
     GB[(size_t)BRICK_AREA * g.nel + e] = eco[12];
     if (!ok) atomicAdd(bad, 1);
@@ -2574,6 +2575,38 @@ __global__ void __launch_bounds__(64) k_brick(Geo g, const float *__restrict__ G
 void brick(hipStream_t s, const Level &L, int *bad) {
     hipLaunchKernelGGL(k_brick, dim3(nblk(L.g.nel, 64)), dim3(64), 0, s, L.g, L.GNX, L.GDA, L.ECO, L.GB, bad);
 }
+
+// one element's geometry, from the compact form or from the arrays (d: axis,
+// a: node, q: Gauss point, from 0)
+template <bool BRICK>
+struct ElemGeo {
+    const float *gnx, *gda, *eco;
+    float b[12], j, size[3];
+    __device__ __forceinline__ ElemGeo(const Geo &g, const float *GB, const float *GNX, const float *GDA,
+                                       const float *ECO, int e) {
+        if constexpr (BRICK) {
+#pragma unroll
+            for (int f = 0; f < 12; f++) b[f] = GB[(size_t)(BRICK_B + f) * g.nel + e];
+            j = GB[(size_t)BRICK_J * g.nel + e];
+#pragma unroll
+            for (int d = 0; d < 3; d++) size[d] = GB[(size_t)(BRICK_SIZE + d) * g.nel + e];
+        } else {
+            gnx = GNX + (size_t)e * GNX_SZ, gda = GDA + (size_t)e * GDA_SZ, eco = ECO + (size_t)e * ECO_SZ;
+        }
+    }
+    __device__ __forceinline__ float dN(int d, int a, int q) const {
+        if constexpr (BRICK) return brick_up(d, a) ? b[4 * d + brick_idx(d, a, q)] : -b[4 * d + brick_idx(d, a, q)];
+        else return gnx[64 * d + 8 * a + q];
+    }
+    // values derived from these are formed anew after this point
+    __device__ __forceinline__ void hold() {
+        if constexpr (BRICK)
+#pragma unroll
+            for (int f = 0; f < 12; f++) asm volatile("" : "+v"(b[f]));
+    }
+    __device__ __forceinline__ float dA(int q) const { return BRICK ? j : gda[q + 1]; }
+    __device__ __forceinline__ float len(int d) const { return BRICK ? size[d] : eco[5 + d]; }
+};
 
 // k_node_ks (below) from the compact geometry: three wavefronts per 64-node
 // tile, wavefront P the 81 coefficients of y-plane dy = P - 1 in registers,
@@ -2889,38 +2922,52 @@ __device__ __forceinline__ unsigned ford(float f) {
 }
 
 // std_timestep (Advection_diffusion.c:737-810): per-element advective limit
-// min into minmax[0]; Tmax (Global_operations.c:394-406) into minmax[1]
-__global__ void __launch_bounds__(TPB) k_timestep_tmax(Geo g, const float *__restrict__ ECO, const float *__restrict__ V,
-                                                       const float *__restrict__ T, unsigned *minmax) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+// min into minmax[0]; Tmax (Global_operations.c:394-406) into minmax[1].
+// The sizes lie ECO_SZ apart in ECO and side by side in the compact geometry
+// (stride nel).  One atomic per wavefront on the same two words was the whole
+// of it (387 us at 128x128x64 elements, so 21): up to 1024 workgroups go over
+// the mesh, and one adds only what the words do not hold already.
+__global__ void __launch_bounds__(TPB) k_timestep_tmax(Geo g, const float *__restrict__ size, int se, long sd,
+                                                       const float *__restrict__ V, const float *__restrict__ T,
+                                                       unsigned *minmax) {
+    __shared__ unsigned sh[2][TPB / 64];
     unsigned mn = ford(1.0e8f), mx = ford(-10.0f);
-    if (V && t < g.nel) {
-        const int e = t;
-        const int ez = e % g.elz, ex = (e / g.elz) % g.elx, ey = e / (g.elz * g.elx);
-        float uc1 = 0.0f, uc2 = 0.0f, uc3 = 0.0f;
+    for (int t = blockIdx.x * TPB + threadIdx.x; t < max(g.nel, g.nno); t += gridDim.x * TPB) {
+        if (V && t < g.nel) {
+            const int e = t;
+            const int ez = e % g.elz, ex = (e / g.elz) % g.elx, ey = e / (g.elz * g.elx);
+            float uc1 = 0.0f, uc2 = 0.0f, uc3 = 0.0f;
 #pragma unroll
-        for (int a = 1; a <= 8; a++) {
-            const int nd = nid(g, ez + cOffz[a], ex + cOffx[a], ey + cOffy[a]);
-            uc1 = (float)(uc1 + cNp[a - 1] * V[nd]);
-            uc2 = (float)(uc2 + cNp[a - 1] * V[g.nno + nd]);
-            uc3 = (float)(uc3 + cNp[a - 1] * V[2 * g.nno + nd]);
+            for (int a = 1; a <= 8; a++) {
+                const int nd = nid(g, ez + cOffz[a], ex + cOffx[a], ey + cOffy[a]);
+                uc1 = (float)(uc1 + cNp[a - 1] * V[nd]);
+                uc2 = (float)(uc2 + cNp[a - 1] * V[g.nno + nd]);
+                uc3 = (float)(uc3 + cNp[a - 1] * V[2 * g.nno + nd]);
+            }
+            const float *h = size + (size_t)e * se;
+            const float uc = (float)(fabs((double)uc1) / h[0] + fabs((double)uc2) / h[sd] + fabs((double)uc3) / h[2 * sd]);
+            const float step = (float)(0.5 / uc);
+            mn = min(mn, ford(step));
         }
-        const float *eco = ECO + (size_t)e * ECO_SZ;
-        const float uc = (float)(fabs((double)uc1) / eco[5] + fabs((double)uc2) / eco[6] + fabs((double)uc3) / eco[7]);
-        const float step = (float)(0.5 / uc);
-        mn = ford(step);
+        if (t < g.nno) mx = max(mx, ford(T[t]));
     }
-    if (t < g.nno) mx = ford(T[t]);
-    // wave reductions, then one atomic per wave
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         mn = min(mn, (unsigned)__shfl_down((int)mn, o, 64));
         mx = max(mx, (unsigned)__shfl_down((int)mx, o, 64));
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicMin(&minmax[0], mn);
-        atomicMax(&minmax[1], mx);
+        sh[0][threadIdx.x >> 6] = mn;
+        sh[1][threadIdx.x >> 6] = mx;
     }
+    __syncthreads();
+    if (threadIdx.x) return;
+    for (int w = 1; w < TPB / 64; w++) {
+        mn = min(mn, sh[0][w]);
+        mx = max(mx, sh[1][w]);
+    }
+    if (mn < __hip_atomic_load(&minmax[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&minmax[0], mn);
+    if (mx > __hip_atomic_load(&minmax[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&minmax[1], mx);
 }
 
 __global__ void k_minmax_init(unsigned *minmax) {
@@ -2931,8 +2978,12 @@ __global__ void k_minmax_init(unsigned *minmax) {
 void timestep_tmax(hipStream_t s, chip_ctx *c, const float *V, const float *T) {
     const Level &L = c->L[c->levmax];
     hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(1), 0, s, c->minmax);
-    hipLaunchKernelGGL(k_timestep_tmax, dim3(nblk(std::max(L.g.nel, L.g.nno))), dim3(TPB), 0, s, L.g, L.ECO, V, T,
-                       c->minmax);
+    const int nb = std::min(nblk(std::max(L.g.nel, L.g.nno)), 1024);
+    if (L.brick)
+        hipLaunchKernelGGL(k_timestep_tmax, dim3(nb), dim3(TPB), 0, s, L.g, L.GB + (size_t)BRICK_SIZE * L.g.nel, 1,
+                           (long)L.g.nel, V, T, c->minmax);
+    else
+        hipLaunchKernelGGL(k_timestep_tmax, dim3(nb), dim3(TPB), 0, s, L.g, L.ECO + 5, ECO_SZ, 1L, V, T, c->minmax);
 }
 
 void tmax(hipStream_t s, chip_ctx *c, const float *T) { timestep_tmax(s, c, nullptr, T); }
@@ -2950,9 +3001,15 @@ void predictor(hipStream_t s, const Level &L, float *T, float *Tdot, float mult)
 }
 
 // pg_shape_fn + element_residual (Advection_diffusion.c:448-727, CART3D,
-// diffusion on, no FBZ flux nodes): Eres[e][a] for the 8 nodes of element e
-__global__ void __launch_bounds__(TPB) k_pg_residual(Geo g, const float *__restrict__ GNX, const float *__restrict__ GDA,
-                                                     const float *__restrict__ ECO, const unsigned *__restrict__ NODE,
+// diffusion on, no FBZ flux nodes): Eres[a][e] for the 8 nodes of element e
+// (elements side by side, for this store and the gather's reads).  Bound by
+// FP64 arithmetic with the compact geometry; by the arrays' reads without it
+// (128x128x64 elements 105 us, from the arrays, every entry a cache line per
+// lane, 713).
+template <bool BRICK>
+__global__ void __launch_bounds__(TPB, 3) k_pg_residual(Geo g, const float *__restrict__ GB, const float *__restrict__ GNX,
+                                                     const float *__restrict__ GDA, const float *__restrict__ ECO,
+                                                     const unsigned *__restrict__ NODE,
                                                      const float *__restrict__ diffusivity, double Q,
                                                      const float *__restrict__ T, const float *__restrict__ Tdot,
                                                      const float *__restrict__ V, double *__restrict__ Eres) {
@@ -2960,9 +3017,7 @@ __global__ void __launch_bounds__(TPB) k_pg_residual(Geo g, const float *__restr
     if (el >= g.nel) return;
     const int ez = el % g.elz, ex = (el / g.elz) % g.elx, ey = el / (g.elz * g.elx);
     const float diff = (float)((diffusivity[ez] + diffusivity[ez + 1]) * 0.5);
-    const float *gnx = GNX + (size_t)el * GNX_SZ;
-    const float *gda = GDA + (size_t)el * GDA_SZ;
-    const float *eco = ECO + (size_t)el * ECO_SZ;
+    ElemGeo<BRICK> eg(g, GB, GNX, GDA, ECO, el);
     int nodes[9];
     float v1n[9], v2n[9], v3n[9];
 #pragma unroll
@@ -2981,70 +3036,60 @@ __global__ void __launch_bounds__(TPB) k_pg_residual(Geo g, const float *__restr
         uc3 += cNp[a - 1] * v3n[a];
     }
     const double twodiff = 2.0 * diff;
-    const double uxse = fabs(uc1 * (double)eco[5]), ueta = fabs(uc2 * (double)eco[6]), ufai = fabs(uc3 * (double)eco[7]);
+    const double uxse = fabs(uc1 * (double)eg.len(0)), ueta = fabs(uc2 * (double)eg.len(1)), ufai = fabs(uc3 * (double)eg.len(2));
     const double xse = (uxse > twodiff) ? (1.0 - twodiff / uxse) : 0.0;
     const double eta = (ueta > twodiff) ? (1.0 - twodiff / ueta) : 0.0;
     const double fai = (ufai > twodiff) ? (1.0 - twodiff / ufai) : 0.0;
     const double unorm = uc1 * uc1 + uc2 * uc2 + uc3 * uc3;
     const double adiff = (unorm > 0.000001) ? ((uxse * xse + ueta * eta + ufai * fai) / (2.0 * unorm)) : 0.0;
-    // element_residual: gauss-point values
-    double dT[9], tx1[9], tx2[9], tx3[9], v1[9], v2[9], v3[9];
-#pragma unroll
-    for (int i = 1; i <= 8; i++) dT[i] = tx1[i] = tx2[i] = tx3[i] = v1[i] = v2[i] = v3[i] = 0.0;
+    // element_residual, one Gauss point after the other
+    float Tn[9], DT[9];
+    double r[9];
 #pragma unroll
     for (int j = 1; j <= 8; j++) {
-        const int node = nodes[j];
-        const double Tn = T[node];
-        const double DT = (NODE[node] & (TBX | TBY | TBZ)) ? 0.0 : (double)Tdot[node];
-#pragma unroll
-        for (int i = 1; i <= 8; i++) {
-            const double sfn = cNv[8 * (j - 1) + i - 1];
-            dT[i] += DT * sfn;
-            tx1[i] += gnx[8 * (j - 1) + i - 1] * Tn;
-            tx2[i] += gnx[64 + 8 * (j - 1) + i - 1] * Tn;
-            tx3[i] += gnx[128 + 8 * (j - 1) + i - 1] * Tn;
-            v1[i] += v1n[j] * sfn;
-            v2[i] += v2n[j] * sfn;
-            v3[i] += v3n[j] * sfn;
-        }
+        Tn[j] = T[nodes[j]];
+        DT[j] = Tdot[nodes[j]];
+        if (NODE[nodes[j]] & (TBX | TBY | TBZ)) DT[j] = 0.0f;
+        r[j] = 0.0;
     }
-    double u1g[9], u2g[9], u3g[9];
 #pragma unroll
     for (int i = 1; i <= 8; i++) {
-        double a1 = 0.0, a2 = 0.0, a3 = 0.0;
+        eg.hold();
+        double dT = 0.0, tx1 = 0.0, tx2 = 0.0, tx3 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
+#pragma unroll
+        for (int j = 1; j <= 8; j++) asm volatile("" : "+v"(Tn[j]), "+v"(DT[j]), "+v"(v1n[j]), "+v"(v2n[j]), "+v"(v3n[j]));
 #pragma unroll
         for (int j = 1; j <= 8; j++) {
             const double sfn = cNv[8 * (j - 1) + i - 1];
-            a1 += v1n[j] * sfn;
-            a2 += v2n[j] * sfn;
-            a3 += v3n[j] * sfn;
+            dT += DT[j] * sfn;
+            tx1 += eg.dN(0, j - 1, i - 1) * (double)Tn[j];
+            tx2 += eg.dN(1, j - 1, i - 1) * (double)Tn[j];
+            tx3 += eg.dN(2, j - 1, i - 1) * (double)Tn[j];
+            v1 += v1n[j] * sfn;
+            v2 += v2n[j] * sfn;
+            v3 += v3n[j] * sfn;
         }
-        u1g[i] = a1;
-        u2g[i] = a2;
-        u3g[i] = a3;
-    }
+        const float w = eg.dA(i - 1), dl = diff * 1.0f * w;
+        const double val = dT - Q + v1 * tx1 + v2 * tx2 + v3 * tx3;
 #pragma unroll
-    for (int j = 1; j <= 8; j++) {
-        double r = 0.0;
-#pragma unroll
-        for (int i = 1; i <= 8; i++) {
-            const float gx = gnx[8 * (j - 1) + i - 1], gy = gnx[64 + 8 * (j - 1) + i - 1], gz = gnx[128 + 8 * (j - 1) + i - 1];
-            const double prod1 = (u1g[i] * gx + u2g[i] * gy + u3g[i] * gz);
+        for (int j = 1; j <= 8; j++) {
+            const float gx = eg.dN(0, j - 1, i - 1), gy = eg.dN(1, j - 1, i - 1), gz = eg.dN(2, j - 1, i - 1);
+            const double prod1 = (v1 * gx + v2 * gy + v3 * gz);
             const double PG = cNv[8 * (j - 1) + i - 1] + adiff * prod1;
-            const float dl = diff * 1.0f * gda[i];
-            r -= PG * gda[i] * (dT[i] - Q + v1[i] * tx1[i] + v2[i] * tx2[i] + v3[i] * tx3[i]) +
-                 dl * (gx * tx1[i] + gy * tx2[i] + gz * tx3[i]);
+            r[j] -= PG * w * val + dl * (gx * tx1 + gy * tx2 + gz * tx3);
         }
-        Eres[(size_t)el * 8 + j - 1] = r;
+        __builtin_amdgcn_sched_barrier(0);   // else the next points' values take the registers of four wavefronts
     }
+#pragma unroll
+    for (int j = 1; j <= 8; j++) Eres[(size_t)(j - 1) * g.nel + el] = r[j];
 }
 
 void pg_residual(hipStream_t s, const chip_ctx *c, const float *T, const float *Tdot, const float *V, double *Eres) {
     const Level &L = c->L[c->levmax];
     // heating_adi = heating_visc = 0 and heating_latent = 1 (Instructions.c:376-381)
     const double Q = (c->p.Q0 - 0.0f + 0.0f) * 1.0f;
-    hipLaunchKernelGGL(k_pg_residual, dim3(nblk(L.g.nel)), dim3(TPB), 0, s, L.g, L.GNX, L.GDA, L.ECO, L.NODE,
-                       c->diffusivity, Q, T, Tdot, V, Eres);
+    hipLaunchKernelGGL(L.brick ? k_pg_residual<true> : k_pg_residual<false>, dim3(nblk(L.g.nel)), dim3(TPB), 0, s, L.g,
+                       L.GB, L.GNX, L.GDA, L.ECO, L.NODE, c->diffusivity, Q, T, Tdot, V, Eres);
 }
 
 // pg_solver's scatter and lumped-mass scaling (Advection_diffusion.c:423-437)
@@ -3065,7 +3110,7 @@ __global__ void __launch_bounds__(TPB) k_pg_gather(Geo g, const unsigned *__rest
                 if ((unsigned)ez >= (unsigned)g.elz) continue;
                 const int e = ez + g.elz * (ex + g.elx * ey);
                 const int a = cLoc[(k - ez) + 2 * (i - ex) + 4 * (j - ey)];
-                dt = (float)(dt + Eres[(size_t)e * 8 + a - 1]);
+                dt = (float)(dt + Eres[(size_t)(a - 1) * g.nel + e]);
             }
         }
     }
@@ -3101,44 +3146,80 @@ __global__ void k_buoy_raw(Geo g, float Ra, const float *__restrict__ expansivit
     b[n] = Ra * T[n] * expansivity[n % g.noz];
 }
 
-// horizontal average of a nodal field on node layer kz = blockIdx.x, with
-// the bilinear surface quadrature of get_global_1d_shape_fn
-__global__ void __launch_bounds__(TPB) k_horiz_ave(Geo g, const float *__restrict__ xc, const float *__restrict__ yc,
-                                                   const float *__restrict__ X, float *__restrict__ H) {
-    __shared__ double sh[4 * 16];
-    const int kz = blockIdx.x;
-    double v[2] = {0.0, 0.0};
-    for (int f = threadIdx.x; f < g.elx * g.ely; f += blockDim.x) {
-        const int ex = f / g.ely, ey = f % g.ely;
-        const int n1 = nid(g, kz, ex, ey), n2 = nid(g, kz, ex + 1, ey), n3 = nid(g, kz, ex + 1, ey + 1),
-                  n4 = nid(g, kz, ex, ey + 1);
-        const double xx1[5] = {0, xc[ex], xc[ex + 1], xc[ex + 1], xc[ex]};
-        const double xx2[5] = {0, yc[ey], yc[ey], yc[ey + 1], yc[ey + 1]};
-        double dG[5];
-#pragma unroll
-        for (int nint = 1; nint <= 4; nint++) {
-            double d11 = 0, d12 = 0, d21 = 0, d22 = 0;
-#pragma unroll
-            for (int ii = 1; ii <= 4; ii++) {
-                const double mx0 = cMxv[4 * (ii - 1) + nint - 1], mx1 = cMxv[16 + 4 * (ii - 1) + nint - 1];
-                d11 += xx1[ii] * mx0;
-                d12 += xx2[ii] * mx0;
-                d21 += xx1[ii] * mx1;
-                d22 += xx2[ii] * mx1;
-            }
-            dG[nint] = d11 * d22 - d12 * d21;
-        }
-        const float xv[5] = {0, X[n1], X[n2], X[n3], X[n4]};
-#pragma unroll
-        for (int d = 1; d <= 4; d++)
+// horizontal averages of a nodal field, with the bilinear surface quadrature of
+// get_global_1d_shape_fn gathered into one weight a column (its corners' shares
+// of the faces around it).  A workgroup takes 64 columns, a thread one face's
+// share of a weight and then a lane one node layer, so that a column is read
+// as it lies; k_horiz_fin adds the workgroups' sums.  Bound by launches (16 us
+// at 129x129x65 nodes; one workgroup a layer, a cache line per value, 64).
+constexpr int HA_COLS = 64;
+
+__global__ void __launch_bounds__(256) k_horiz_part(Geo g, const float *__restrict__ xc, const float *__restrict__ yc,
+                                                    const float *__restrict__ X, double *__restrict__ part) {
+    __shared__ double share[4][HA_COLS], sum[4][64];
+    const int ncol = g.nox * g.noy, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    {
+        const int q = blockIdx.x * HA_COLS + lane, i = q % g.nox, j = q / g.nox;
+        const int ex = i - 1 + (w & 1), ey = j - 1 + (w >> 1);
+        double t = 0.0;
+        if (q < ncol && (unsigned)ex < (unsigned)g.elx && (unsigned)ey < (unsigned)g.ely) {
+            const int d = i == ex ? (j == ey ? 1 : 4) : (j == ey ? 2 : 3);   // the column's corner of the face
+            const double xx1[5] = {0, xc[ex], xc[ex + 1], xc[ex + 1], xc[ex]};
+            const double xx2[5] = {0, yc[ey], yc[ey], yc[ey + 1], yc[ey + 1]};
 #pragma unroll
             for (int nint = 1; nint <= 4; nint++) {
-                v[0] += xv[d] * cMv[4 * (d - 1) + nint - 1] * dG[nint];
-                v[1] += cMv[4 * (d - 1) + nint - 1] * dG[nint];
+                double d11 = 0, d12 = 0, d21 = 0, d22 = 0;
+#pragma unroll
+                for (int ii = 1; ii <= 4; ii++) {
+                    const double mx0 = cMxv[4 * (ii - 1) + nint - 1], mx1 = cMxv[16 + 4 * (ii - 1) + nint - 1];
+                    d11 += xx1[ii] * mx0;
+                    d12 += xx2[ii] * mx0;
+                    d21 += xx1[ii] * mx1;
+                    d22 += xx2[ii] * mx1;
+                }
+                t += cMv[4 * (d - 1) + nint - 1] * (d11 * d22 - d12 * d21);
             }
+        }
+        share[w][lane] = t;
     }
-    block_sum<2>(v, sh);
-    if (threadIdx.x == 0 && v[1] != 0.0) H[kz] = (float)(v[0] / v[1]);
+    __syncthreads();
+    const int k = blockIdx.y * 64 + lane;
+    const float *x = X + (size_t)blockIdx.x * HA_COLS * g.noz + k;
+    double v = 0.0, wt = 0.0;
+#pragma unroll 4
+    for (int q = w; q < HA_COLS; q += 4) {
+        const double c = share[0][q] + share[1][q] + share[2][q] + share[3][q];
+        if (blockIdx.x * HA_COLS + q < ncol) {
+            wt += c;
+            if (k < g.noz) v += c * x[(size_t)q * g.noz];
+        }
+    }
+    sum[w][lane] = v;
+    __syncthreads();
+    share[0][w] = wt;   // read above by all before the barrier
+    __syncthreads();
+    double *p = part + (size_t)blockIdx.x * (g.noz + 1);
+    if (w == 0 && k < g.noz) p[k] = sum[0][lane] + sum[1][lane] + sum[2][lane] + sum[3][lane];
+    if (threadIdx.x == 0 && blockIdx.y == 0) p[g.noz] = share[0][0] + share[0][1] + share[0][2] + share[0][3];
+}
+
+__global__ void __launch_bounds__(64) k_horiz_fin(Geo g, int nb, const double *__restrict__ part, float *__restrict__ H) {
+    double v = 0.0, w = 0.0;
+    for (int b = threadIdx.x; b < nb; b += 64) {
+        v += part[(size_t)b * (g.noz + 1) + blockIdx.x];
+        w += part[(size_t)b * (g.noz + 1) + g.noz];
+    }
+    v = wave_sum(v);
+    w = wave_sum(w);
+    if (threadIdx.x == 0 && w != 0.0) H[blockIdx.x] = (float)(v / w);
+}
+
+// part: noz + 1 doubles per 64 columns, of the element scratch
+void horiz_ave(hipStream_t s, const chip_ctx *c, const float *X, float *H) {
+    const Geo &g = c->L[c->levmax].g;
+    const int nb = nblk((long)g.nox * g.noy, HA_COLS);
+    hipLaunchKernelGGL(k_horiz_part, dim3(nb, nblk(g.noz, 64)), dim3(256), 0, s, g, c->xc_d, c->yc_d, X, c->Eres);
+    hipLaunchKernelGGL(k_horiz_fin, dim3(g.noz), dim3(64), 0, s, g, nb, c->Eres, H);
 }
 
 // averages (Process_velocity.c:179-224): per-layer horizontal averages of
@@ -3154,12 +3235,11 @@ __global__ void k_vsq(long nno, const float *__restrict__ V, float *__restrict__
 
 void averages(hipStream_t s, chip_ctx *c, float *Have /* [3 noz] */, float *scratch /* [nno] */) {
     Level &L = c->L[c->levmax];
-    hipLaunchKernelGGL(k_horiz_ave, dim3(L.g.noz), dim3(TPB), 0, s, L.g, c->xc_d, c->yc_d, c->T, Have);
+    horiz_ave(s, c, c->T, Have);
     hipLaunchKernelGGL(k_vsq, dim3(nblk(L.g.nno)), dim3(TPB), 0, s, (long)L.g.nno, c->V, scratch);
-    hipLaunchKernelGGL(k_horiz_ave, dim3(L.g.noz), dim3(TPB), 0, s, L.g, c->xc_d, c->yc_d, scratch, Have + L.g.noz);
+    horiz_ave(s, c, scratch, Have + L.g.noz);
     hipLaunchKernelGGL(k_visc_to_nodes, dim3(nblk(L.g.nno)), dim3(TPB), 0, s, L.g, L.EVI, L.TWW, L.MASS, scratch);
-    hipLaunchKernelGGL(k_horiz_ave, dim3(L.g.noz), dim3(TPB), 0, s, L.g, c->xc_d, c->yc_d, scratch,
-                       Have + 2 * L.g.noz);
+    horiz_ave(s, c, scratch, Have + 2 * L.g.noz);
 }
 
 __global__ void k_sub_layer(Geo g, const float *__restrict__ H, float *b) {
@@ -3171,7 +3251,7 @@ __global__ void k_sub_layer(Geo g, const float *__restrict__ H, float *b) {
 void thermal_buoyancy(hipStream_t s, const chip_ctx *c, const float *T, float *buoy) {
     const Level &L = c->L[c->levmax];
     hipLaunchKernelGGL(k_buoy_raw, dim3(nblk(L.g.nno)), dim3(TPB), 0, s, L.g, c->p.rayleigh, c->expansivity, T, buoy);
-    hipLaunchKernelGGL(k_horiz_ave, dim3(L.g.noz), dim3(TPB), 0, s, L.g, c->xc_d, c->yc_d, buoy, c->H);
+    horiz_ave(s, c, buoy, c->H);
     hipLaunchKernelGGL(k_sub_layer, dim3(nblk(L.g.nno)), dim3(TPB), 0, s, L.g, c->H, buoy);
 }
 
@@ -3198,7 +3278,7 @@ __global__ void __launch_bounds__(TPB) k_elt_f(Geo g, const float *__restrict__ 
         double f = 0.0;
 #pragma unroll
         for (int j = 1; j <= 8; j++) f += fg[j] * cNv[8 * (a - 1) + j - 1] * gda[j] * 1.0f;
-        Ef[(size_t)e * 8 + a - 1] = f;
+        Ef[(size_t)(a - 1) * g.nel + e] = f;
     }
 }
 
@@ -3216,7 +3296,7 @@ __global__ void __launch_bounds__(TPB) k_forces_gather(Geo g, const unsigned *__
             for (int ez = k - 1; ez <= k; ez++) {
                 if ((unsigned)ez >= (unsigned)g.elz) continue;
                 const int e = ez + g.elz * (ex + g.elx * ey);
-                acc += Ef[(size_t)e * 8 + cLoc[(k - ez) + 2 * (i - ex) + 4 * (j - ey)] - 1];
+                acc += Ef[(size_t)(cLoc[(k - ez) + 2 * (i - ex) + 4 * (j - ey)] - 1) * g.nel + e];
             }
         }
     }
@@ -3232,17 +3312,26 @@ void assemble_forces(hipStream_t s, const chip_ctx *c, const float *buoy, double
     hipLaunchKernelGGL(k_forces_gather, dim3(nblk(L.g.nno)), dim3(TPB), 0, s, L.g, L.NODE, c->Eres, F);
 }
 
-// heat_flux (Process_buoyancy.c:63-203)
-__global__ void __launch_bounds__(TPB) k_hf_elem(Geo g, const float *__restrict__ GNX, const float *__restrict__ GDA,
+// heat_flux (Process_buoyancy.c:63-203).  The surface values extrapolate from
+// the two node layers at each end of the columns, so only the element layers
+// that these touch (two at each end, all where there are fewer than four) are
+// integrated, only those nodes averaged (k_hf_columns: one thread a column and
+// end) and the columns summed by one workgroup (k_hf_surface).  Bound by launches
+// and latency: over the whole mesh 268 us at 128x128x64 elements, 140 of them one
+// workgroup on strided columns; so 30.
+template <bool BRICK>
+__global__ void __launch_bounds__(TPB) k_hf_elem(Geo g, int nl, const float *__restrict__ GB,
+                                                 const float *__restrict__ GNX, const float *__restrict__ GDA,
                                                  const float *__restrict__ ECO, const float *__restrict__ diffusivity,
                                                  const float *__restrict__ T, const float *__restrict__ V,
                                                  double *__restrict__ uTe) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= g.nel) return;
-    const int ez = e % g.elz, ex = (e / g.elz) % g.elx, ey = e / (g.elz * g.elx);
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nl * g.elx * g.ely) return;
+    const int ec = t / nl, l = t - ec * nl;
+    const int ez = l < 2 ? l : g.elz - nl + l, ex = ec % g.elx, ey = ec / g.elx;
+    const int e = ez + g.elz * ec;
     const double diff = (diffusivity[ez] + diffusivity[ez + 1]) * 0.5;
-    const float *gnx = GNX + (size_t)e * GNX_SZ;
-    const float *gda = GDA + (size_t)e * GDA_SZ;
+    const ElemGeo<BRICK> eg(g, GB, GNX, GDA, ECO, e);
     double VZ[9];
     float Tn[9];
 #pragma unroll
@@ -3259,11 +3348,11 @@ __global__ void __launch_bounds__(TPB) k_hf_elem(Geo g, const float *__restrict_
         for (int j = 1; j <= 8; j++) {
             u += VZ[j] * cNv[8 * (j - 1) + i - 1];
             Tg += Tn[j] * cNv[8 * (j - 1) + i - 1];
-            dTdz = dTdz + Tn[j] * gnx[128 + 8 * (j - 1) + i - 1];
+            dTdz = dTdz + Tn[j] * eg.dN(2, j - 1, i - 1);
         }
-        uT = uT + (u * Tg - diff * dTdz) * gda[i];
+        uT = uT + (u * Tg - diff * dTdz) * eg.dA(i - 1);
     }
-    uTe[e] = uT / ECO[(size_t)e * ECO_SZ + 12];
+    uTe[e] = uT / (BRICK ? GB[(size_t)BRICK_AREA * g.nel + e] : ECO[(size_t)e * ECO_SZ + 12]);
 }
 
 // Volume-RMS velocity (no counterpart in the reference): per element the Q1
@@ -3311,47 +3400,55 @@ void vrms(hipStream_t s, chip_ctx *c, const float *V, double *out2) {
          nullptr, nullptr, nullptr, nullptr, out2);
 }
 
-__global__ void __launch_bounds__(TPB) k_hf_gather(Geo g, const float *__restrict__ TWW, const float *__restrict__ MASS,
-                                                   const double *__restrict__ uTe, float *__restrict__ hf) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= g.nno) return;
-    int k, i, j;
-    node_kij(g, n, k, i, j);
-    float acc = 0.0f;
-    for (int ey = j - 1; ey <= j; ey++) {
-        if ((unsigned)ey >= (unsigned)g.ely) continue;
-        for (int ex = i - 1; ex <= i; ex++) {
-            if ((unsigned)ex >= (unsigned)g.elx) continue;
-            for (int ez = k - 1; ez <= k; ez++) {
-                if ((unsigned)ez >= (unsigned)g.elz) continue;
-                const int e = ez + g.elz * (ex + g.elx * ey);
-                const int a = cLoc[(k - ez) + 2 * (i - ex) + 4 * (j - ey)];
-                acc = (float)(acc + TWW[(size_t)e * TWW_SZ + a] * uTe[e]);
+// out: [2][ncol] surface values (bottom, top), then [2][nface] element areas
+__global__ void __launch_bounds__(TPB) k_hf_columns(Geo g, const float *__restrict__ TWW, const float *__restrict__ MASS,
+                                                    const float *__restrict__ ECO, const double *__restrict__ uTe,
+                                                    float *__restrict__ out) {
+    const int ncol = g.nox * g.noy, t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 2 * ncol) return;
+    const int top = t >= ncol, q = t - top * ncol, i = q % g.nox, j = q / g.nox;
+    float hf[2];
+#pragma unroll
+    for (int l = 0; l < 2; l++) {   // the surface node, the next one inwards
+        const int k = top ? g.noz - 1 - l : l;
+        float acc = 0.0f;
+        for (int ey = j - 1; ey <= j; ey++) {
+            if ((unsigned)ey >= (unsigned)g.ely) continue;
+            for (int ex = i - 1; ex <= i; ex++) {
+                if ((unsigned)ex >= (unsigned)g.elx) continue;
+                for (int ez = k - 1; ez <= k; ez++) {
+                    if ((unsigned)ez >= (unsigned)g.elz) continue;
+                    const int e = ez + g.elz * (ex + g.elx * ey);
+                    const int a = cLoc[(k - ez) + 2 * (i - ex) + 4 * (j - ey)];
+                    acc = (float)(acc + TWW[(size_t)e * TWW_SZ + a] * uTe[e]);
+                }
             }
         }
+        hf[l] = acc * MASS[nid(g, k, i, j)];
     }
-    hf[n] = acc * MASS[n];
+    out[t] = 2 * hf[0] - hf[1];
+    if (i < g.elx && j < g.ely) {
+        const int f = i + g.elx * j, nface = g.elx * g.ely;
+        out[2 * ncol + top * nface + f] = ECO[(size_t)(g.elz * f + (top ? g.elz - 1 : 0)) * ECO_SZ + 12];
+    }
 }
 
-// surface extrapolation and surface-element sums (Process_buoyancy.c:158-193)
-__global__ void __launch_bounds__(TPB) k_hf_surface(Geo g, const float *__restrict__ ECO, const float *__restrict__ hf,
-                                                    double *__restrict__ out) {
+// surface-element sums (Process_buoyancy.c:158-193)
+__global__ void __launch_bounds__(1024) k_hf_surface(Geo g, const float *__restrict__ col, double *__restrict__ out) {
     __shared__ double sh[4 * 16];
+    const int ncol = g.nox * g.noy, nface = g.elx * g.ely;
+    const float *area = col + 2 * ncol;
     double v[4] = {0, 0, 0, 0};
-    for (int f = threadIdx.x; f < g.elx * g.ely; f += blockDim.x) {
+    for (int f = threadIdx.x; f < nface; f += blockDim.x) {
         const int ex = f % g.elx, ey = f / g.elx;
-        double tb = 0.0, tt = 0.0;
         const int cols[4] = {ex + g.nox * ey, ex + 1 + g.nox * ey, ex + 1 + g.nox * (ey + 1), ex + g.nox * (ey + 1)};
+        double tb = 0.0, tt = 0.0;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int bot = cols[q] * g.noz, top = bot + g.noz - 1;
-            const float sh_ = 2 * hf[top] - hf[top - 1];
-            const float bh_ = 2 * hf[bot] - hf[bot + 1];
-            tb += bh_;
-            tt += sh_;
+            tb += col[cols[q]];
+            tt += col[ncol + cols[q]];
         }
-        const int eb = g.elz * (ex + g.elx * ey), et = eb + g.elz - 1;
-        const float ab = ECO[(size_t)eb * ECO_SZ + 12], at = ECO[(size_t)et * ECO_SZ + 12];
+        const float ab = area[f], at = area[nface + f];
         v[0] += tb * ab;
         v[1] += ab;
         v[2] += tt * at;
@@ -3364,10 +3461,14 @@ __global__ void __launch_bounds__(TPB) k_hf_surface(Geo g, const float *__restri
 
 void heat_flux(hipStream_t s, chip_ctx *c, const float *T, const float *V) {
     const Level &L = c->L[c->levmax];
-    hipLaunchKernelGGL(k_hf_elem, dim3(nblk(L.g.nel)), dim3(TPB), 0, s, L.g, L.GNX, L.GDA, L.ECO, c->diffusivity, T, V,
-                       c->Eres);
-    hipLaunchKernelGGL(k_hf_gather, dim3(nblk(L.g.nno)), dim3(TPB), 0, s, L.g, L.TWW, L.MASS, c->Eres, c->hf);
-    hipLaunchKernelGGL(k_hf_surface, dim3(1), dim3(TPB), 0, s, L.g, L.ECO, c->hf, c->dots + 24);
+    const Geo &g = L.g;
+    const int nl = std::min(g.elz, 4);
+    float *col = reinterpret_cast<float *>(c->Eres + g.nel);   // at most 6.5 values a face, of the scratch's 14 an element
+    hipLaunchKernelGGL(L.brick ? k_hf_elem<true> : k_hf_elem<false>, dim3(nblk((long)nl * g.elx * g.ely)), dim3(TPB), 0, s,
+                       g, nl, L.GB, L.GNX, L.GDA, L.ECO, c->diffusivity, T, V, c->Eres);
+    hipLaunchKernelGGL(k_hf_columns, dim3(nblk(2L * g.nox * g.noy)), dim3(TPB), 0, s, g, L.TWW, L.MASS, L.ECO, c->Eres,
+                       col);
+    hipLaunchKernelGGL(k_hf_surface, dim3(1), dim3(1024), 0, s, g, col, c->dots + 24);
 }
 
 // ---------------------------------------------------------------------------

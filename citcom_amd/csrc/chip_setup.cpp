@@ -499,7 +499,7 @@ int build_mesh(chip_ctx *c) {
     if (dev_alloc(c, &c->U, neq) || dev_alloc(c, &c->P, nel) || dev_alloc(c, &c->F, neq) ||
         dev_alloc(c, &c->T, nno) || dev_alloc(c, &c->Tdot, nno) || dev_alloc(c, &c->V, 3 * nno) ||
         dev_alloc(c, &c->buoy, nno) || dev_alloc(c, &c->T1, nno) || dev_alloc(c, &c->Tdot1, nno) ||
-        dev_alloc(c, &c->Eres, nel * 8) || dev_alloc(c, &c->H, g.noz) || dev_alloc(c, &c->hf, nno) ||
+        dev_alloc(c, &c->Eres, nel * 8) || dev_alloc(c, &c->H, g.noz) ||
         dev_alloc(c, &c->r0, nel) || dev_alloc(c, &c->r1, nel) || dev_alloc(c, &c->r2, nel) ||
         dev_alloc(c, &c->z0, nel) || dev_alloc(c, &c->z1, nel) || dev_alloc(c, &c->s1, nel) ||
         dev_alloc(c, &c->s2, nel) || dev_alloc(c, &c->Ah, neq) || dev_alloc(c, &c->u1, neq) ||

@@ -141,11 +141,13 @@ void mg_gs(chip_ctx *c, int lev, V *d, const V *F, V *Ad, int sweeps, int guess,
            V *res = nullptr) {
     const Level &L = c->L[lev];
     if (L.Ma && c->small_levels && sweeps == L.affine_sweeps) {
-        V *out;
-        if constexpr (sizeof(V) == sizeof(double)) out = L.tmp;
-        else out = L.tmpf;
+        V *out = d;
+        if (guess == 1) {
+            if constexpr (sizeof(V) == sizeof(double)) out = L.tmp;
+            else out = L.tmpf;
+        }
         affine_apply(S(c), L, guess == 1 ? (const V *)d : nullptr, F, out);
-        do_matvec(c, lev, (const V *)out, Ad, rhs, res, d);   // and d = out
+        do_matvec(c, lev, (const V *)out, Ad, rhs, res, out == d ? nullptr : d);   // and d = out
         return;
     }
     do_gs(c, lev, d, F, Ad, sweeps, guess, rhs, res);
@@ -252,6 +254,8 @@ void enqueue_cycles(chip_ctx *c, V *F) {
         else
             coarse_smooth(c, vel, rhs);
     };
+    // the way up to the level above the coarsest as one matrix of its residual
+    const bool joined = !direct && !c->cnet_on && c->small_levels && L[levmin + 1].Mu;
     for (int lev = levmax; lev > levmin; lev--) project(S(c), L[lev], L[lev - 1], (const V *)fl(lev), fl(lev - 1));
     bottom(vecs<V>(L[levmin]).vel, (const V *)fl(levmin));
     for (int lev = levmin + 1; lev <= levmax; lev++) {
@@ -265,16 +269,22 @@ void enqueue_cycles(chip_ctx *c, V *F) {
                 // the top of the V-cycle the smoother starts from zero, which
                 // the restriction above it has written
                 mg_gs(c, dlev, v.vel, (const V *)rhs, v.AU, cycles, dlev == lev ? 1 : 2, (const V *)rhs, v.res);
-                project(S(c), L[dlev], L[dlev - 1], (const V *)v.res, vecs<V>(L[dlev - 1]).fl, true,
-                        vecs<V>(L[dlev - 1]).vel);
+                if (!joined || dlev > levmin + 1)
+                    project(S(c), L[dlev], L[dlev - 1], (const V *)v.res, vecs<V>(L[dlev - 1]).fl, true,
+                            vecs<V>(L[dlev - 1]).vel);
             }
-            bottom(vecs<V>(L[levmin]).vel, (const V *)vecs<V>(L[levmin]).fl);
+            if (!joined) bottom(vecs<V>(L[levmin]).vel, (const V *)vecs<V>(L[levmin]).fl);
             for (int ulev = levmin + 1; ulev <= lev; ulev++) {
                 const LV<V> v = vecs<V>(L[ulev]);
                 const int cycles = (ulev == levmax) ? p.v_steps_high : p.up_heavy;
                 const long n = 3L * L[ulev].g.nno;
-                interp(S(c), L[ulev - 1], L[ulev], (const V *)vecs<V>(L[ulev - 1]).vel, v.del);
-                mg_gs(c, ulev, v.del, (const V *)v.res, v.AU, cycles, 1);
+                if (joined && ulev == levmin + 1) {
+                    up_apply(S(c), L[ulev], (const V *)v.res, v.del);
+                    do_matvec(c, ulev, (const V *)v.del, v.AU);
+                } else {
+                    interp(S(c), L[ulev - 1], L[ulev], (const V *)vecs<V>(L[ulev - 1]).vel, v.del);
+                    mg_gs(c, ulev, v.del, (const V *)v.res, v.AU, cycles, 1);
+                }
                 V *resout = ulev == levmax ? v.res : nullptr;
                 if (line_search_ok(n)) {
                     line_search(S(c), n, v.vel, (const V *)v.del, resout, (const V *)v.AU, (const V *)v.res,
@@ -666,9 +676,9 @@ int rebuild(chip_ctx *c) {
     for (int lev = c->levmax; lev >= c->levmin; lev--) node_ks(q, c->L[lev], c->p);
     for (int lev = c->levmax; lev >= c->levmin; lev--) build_bpi(q, c->L[lev], c->p.precond);
     if (c->cnet_w) cnet_logeta(q, c->L[c->levmin], c->cnet_logeta);
-    if (c->L[c->levmin].Mc) coarse_build(q, c->L[c->levmin], c->p.v_steps_low);
+    if (c->L[c->levmin].Mc && coarse_build(q, c->L[c->levmin], c->p.v_steps_low)) return -1;
     for (int lev = c->levmin; lev <= c->levmax; lev++)
-        if (c->L[lev].Ma) affine_build(q, c->L[lev], c->L[lev].affine_sweeps);
+        if (c->L[lev].Ma && affine_build(q, c->L[lev], c->L[lev - 1])) return -1;
     if (c->p.mixed)
         for (int lev = c->levmin; lev <= c->levmax; lev++) to_f32(q, c->L[lev].BIf, c->L[lev].BI, 3L * c->L[lev].g.nno);
     for (int lev = c->levmin; lev <= c->levmax; lev++)
@@ -1121,7 +1131,7 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
         CHIP_CHECK(down(out2, d, nv));
         CHIP_CHECK(hipStreamSynchronize(q));
     } else if (o == "affine0" || o == "affine1") {
-        if (!L.Ma) {
+        if (!L.Ma || lev != c->levmin + 1 || !affine_ok(L)) {
             set_error("affine: the level has no affine smoother form");
             return -1;
         }

@@ -74,6 +74,12 @@ struct XcdBar {
     unsigned pad;
 };
 
+// the maps of a level, in the order Ma, Mb, Mu
+struct MapSet {
+    double *m[3];
+    float *f[3];
+};
+
 struct Level {
     Geo g;
     // operator
@@ -100,11 +106,12 @@ struct Level {
     double *vel = nullptr, *res = nullptr, *fl = nullptr, *del = nullptr, *AU = nullptr;
     // coarsest level: its smoother call as a matrix [3nno][3nno], row-major
     double *Mc = nullptr;
-    // level above the coarsest: its smoother call as d = Ma din + Mb F
-    // ([3nno][3nno] each, row-major), for affine_sweeps sweeps; scratch
-    // vectors for the result in both precisions
-    double *Ma = nullptr, *Mb = nullptr;
-    float *Maf = nullptr, *Mbf = nullptr;   // FP32 copies for the FP32 cycles (mixed forms)
+    // small levels above the coarsest: the smoother call as d = Ma din + Mb F
+    // ([3nno][3nno] each, row-major), for affine_sweeps sweeps; right above the
+    // coarsest also the way up from a residual, Mu; scratch vectors for the
+    // result in both precisions
+    double *Ma = nullptr, *Mb = nullptr, *Mu = nullptr;
+    float *Maf = nullptr, *Mbf = nullptr, *Muf = nullptr;   // FP32 copies for the FP32 cycles (mixed forms)
     int affine_sweeps = 0;
     double *tmp = nullptr;
     float *tmpf = nullptr;

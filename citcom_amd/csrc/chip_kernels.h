@@ -70,9 +70,12 @@ void gs_box(hipStream_t s, const Level &L, const float *BI, const float *din, fl
 int xcd_colocated(hipStream_t s, int nwg, unsigned *ids_dev, bool *same);
 // level above the coarsest: its smoother call as d = Ma din + Mb F
 bool affine_ok(const Level &L);
-void affine_build(hipStream_t s, const Level &L, int sweeps);
+bool map_ok(const Level &L);
+int affine_build(hipStream_t s, const Level &L, const Level &coarse);
 template <typename V>
 void affine_apply(hipStream_t s, const Level &L, const V *din, const V *F, V *out);
+template <typename V>
+void up_apply(hipStream_t s, const Level &L, const V *res, V *out);
 // exact coarsest-level solve of the FP32 cycles: A (column-major, n = 3 nno)
 // <- the level's stiffness with identity rows and columns at fixed
 // components (zeroed first); M (row-major FP32) <- the symmetric matrix
@@ -84,7 +87,7 @@ void rowscale_f16(hipStream_t s, const float *M, uint16_t *H, float *sc, int n);
 template <typename V>
 void dense_apply(hipStream_t s, const uint16_t *H, const float *sc, const V *F, V *out, int n);
 // coarsest level: Mc = the v_steps_low-sweep smoother as a matrix, d = Mc F
-void coarse_build(hipStream_t s, const Level &L, int sweeps);
+int coarse_build(hipStream_t s, const Level &L, int sweeps);
 template <typename V>
 void coarse_apply(hipStream_t s, const Level &L, const V *F, V *d);
 // (zero, if given, is a coarse vector set to zero in the same launch)

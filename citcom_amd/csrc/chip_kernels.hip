@@ -1004,11 +1004,14 @@ __global__ void __launch_bounds__(SMALL_TPB) k_gs_lds(Geo g, const float *__rest
         for (int idx = tid; idx < 3 * nno; idx += blockDim.x) d[idx] = ds[idx];
 }
 
-// smoother calls applied as matrices on levels of at most this many dofs
-// (two FP64 matrices of 18 MB at most)
-constexpr long AFFINE_MAX_DOF = 1500;
+// the coarsest level's smoother call is a matrix on levels of at most this many
+// dofs, and with it the calls of the levels above it of at most MAP_MAX_DOF
+// (their rule beside k_map_columns)
+constexpr long AFFINE_MAX_DOF = 1500, MAP_MAX_DOF = 3300;
 
 bool affine_ok(const Level &L) { return 3L * L.g.nno <= AFFINE_MAX_DOF; }
+
+bool map_ok(const Level &L) { return 3L * L.g.nno <= MAP_MAX_DOF; }
 
 // largest level of the one-XCD smoother (k_gs_xcd, below): its FP32
 // stiffness (972 B a node) stays within about one XCD's 4 MB L2; polls per
@@ -1615,146 +1618,302 @@ void dense_apply(hipStream_t s, const uint16_t *H, const float *sc, const V *F, 
 template void dense_apply<double>(hipStream_t, const uint16_t *, const float *, const double *, double *, int);
 template void dense_apply<float>(hipStream_t, const uint16_t *, const float *, const float *, float *, int);
 
-// multi_grid (v_steps_low sweeps from a zero guess, General_matrix_functions.c
-// :574, :613) is linear in its right-hand side apart from the FP32 rounding
-// of each increment, and its Ad is not read afterwards.  Column j of Mc is
-// the smoother's result for e_j (one workgroup per column, rebuilt with the
-// stiffness); a call is then d = Mc F.
-
-__global__ void k_gs_unit(Geo g, const float *__restrict__ K, const double *__restrict__ BI, double *__restrict__ Ma,
-                          double *__restrict__ Mb, int sweeps);
-
-void coarse_build(hipStream_t s, const Level &L, int sweeps) {
-    const int nno = L.g.nno;
-    if (gs_small_kind(L))
-        hipLaunchKernelGGL(k_gs_lds, dim3(3 * nno), dim3(SMALL_TPB), kstage_bytes(nno) + vstage_bytes(nno), s, L.g,
-                           L.K, L.BI, L.NODE, L.Mc, nullptr, nullptr, sweeps, 0, 1);
-    else
-        hipLaunchKernelGGL(k_gs_unit, dim3(3 * nno), dim3(192), (size_t)3 * nno * 8, s, L.g, L.K, L.BI, nullptr, L.Mc,
-                           sweeps);
+// interp_vector + un_inject_vector (Solver_multigrid.c:173-298, 581-634):
+// injection, then linear fills along x, z, y in the reference's order; at(cn, d)
+// is component d of coarse node cn
+template <typename V, typename At>
+__device__ __forceinline__ void interp_node(const Geo &gc, const Geo &gf, const float *__restrict__ iw, int k, int i, int j,
+                                            At at, V v[3]) {
+    const float *wx = iw, *wz = iw + 2 * gf.nox, *wy = iw + 2 * (gf.nox + gf.noz);
+    // the (up to) 8 coarse nodes around the fine node are loaded together,
+    // then the linear fills along x, then z, then y: an odd fine index
+    // interpolates its two coarse neighbours n1 a + n2 b, an even one takes
+    // its single coarse value
+    const int kc[2] = {k >> 1, (k + 1) >> 1}, ic[2] = {i >> 1, (i + 1) >> 1}, jc[2] = {j >> 1, (j + 1) >> 1};
+    V c[2][2][2][3];   // [y][z][x][component]
+#pragma unroll
+    for (int yy = 0; yy < 2; yy++)
+#pragma unroll
+        for (int zz = 0; zz < 2; zz++)
+#pragma unroll
+            for (int xx = 0; xx < 2; xx++) {
+                const int cn = nid(gc, kc[zz], ic[xx], jc[yy]);
+#pragma unroll
+                for (int d = 0; d < 3; d++) c[yy][zz][xx][d] = at(cn, d);
+            }
+    const float nx1 = wx[2 * i], nx2 = wx[2 * i + 1], nz1 = wz[2 * k], nz2 = wz[2 * k + 1];
+    const float ny1 = wy[2 * j], ny2 = wy[2 * j + 1];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        V lx[2][2];
+#pragma unroll
+        for (int yy = 0; yy < 2; yy++)
+#pragma unroll
+            for (int zz = 0; zz < 2; zz++)
+                lx[yy][zz] = (i & 1) ? nx1 * c[yy][zz][0][d] + nx2 * c[yy][zz][1][d] : c[yy][zz][0][d];
+        V pz[2];
+#pragma unroll
+        for (int yy = 0; yy < 2; yy++) pz[yy] = (k & 1) ? nz1 * lx[yy][0] + nz2 * lx[yy][1] : lx[yy][0];
+        v[d] = (j & 1) ? ny1 * pz[0] + ny2 * pz[1] : pz[0];
+    }
 }
 
+constexpr int MAP_PAD = 2;
+
 // ---------------------------------------------------------------------------
-// The level above the coarsest as an affine operator.  Its gauss_seidel calls
-// in multi_grid (down_heavy = up_heavy sweeps) are, apart from the FP32
-// rounding of each increment, d_out = Ma d_in + Mb F (guess) or Mb F (zero
-// guess).  Column j of Ma is the smoother's result for d_in = e_j, F = 0;
-// column j of Mb for d_in = 0, F = e_j; one workgroup per column (three
-// wavefronts per 64-node tile, as k_gs_colour), d kept in LDS.
-// (Ma null: the Mb columns only, one workgroup each)
-__global__ void __launch_bounds__(192) k_gs_unit(Geo g, const float *__restrict__ K, const double *__restrict__ BI,
-                                                 double *__restrict__ Ma, double *__restrict__ Mb, int sweeps) {
+// Smoother calls of multi_grid as matrices.  On the coarsest level a call
+// (v_steps_low sweeps from a zero guess, General_matrix_functions.c:574, :613)
+// is linear in its right-hand side apart from the FP32 rounding of each
+// increment, and its Ad is not read afterwards: d = Mc F.  On the levels above
+// it (down_heavy = up_heavy sweeps) a call is likewise d = Ma d_in + Mb F, or
+// Mb F from a zero guess; and on the level right above the coarsest the way up
+// (restriction, coarsest call, prolongation, call with that guess) is one
+// matrix of the residual, Mu = Ma (P Mc R) + Mb.  The columns are the smoother's
+// results for unit vectors, formed when the stiffness is rebuilt.
+//
+// A sweep of such a level is bound by latency (two launches of 8 us whatever
+// its size), a map by reading 8 n^2 bytes; the FP64 cycle, three sweeps: 405
+// nodes 46 us -> 5.8, 729 nodes 47 us -> 11 to 12.  The line: a Stokes solve on
+// 20x20x16 elements (level of 1089 nodes) 41.7 ms with sweeps, 34.7 with maps;
+// on 20x20x20 (1331 nodes) 40.7 and 39.0, and with a rebuild a step 68.3 and
+// 69.2.  The columns are formed NC at a time by a workgroup that keeps them in
+// LDS; lanes are columns by nodes, so a stiffness entry is fetched once for NC
+// columns (one column a workgroup -> NC: 462 nodes, 20 sweeps 1.27 ms -> 1.02;
+// 405 nodes, two maps of three sweeps 0.29 -> 0.30; 729 nodes, three maps 0.9).
+
+// share of fine node (2k-1 + t%3, ...) in coarse node (k, i, j) by project_vector
+__device__ double project_share(const Geo &gc, const float *__restrict__ TWW, const float *__restrict__ MASS, int k,
+                                int i, int j, int t) {
+    const int tz = t % 3, tx = t / 3 % 3, ty = t / 9;
+    double w = 0.0;
+    for (int m = 0; m < 8; m++) {
+        const int oz = m & 1, ox = (m >> 1) & 1, oy = m >> 2;
+        const int ez = k - 1 + oz, ex = i - 1 + ox, ey = j - 1 + oy;
+        if ((unsigned)ez >= (unsigned)gc.elz || (unsigned)ex >= (unsigned)gc.elx || (unsigned)ey >= (unsigned)gc.ely) continue;
+        if ((unsigned)(tz - oz) > 1u || (unsigned)(tx - ox) > 1u || (unsigned)(ty - oy) > 1u) continue;
+        w += TWW[(size_t)(ez + gc.elz * (ex + gc.elx * ey)) * TWW_SZ + cLoc[(k - ez) + 2 * (i - ex) + 4 * (j - ey)]];
+    }
+    return w * MASS[nid(gc, k, i, j)];
+}
+
+// X = Mc R, R the restriction with multi_grid's strip: column j (a fine dof)
+// has the up to eight coarse nodes around it.  X [3 coarse nno][3 fine nno].
+__global__ void __launch_bounds__(256) k_map_restrict(Geo gf, Geo gc, const float *__restrict__ TWW,
+                                                      const float *__restrict__ MASS, const unsigned *__restrict__ NODE,
+                                                      const double *__restrict__ Mc, double *__restrict__ X) {
+    const int j = blockIdx.x * 256 + threadIdx.x, n3f = 3 * gf.nno, n3c = 3 * gc.nno;
+    if (j >= n3f) return;
+    const int d = j % 3;
+    int kf, xf, yf;
+    node_kij(gf, j / 3, kf, xf, yf);
+    const unsigned fixed = d == 0 ? VBX : d == 1 ? VBY : VBZ;
+    double wt[8];
+    int col[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+        const int k = (kf + (m & 1)) >> 1, i = (xf + ((m >> 1) & 1)) >> 1, y = (yf + (m >> 2)) >> 1;
+        // an even index has one coarse node, counted once
+        const bool twice = ((m & 1) && !(kf & 1)) || ((m & 2) && !(xf & 1)) || ((m & 4) && !(yf & 1));
+        const int n = nid(gc, k, i, y);
+        const int t = (kf - 2 * k + 1) + 3 * (xf - 2 * i + 1) + 9 * (yf - 2 * y + 1);
+        col[m] = 3 * n + d;
+        wt[m] = twice || (NODE[n] & fixed) ? 0.0 : project_share(gc, TWW, MASS, k, i, y, t);
+    }
+    for (int r = blockIdx.y; r < n3c; r += gridDim.y) {
+        double v = 0.0;
+#pragma unroll
+        for (int m = 0; m < 8; m++) v += Mc[(size_t)r * n3c + col[m]] * wt[m];
+        X[(size_t)r * n3f + j] = v;
+    }
+}
+
+// Map blockIdx.y + kind0 (0: Ma, 1: Mb, 2: Mu, whose first rows hold X on
+// entry), columns blockIdx.x NC ..: a level of one colour pass after the
+// other, each thread the three rows of a (node, column), in the order of
+// k_gs_colour.
+template <int NC>
+__global__ void __launch_bounds__(1024) k_map_columns(Geo g, Geo gc, const float *__restrict__ K,
+                                                      const double *__restrict__ BI, const float *__restrict__ iw,
+                                                      const unsigned *__restrict__ NODE, int sweeps, int kind0, MapSet ms) {
     extern __shared__ __align__(16) unsigned char smem[];
-    double *ds = (double *)smem;   // [3 nno]
-    __shared__ double Ps[3][3][64];
-    const int n3 = 3 * g.nno, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const bool forA = Ma && (int)blockIdx.x < n3;
-    const int jcol = (forA || !Ma) ? blockIdx.x : blockIdx.x - n3;
-    for (int idx = threadIdx.x; idx < n3; idx += blockDim.x) ds[idx] = (forA && idx == jcol) ? 1.0 : 0.0;
+    double *ds = (double *)smem;   // [nno][3][NC], a node's run MAP_PAD longer against bank conflicts
+    constexpr int ST = 3 * NC + MAP_PAD;
+    const int n3 = 3 * g.nno, kind = blockIdx.y + kind0, j0 = blockIdx.x * NC;
+    double *M = ms.m[kind];
+    for (int idx = threadIdx.x; idx < g.nno * NC; idx += 1024) {
+        const int n = idx / NC, col = idx % NC, jc = j0 + col;
+        double v[3] = {0.0, 0.0, 0.0};
+        if (kind == 0) {
+            if (jc / 3 == n) v[jc % 3] = 1.0;
+        } else if (kind == 2 && jc < n3) {
+            int k, i, j;
+            node_kij(g, n, k, i, j);
+            interp_node<double>(gc, g, iw, k, i, j, [&](int cn, int d) { return M[(size_t)(3 * cn + d) * n3 + jc]; }, v);
+            strip3(NODE[n], v);
+        }
+#pragma unroll
+        for (int e = 0; e < 3; e++) ds[n * ST + e * NC + col] = v[e];
+    }
     __syncthreads();
     for (int cyc = 0; cyc < sweeps; cyc++)
         for (int c = 0; c < 8; c++) {
-            const int tiles = (g.cn[c] + 63) >> 6;
-            for (int t = 0; t < tiles; t++) {
-                const int q = g.cs[c] + t * 64 + lane;
-                const bool act = q < g.cs[c] + g.cn[c];
-                int k = 0, i = 0, j = 0;
-                if (act) colour_kij(g, c, q, k, i, j);
+            for (int idx = threadIdx.x; idx < g.cn[c] * NC; idx += 1024) {
+                const int q = g.cs[c] + idx / NC, col = idx % NC;
+                int k, i, j;
+                colour_kij(g, c, q, k, i, j);
                 const int self = nid(g, k, i, j);
-                if (act) {
-                    double out[3];
-                    const float *kp = K + ktile(q);
-                    if (w == 0)
-                        plane_rows<0>(g, kp, k, i, j, self, (const double *)ds, out);
-                    else if (w == 1)
-                        plane_rows<1>(g, kp, k, i, j, self, (const double *)ds, out);
-                    else
-                        plane_rows<2>(g, kp, k, i, j, self, (const double *)ds, out);
-                    Ps[w][0][lane] = out[0];
-                    Ps[w][1][lane] = out[1];
-                    Ps[w][2][lane] = out[2];
+                const float *kp = K + ktile(q);
+                double o[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1
+                for (int P = 0; P < 3; P++) {
+                    double uv[27];
+#pragma unroll
+                    for (int b = 0; b < 9; b++) {
+                        const int dz = b % 3 - 1, dx = b / 3 - 1, dy = P - 1;
+                        const bool ok = (unsigned)(k + dz) < (unsigned)g.noz && (unsigned)(i + dx) < (unsigned)g.nox &&
+                                        (unsigned)(j + dy) < (unsigned)g.noy;   // else a zero block of the row
+                        const double *u = ds + (ok ? nid(g, k + dz, i + dx, j + dy) : self) * ST + col;
+#pragma unroll
+                        for (int e = 0; e < 3; e++) uv[3 * b + e] = u[e * NC];
+                    }
+#pragma unroll
+                    for (int r = 0; r < 3; r++) {
+                        float kv[27];
+#pragma unroll
+                        for (int b = 0; b < 9; b++)
+#pragma unroll
+                            for (int e = 0; e < 3; e++) kv[3 * b + e] = kp[(81 * P + 9 * b + 3 * r + e) * 64];
+                        o[r] += plane_sum_row<double>(kv, uv);
+                        __builtin_amdgcn_sched_barrier(0);   // one row's entries live at a time
+                    }
                 }
-                __syncthreads();
-                if (act) {
-                    const int r = w, e = 3 * self + r;
-                    const double Fr = (!forA && e == jcol) ? 1.0 : 0.0;
-                    const double o = (Ps[0][r][lane] + Ps[1][r][lane]) + Ps[2][r][lane];
-                    const float tt = (float)((Fr - o) * BI[e]);
-                    ds[e] = ds[e] + tt;
+                double *u = ds + self * ST + col;
+#pragma unroll
+                for (int r = 0; r < 3; r++) {
+                    const double F = kind != 0 && 3 * self + r == j0 + col ? 1.0 : 0.0;
+                    u[r * NC] += (float)((F - o[r]) * BI[3 * self + r]);
                 }
-                __syncthreads();
+            }
+            __syncthreads();
+        }
+    float *Mf = ms.f[kind];
+    for (int idx = threadIdx.x; idx < n3 * NC; idx += 1024) {
+        const int row = idx / NC, col = idx % NC;
+        if (j0 + col >= n3) continue;
+        const double v = ds[row / 3 * ST + row % 3 * NC + col];
+        M[(size_t)row * n3 + j0 + col] = v;
+        if (Mf) Mf[(size_t)row * n3 + j0 + col] = (float)v;   // the FP32 cycles read half the bytes
+    }
+}
+
+// as many columns a workgroup as its LDS takes
+static int map_columns(hipStream_t s, const Level &L, const Geo &gc, int sweeps, int kind0, int kinds, const MapSet &ms) {
+    const int n3 = 3 * L.g.nno;
+    auto launch = [&](auto kern, int nc) {
+        const size_t lds = (size_t)L.g.nno * (3 * nc + MAP_PAD) * 8;
+        if (lds > lds_limit()) return false;
+        if (lds > 65536 && hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return false;
+        hipLaunchKernelGGL(kern, dim3((n3 + nc - 1) / nc, kinds), dim3(1024), lds, s, L.g, gc, L.K, L.BI, L.iw, L.NODE,
+                           sweeps, kind0, ms);
+        return true;
+    };
+    if (launch(k_map_columns<8>, 8) || launch(k_map_columns<4>, 4) || launch(k_map_columns<1>, 1)) return 0;
+    set_error("the smoother's maps do not fit the workgroup memory");
+    return -1;
+}
+
+int coarse_build(hipStream_t s, const Level &L, int sweeps) {
+    const int nno = L.g.nno;
+    if (gs_small_kind(L)) {
+        hipLaunchKernelGGL(k_gs_lds, dim3(3 * nno), dim3(SMALL_TPB), kstage_bytes(nno) + vstage_bytes(nno), s, L.g,
+                           L.K, L.BI, L.NODE, L.Mc, nullptr, nullptr, sweeps, 0, 1);
+        return 0;
+    }
+    return map_columns(s, L, L.g, sweeps, 1, 1, MapSet{{nullptr, L.Mc, nullptr}, {}});
+}
+
+int affine_build(hipStream_t s, const Level &L, const Level &coarse) {
+    const MapSet ms{{L.Ma, L.Mb, L.Mu}, {L.Maf, L.Mbf, L.Muf}};
+    if (L.Mu)
+        hipLaunchKernelGGL(k_map_restrict, dim3(nblk(3L * L.g.nno), std::min(3 * coarse.g.nno, 64)), dim3(256), 0, s, L.g,
+                           coarse.g, coarse.TWW, coarse.MASS, coarse.NODE, coarse.Mc, L.Mu);
+    return map_columns(s, L, coarse.g, L.affine_sweeps, 0, L.Mu ? 3 : 2, ms);
+}
+
+// out = A din + B F (A may be null): LANES lanes a row; lane t sums A's terms
+// j = t, t + LANES, ... in order, then B's likewise, into S[t]; the S[t] meet in
+// a pairwise tree (S[q] += S[q+w], w = 1, 2, ...) formed by a butterfly.  Bound
+// by the latency of its loads: up to NB terms of a lane are requested together
+// (past the row's end the last one again, counted as 0), a whole row where it
+// fits (729 nodes, rows of 2187: 15.8 us -> 11.0 a call; eight terms at a time
+// and the rest one by one before).
+template <typename V, typename M, int LANES, int NB>
+__global__ void __launch_bounds__(64) k_map_apply(const M *A, const M *B, const V *__restrict__ din,
+                                                  const V *__restrict__ F, V *__restrict__ out, int n3) {
+    const int t = threadIdx.x % LANES, i = blockIdx.x * (64 / LANES) + threadIdx.x / LANES;
+    double S = 0.0;
+    if (i < n3) {
+#pragma unroll 1
+        for (int h = A ? 0 : 1; h < 2; h++) {
+            const M *row = (h ? B : A) + (size_t)i * n3;
+            const V *x = h ? F : din;
+#pragma unroll 1
+            for (int b = t; b < n3; b += NB * LANES) {
+                M m[NB];
+                V v[NB];
+#pragma unroll
+                for (int q = 0; q < NB; q++) {
+                    const int j = min(b + q * LANES, n3 - 1);
+                    m[q] = row[j];
+                    v[q] = x[j];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int q = 0; q < NB; q++) S = S + (b + q * LANES < n3 ? (double)m[q] * (double)v[q] : 0.0);
             }
         }
-    double *M = forA ? Ma : Mb;
-    for (int idx = threadIdx.x; idx < n3; idx += blockDim.x) M[(size_t)idx * n3 + jcol] = ds[idx];
-}
-
-void affine_build(hipStream_t s, const Level &L, int sweeps) {
-    const int n3 = 3 * L.g.nno;
-    hipLaunchKernelGGL(k_gs_unit, dim3(2 * n3), dim3(192), (size_t)n3 * 8, s, L.g, L.K, L.BI, L.Ma, L.Mb, sweeps);
-    if (L.Maf) {   // the FP32 cycles read the maps rounded to FP32: half the bytes
-        to_f32(s, L.Maf, L.Ma, (long)n3 * n3);
-        to_f32(s, L.Mbf, L.Mb, (long)n3 * n3);
-    }
-}
-
-// out = Ma din + Mb F (din may be null: zero guess).  One wavefront per row
-// i: lane t sums the Ma terms j = t, t+64, ... in order, then the Mb terms
-// likewise, into S[t]; the S[t] meet in a pairwise tree (S[q] += S[q+w],
-// w = 1 .. 32) formed by a butterfly over the wavefront.
-template <typename V, typename M>
-__global__ void __launch_bounds__(256) k_affine_apply(const M *__restrict__ Ma, const M *__restrict__ Mb,
-                                                      const V *__restrict__ din, const V *__restrict__ F,
-                                                      V *__restrict__ out, int n3) {
-    const int t = threadIdx.x & 63, i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    double S = 0.0;
-    if (i < n3) {   // unrolled so that the loads of several terms are in flight; the sum keeps its order
-        if (din)
-#pragma unroll 8
-            for (int j = t; j < n3; j += 64) S = S + (double)Ma[(size_t)i * n3 + j] * (double)din[j];
-#pragma unroll 8
-        for (int j = t; j < n3; j += 64) S = S + (double)Mb[(size_t)i * n3 + j] * (double)F[j];
     }
 #pragma unroll
-    for (int w = 1; w < 64; w *= 2) S = S + __shfl_xor(S, w, 64);
+    for (int w = 1; w < LANES; w *= 2) S = S + __shfl_xor(S, w, 64);
     if (i < n3 && t == 0) out[i] = (V)S;
+}
+
+template <typename V, typename M>
+static void map_apply(hipStream_t s, const M *A, const M *B, const V *din, const V *F, V *out, int n3) {
+    const int terms = (n3 + 63) / 64;
+    auto kern = terms <= 8 ? k_map_apply<V, M, 64, 8> : terms <= 20 ? k_map_apply<V, M, 64, 20> : k_map_apply<V, M, 64, 36>;
+    hipLaunchKernelGGL(kern, dim3(n3), dim3(64), 0, s, A, B, din, F, out, n3);
 }
 
 template <typename V>
 void affine_apply(hipStream_t s, const Level &L, const V *din, const V *F, V *out) {
     const int n3 = 3 * L.g.nno;
     if (sizeof(V) == 4 && L.Maf)
-        hipLaunchKernelGGL((k_affine_apply<V, float>), dim3((n3 + 3) / 4), dim3(256), 0, s, (const float *)L.Maf,
-                           (const float *)L.Mbf, din, F, out, n3);
+        map_apply<V, float>(s, din ? L.Maf : nullptr, L.Mbf, din, F, out, n3);
     else
-        hipLaunchKernelGGL((k_affine_apply<V, double>), dim3((n3 + 3) / 4), dim3(256), 0, s, (const double *)L.Ma,
-                           (const double *)L.Mb, din, F, out, n3);
+        map_apply<V, double>(s, din ? L.Ma : nullptr, L.Mb, din, F, out, n3);
 }
 template void affine_apply<double>(hipStream_t, const Level &, const double *, const double *, double *);
 template void affine_apply<float>(hipStream_t, const Level &, const float *, const float *, float *);
 
-// d = Mc F: sixteen lanes per row i, lane t summing j = t, t+16, ... in
-// order into S[t]; the S[t] meet in a pairwise tree (S[q] += S[q+w],
-// w = 1, 2, 4, 8) formed by a butterfly over the 16 lanes
+// the way up to the level above the coarsest: out = Mu res
 template <typename V>
-__global__ void __launch_bounds__(256) k_coarse_apply(const double *__restrict__ M, const V *__restrict__ F,
-                                                      V *__restrict__ d, int n3) {
-    const int t = threadIdx.x & 15, i = blockIdx.x * 16 + (threadIdx.x >> 4);
-    double S = 0.0;
-    if (i < n3)
-#pragma unroll 8
-        for (int j = t; j < n3; j += 16) S = S + M[(size_t)i * n3 + j] * (double)F[j];
-    S = S + __shfl_xor(S, 1, 64);
-    S = S + __shfl_xor(S, 2, 64);
-    S = S + __shfl_xor(S, 4, 64);
-    S = S + __shfl_xor(S, 8, 64);
-    if (i < n3 && t == 0) d[i] = (V)S;
+void up_apply(hipStream_t s, const Level &L, const V *res, V *out) {
+    const int n3 = 3 * L.g.nno;
+    if (sizeof(V) == 4 && L.Muf)
+        map_apply<V, float>(s, nullptr, L.Muf, nullptr, res, out, n3);
+    else
+        map_apply<V, double>(s, nullptr, L.Mu, nullptr, res, out, n3);
 }
+template void up_apply<double>(hipStream_t, const Level &, const double *, double *);
+template void up_apply<float>(hipStream_t, const Level &, const float *, float *);
 
+// d = Mc F, sixteen lanes a row
 template <typename V>
 void coarse_apply(hipStream_t s, const Level &L, const V *F, V *d) {
     const int n3 = 3 * L.g.nno;
-    hipLaunchKernelGGL(k_coarse_apply<V>, dim3((n3 + 15) / 16), dim3(256), 0, s, L.Mc, F, d, n3);
+    hipLaunchKernelGGL((k_map_apply<V, double, 16, 24>), dim3((n3 + 3) / 4), dim3(64), 0, s, nullptr, L.Mc, nullptr, F, d, n3);
 }
 template void coarse_apply<double>(hipStream_t, const Level &, const double *, double *);
 template void coarse_apply<float>(hipStream_t, const Level &, const float *, float *);
@@ -1844,8 +2003,6 @@ void project(hipStream_t s, const Level &fine, const Level &coarse, const V *AU,
 template void project<double>(hipStream_t, const Level &, const Level &, const double *, double *, bool, double *);
 template void project<float>(hipStream_t, const Level &, const Level &, const float *, float *, bool, float *);
 
-// interp_vector + un_inject_vector (Solver_multigrid.c:173-298, 581-634):
-// injection, then linear fills along x, z, y in the reference's order,
 // optionally followed by multi_grid's strip_bcs_from_residual
 template <typename V>
 __global__ void __launch_bounds__(TPB) k_interp(Geo gc, Geo gf, const float *__restrict__ iw,
@@ -1855,39 +2012,8 @@ __global__ void __launch_bounds__(TPB) k_interp(Geo gc, Geo gf, const float *__r
     if (n >= gf.nno) return;
     int k, i, j;
     node_kij(gf, n, k, i, j);
-    const float *wx = iw, *wz = iw + 2 * gf.nox, *wy = iw + 2 * (gf.nox + gf.noz);
-    // the (up to) 8 coarse nodes around the fine node are loaded together,
-    // then the linear fills along x, then z, then y: an odd fine index
-    // interpolates its two coarse neighbours n1 a + n2 b, an even one takes
-    // its single coarse value
-    const int kc[2] = {k >> 1, (k + 1) >> 1}, ic[2] = {i >> 1, (i + 1) >> 1}, jc[2] = {j >> 1, (j + 1) >> 1};
-    V c[2][2][2][3];   // [y][z][x][component]
-#pragma unroll
-    for (int yy = 0; yy < 2; yy++)
-#pragma unroll
-        for (int zz = 0; zz < 2; zz++)
-#pragma unroll
-            for (int xx = 0; xx < 2; xx++) {
-                const int cn = nid(gc, kc[zz], ic[xx], jc[yy]);
-#pragma unroll
-                for (int d = 0; d < 3; d++) c[yy][zz][xx][d] = AD[3 * cn + d];
-            }
-    const float nx1 = wx[2 * i], nx2 = wx[2 * i + 1], nz1 = wz[2 * k], nz2 = wz[2 * k + 1];
-    const float ny1 = wy[2 * j], ny2 = wy[2 * j + 1];
     V v[3];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        V lx[2][2];
-#pragma unroll
-        for (int yy = 0; yy < 2; yy++)
-#pragma unroll
-            for (int zz = 0; zz < 2; zz++)
-                lx[yy][zz] = (i & 1) ? nx1 * c[yy][zz][0][d] + nx2 * c[yy][zz][1][d] : c[yy][zz][0][d];
-        V pz[2];
-#pragma unroll
-        for (int yy = 0; yy < 2; yy++) pz[yy] = (k & 1) ? nz1 * lx[yy][0] + nz2 * lx[yy][1] : lx[yy][0];
-        v[d] = (j & 1) ? ny1 * pz[0] + ny2 * pz[1] : pz[0];
-    }
+    interp_node<V>(gc, gf, iw, k, i, j, [&](int cn, int d) { return AD[3 * cn + d]; }, v);
     if (do_strip) strip3(NODE[n], v);
     AU[3 * n] = v[0];
     AU[3 * n + 1] = v[1];

@@ -446,18 +446,23 @@ int build_mesh(chip_ctx *c) {
     {
         Level &C = c->L[c->levmin];
         if (affine_ok(C) && dev_alloc(c, &C.Mc, 9 * (size_t)C.g.nno * C.g.nno)) return -1;
-        // the level above: affine form when its two smoother calls in
-        // multi_grid use the same number of sweeps
-        if (C.Mc && c->levmin + 1 < c->levmax && p.down_heavy == p.up_heavy) {
-            Level &A = c->L[c->levmin + 1];
-            if (affine_ok(A)) {
-                const size_t n3 = 3 * (size_t)A.g.nno;
-                if (dev_alloc(c, &A.Ma, n3 * n3) || dev_alloc(c, &A.Mb, n3 * n3) || dev_alloc(c, &A.tmp, n3) ||
-                    (p.mixed && (dev_alloc(c, &A.Maf, n3 * n3) || dev_alloc(c, &A.Mbf, n3 * n3))) ||
-                    dev_alloc(c, &A.tmpf, n3))
-                    return -1;
-                A.affine_sweeps = p.down_heavy;
-            }
+        // the levels above: affine form when their two smoother calls in
+        // multi_grid use the same number of sweeps.  Cycles that stop at a
+        // level solved exactly reach them only where that is switched off:
+        // there, the level above the coarsest only, and not its way up
+        const bool exact = p.mixed && c->levmin + 2 < c->levmax && 3L * c->L[c->levmin + 2].g.nno <= DIRECT_MAX_DOF;
+        for (int lev = c->levmin + 1; C.Mc && lev < c->levmax && p.down_heavy == p.up_heavy; lev++) {
+            Level &A = c->L[lev];
+            if (exact ? lev > c->levmin + 1 || !affine_ok(A) : !map_ok(A)) break;
+            const size_t n3 = 3 * (size_t)A.g.nno;
+            if (dev_alloc(c, &A.Ma, n3 * n3) || dev_alloc(c, &A.Mb, n3 * n3) || dev_alloc(c, &A.tmp, n3) ||
+                (p.mixed && (dev_alloc(c, &A.Maf, n3 * n3) || dev_alloc(c, &A.Mbf, n3 * n3))) ||
+                dev_alloc(c, &A.tmpf, n3))
+                return -1;
+            if (!exact && lev == c->levmin + 1 &&
+                (dev_alloc(c, &A.Mu, n3 * n3) || (p.mixed && dev_alloc(c, &A.Muf, n3 * n3))))
+                return -1;
+            A.affine_sweeps = p.down_heavy;
         }
     }
     // the FP32 cycles' exact coarsest-level solve: the largest level of at

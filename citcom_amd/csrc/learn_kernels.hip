@@ -30,7 +30,43 @@ __global__ void k_relu_bwd(const uint16_t *__restrict__ Y, uint16_t *__restrict_
     if (i < n && !(bf2f(Y[i]) > 0.f)) dY[i] = 0;
 }
 
-// ---- backward data, less aligned operands: dX[v][c] = sum_t sum_o dY[v-off_t][o] W[o][t][c]
+// Up to this many voxels a wavefront that takes 16 of them and all their loads
+// at once beats the staged blocks (unet_kernels.hip): four layers and their
+// launches at 16 x 11^3 voxels 37.6 us against 42.3, 17^3 31.9 and 36.1, but
+// 4 x 24x30x20 54.5 and 47.2, 40^3 58.7 and 47.5.
+constexpr long SMALL_VOXELS = 32768;
+
+// ---- forward, small volumes: Y[v][o] = act(sum_t sum_c X[v+off_t][c] W[o][t][c] + bias[o])
+__global__ void __launch_bounds__(256) k_conv_fwd(Vol g, const uint16_t *__restrict__ X, const uint16_t *__restrict__ W,
+                                                  const float *__restrict__ bias, int relu, uint16_t *__restrict__ Y,
+                                                  float *__restrict__ Yf) {
+    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, b = blockIdx.y;
+    const int v0 = (blockIdx.x * 4 + wv) * 16;
+    if (v0 >= g.nv) return;
+    const uint16_t *Xb = X + (size_t)b * g.nv * CH;
+    const int m = v0 + (l & 15), kq = 4 * (l >> 4);
+    const Cell cm = cell(g, m);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < TAPS; t++) {
+        const int vn = nbr(g, cm, t);
+        bf16x4 a = {0, 0, 0, 0};
+        if (vn >= 0) a = load4(Xb + (size_t)vn * CH + kq);
+        const bf16x4 w = load4(W + ((size_t)(l & 15) * TAPS + t) * CH + kq);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, w, acc, 0, 0, 0);
+    }
+    const int o = l & 15;
+    for (int i = 0; i < 4; i++) {
+        const int v = v0 + kq + i;
+        if (v >= g.nv) continue;
+        float y = acc[i] + bias[o];
+        if (relu) y = y > 0.f ? y : 0.f;
+        Y[((size_t)b * g.nv + v) * CH + o] = f2bf(y);
+        if (Yf) Yf[((size_t)b * g.nv + v) * CH + o] = y;
+    }
+}
+
+// ---- backward data, small volumes or less aligned operands: dX[v][c] = sum_t sum_o dY[v-off_t][o] W[o][t][c]
 __global__ void __launch_bounds__(256) k_conv_bwd_data(Vol g, const uint16_t *__restrict__ dY,
                                                        const uint16_t *__restrict__ W, uint16_t *__restrict__ dX) {
     __shared__ __align__(16) uint16_t Wt[TAPS][CH][CH];   // [t][c][o]
@@ -148,6 +184,11 @@ extern "C" {
 
 int cl_conv3d_fwd(const uint16_t *x, int nb, int nx, int ny, int nz, const uint16_t *w, const float *bias, int relu,
                   uint16_t *y, float *yf, void *stream) {
+    const Vol g{nx, ny, nz, nx * ny * nz};
+    if (bias && nb > 0 && g.nv > 0 && (long)nb * g.nv <= SMALL_VOXELS) {
+        hipLaunchKernelGGL(k_conv_fwd, dim3((g.nv + 63) / 64, nb), dim3(256), 0, st(stream), g, x, w, bias, relu, y, yf);
+        return ret();
+    }
     return cl_conv3d_fwd_c(x, nb, nx, ny, nz, CH, CH, w, bias, nullptr, relu, 0, y, yf, stream);
 }
 
@@ -161,7 +202,7 @@ int cl_conv3d_bwd_data(const uint16_t *dy, int nb, int nx, int ny, int nz, const
     const Vol g{nx, ny, nz, nx * ny * nz};
     // the forward convolution of dy with the weights read transposed and the
     // taps mirrored
-    if (nb > 0 && g.nv > 0 && conv_block_ok(CH, dy, w, nullptr, dx, nullptr) &&
+    if (nb > 0 && g.nv > 0 && (long)nb * g.nv > SMALL_VOXELS && conv_block_ok(CH, dy, w, nullptr, dx, nullptr) &&
         conv_fwd(g, nb, CH, CH, dy, w, 1, nullptr, nullptr, 0, 1, dx, nullptr, st(stream)) == 0)
         return ret();
     hipLaunchKernelGGL(k_conv_bwd_data, dim3((g.nv + 63) / 64, nb), dim3(256), 0, st(stream), g, dy, w, dx);
@@ -175,6 +216,9 @@ long cl_conv3d_bwd_weight_workspace(int nb, int nx, int ny, int nz) {
 
 int cl_conv3d_bwd_weight(const uint16_t *x, const uint16_t *dy, int nb, int nx, int ny, int nz, float *grad,
                          float *workspace, void *stream) {
+    const Vol g{nx, ny, nz, nx * ny * nz};
+    const long slots = cl_conv3d_bwd_weight_workspace(nb, nx, ny, nz) / ((TAPS * CH * CH + CH) * (long)sizeof(float));
+    if (nb > 0 && g.nv > 0 && conv_wgrad(g, nb, CH, CH, x, dy, workspace, slots, grad, st(stream)) == 0) return ret();
     // (a slot for 256 voxels holds at least as many as the general call's for 512)
     return cl_conv3d_bwd_weight_c(x, dy, nb, nx, ny, nz, CH, CH, grad, workspace, stream);
 }

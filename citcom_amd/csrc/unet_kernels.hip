@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdint>
 
 #include "../../include/citcom_learn.h"
@@ -220,31 +221,31 @@ __global__ void __launch_bounds__(CONV_TPB) k_conv_block(Vol g, ConvBlock cb, in
 // The block of a grid: of the shapes whose tiles (at most `most`) and region
 // (at most `lds` bytes) fit, the one with the least positions computed and
 // voxels staged per output (a staged voxel costs about as much as a quarter
-// of a computed one at 16 channels), a grid of too few blocks for the chip
-// counting as work too.
-ConvBlock conv_block(const Vol &g, int nb, int groups, int ncb, int most, long lds) {
+// of a computed one at 16 channels, a block `start` tiles before its first),
+// a grid of too few blocks for `wide` workgroups a group counting as work too.
+ConvBlock conv_block(const Vol &g, int nb, int ncb, int most, long lds, long wide, double start) {
     ConvBlock best{};
     double cost = 0.0;
+    const double turn = 1.0 / (CONV_WAVES * CONV_M), share = 1.0 / (double)wide;
     for (int cuts = 1; cuts <= g.nz && (cuts <= 8 || !best.TZ); cuts++) {
         const int TZ = (g.nz + cuts - 1) / cuts;
         if (cuts > 1 && TZ == (g.nz + cuts - 2) / (cuts - 1)) continue;
-        for (int TX = 1; TX <= 8 && TX <= g.nx; TX++)
+        const int nbz = (g.nz + TZ - 1) / TZ;
+        for (int TX = 1, last = 0; TX <= 8 && TX <= g.nx; TX++) {
+            const int nbx = (g.nx + TX - 1) / TX, tpp = ((TZ + 2) * TX + 15) / 16;
+            if (nbx == last) continue;   // as many blocks, larger
+            last = nbx;
             for (int TY = 1; TY <= 4 && TY <= g.ny; TY++) {
-                ConvBlock c{TZ, TX, TY, TZ + 2, TX + 2, TY + 2};
-                c.tpp = (c.LZ * TX + 15) / 16;
-                c.tiles = TY * c.tpp;
-                c.region = c.LZ * c.LX * c.LY + CONV_PAD;
-                if (c.tiles > most || (long)c.region * ncb * 32 > lds) continue;
-                c.nbz = (g.nz + TZ - 1) / TZ;
-                c.nbx = (g.nx + TX - 1) / TX;
-                c.nby = (g.ny + TY - 1) / TY;
-                const double blocks = (double)nb * c.nbz * c.nbx * c.nby;
-                // rounds of 512 workgroups; each as long as its tiles (in whole turns of the wavefronts) and staging
-                const int turns = (c.tiles + CONV_WAVES * CONV_M - 1) / (CONV_WAVES * CONV_M);
-                const double rounds = std::max(1.0, blocks * groups / 512.0);
-                const double v = rounds * (16.0 * turns + 0.25 * c.region / 16.0 + 4.0);
-                if (!best.TZ || v < cost) best = c, cost = v;
+                const int tiles = TY * tpp, region = (TZ + 2) * (TX + 2) * (TY + 2) + CONV_PAD;
+                if (tiles > most || (long)region * ncb * 32 > lds) break;
+                const int nby = (g.ny + TY - 1) / TY;
+                const double blocks = (double)nb * nbz * nbx * nby;
+                // rounds of `wide` workgroups; each as long as its tiles (in whole turns of the wavefronts) and staging
+                const double rounds = std::max(1.0, blocks * share);
+                const double v = rounds * (16.0 * std::ceil(tiles * turn) + 0.25 / 16.0 * region + start);
+                if (!best.TZ || v < cost) best = {TZ, TX, TY, TZ + 2, TX + 2, TY + 2, nbz, nbx, nby, tpp, tiles, region}, cost = v;
             }
+        }
     }
     return best;
 }
@@ -270,7 +271,8 @@ int conv_launch(const Vol &g, int nb, int co, const uint16_t *x, const uint16_t 
     if (raise_lds((const void *)kern, raised)) return -1;
     const long wlds = WREG ? 0 : 9L * NCB * NBO * 512;
     const int groups = co / (16 * NBO);
-    const ConvBlock cb = conv_block(g, nb, groups, NCB, WREG ? 1 << 20 : CONV_WAVES * CONV_M, (NCB * NBO == 1 ? CONV_LDS / 2 : CONV_LDS) - wlds);
+    const ConvBlock cb = conv_block(g, nb, NCB, WREG ? 1 << 20 : CONV_WAVES * CONV_M,
+                                    (NCB * NBO == 1 ? CONV_LDS / 2 : CONV_LDS) - wlds, std::max(1, 512 / groups), 4.0);
     if (!cb.TZ) return -1;
     const long blocks = (long)nb * cb.nbz * cb.nbx * cb.nby;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks, groups), dim3(CONV_TPB), (size_t)NCB * cb.region * 32 + wlds, s, g, cb,
@@ -395,6 +397,7 @@ __device__ __forceinline__ bf16x4 lds_read_tr(const unsigned char *p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p);
 }
 
+constexpr double WG_START = 20.0;   // a block's staging and table, in 16-voxel tiles' time
 constexpr int WG_TAPS = 7;   // taps of a wavefront: 0-6, 7-13, 14-20, 21-26 and the bias
 
 template <int NCB, int NOB>
@@ -515,12 +518,14 @@ int wgrad_launch(const Vol &g, int nb, int ci, int co, const uint16_t *x, const 
     if (raise_lds((const void *)kern, raised)) return -1;
     const int groups = (ci / (16 * NCB)) * (co / (16 * NOB));
     // dY and the table take less than NOB + 1/8 blocks' regions
-    const ConvBlock cb = conv_block(g, nb, groups, NCB + NOB, 1 << 20, CONV_LDS * 8 / 9);
+    // two workgroups to a CU; no more slots than the workspace has, whose
+    // workgroups take larger blocks where they are few
+    const long wide = std::min(slots, std::max(1L, 512L / groups));
+    const ConvBlock cb = conv_block(g, nb, NCB + NOB, 1 << 20, CONV_LDS * 8 / 9, wide, WG_START);
     if (!cb.TZ) return -1;
     const long blocks = (long)nb * cb.nbz * cb.nbx * cb.nby;
     if (blocks >= 1L << 31) return -1;
-    // two workgroups to a CU; no more slots than the workspace has
-    const long nslots = std::min(std::min(blocks, slots), std::max(1L, 512L / groups));
+    const long nslots = std::min(blocks, wide);
     const long most = ((long)cb.TZ * cb.TX * cb.TY + 15) & ~15L;
     hipLaunchKernelGGL(kern, dim3((unsigned)nslots, groups), dim3(CONV_TPB),
                        (size_t)NCB * cb.region * 32 + NOB * most * 32 + most * 4, s, g, cb, (int)blocks, ci, co, x, dy, part);

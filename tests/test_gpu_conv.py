@@ -111,3 +111,27 @@ def test_block_weight_gradient(dims):
             fine = torch.isfinite(b)
             assert torch.equal(torch.isfinite(a), fine) and torch.equal(torch.isnan(a), torch.isnan(b)), (dims, ci, co)
             assert float((a - b)[fine].norm()) <= 1e-5 * float(b[fine].norm()) + 1e-30, (dims, ci, co, nb)
+
+
+@pytest.mark.parametrize("nb,dims", [(1, (1, 1, 1)), (3, (5, 7, 9)), (1, (32, 32, 32)), (1, (31, 33, 33)), (2, (33, 30, 37))])
+def test_sixteen_channels_small_and_block_kernels_same_bits(nb, dims):
+    """the kernel of small volumes (up to 32768 voxels) and the blocks', on
+    either side of the line: forward against the general entry point, data
+    gradient against less aligned operands"""
+    import torch
+    from citcom_amd import unet
+    from citcom_amd.learn import _p
+    L = unet._lib()
+    g = torch.Generator(device="cuda").manual_seed(8)
+    nv = dims[0] * dims[1] * dims[2]
+    x = torch.randn((nb, nv, 16), generator=g, device="cuda").bfloat16()
+    w = (0.1 * torch.randn((16, 27, 16), generator=g, device="cuda")).bfloat16()
+    b = torch.randn(16, generator=g, device="cuda")
+    nan = lambda dt: torch.full((nb, nv, 16), float("nan"), dtype=dt, device="cuda")
+    y, yf, yg, yfg, d, ds = nan(x.dtype), nan(b.dtype), nan(x.dtype), nan(b.dtype), nan(x.dtype), nan(x.dtype)
+    assert L.cl_conv3d_fwd(_p(x), nb, *dims, _p(w), _p(b), 1, _p(y), _p(yf), None) == 0
+    assert L.cl_conv3d_fwd_c(_p(x), nb, *dims, 16, 16, _p(w), _p(b), None, 1, 0, _p(yg), _p(yfg), None) == 0
+    assert torch.equal(y, yg) and torch.equal(yf, yfg)
+    assert L.cl_conv3d_bwd_data(_p(x), nb, *dims, _p(w), _p(d), None) == 0
+    assert L.cl_conv3d_bwd_data(_p(shifted(x, 4)), nb, *dims, _p(w), _p(ds), None) == 0
+    assert torch.equal(d, ds)

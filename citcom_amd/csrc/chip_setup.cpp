@@ -450,10 +450,18 @@ int build_mesh(chip_ctx *c) {
         // multi_grid use the same number of sweeps.  Cycles that stop at a
         // level solved exactly reach them only where that is switched off:
         // there, the level above the coarsest only, and not its way up
+        // there, the level above the coarsest only, and not its way up.  The
+        // sweeps' FP32 increments, which the maps do not round, move the
+        // solution by 2e-11 at constant viscosity (28 solves), but by up to
+        // 1.5e-9 in the pressure at the 64^3 workload's contrast of 10^4 (one
+        // solve in thirty; the median 1e-11): FP64 cycles with varying
+        // viscosity keep the sweeps above AFFINE_MAX_DOF
+        bool constant = !p.tdepv;
+        for (int m = 1; m < p.num_mat; m++) constant = constant && p.visc0[m] == p.visc0[0];
         const bool exact = p.mixed && c->levmin + 2 < c->levmax && 3L * c->L[c->levmin + 2].g.nno <= DIRECT_MAX_DOF;
         for (int lev = c->levmin + 1; C.Mc && lev < c->levmax && p.down_heavy == p.up_heavy; lev++) {
             Level &A = c->L[lev];
-            if (exact ? lev > c->levmin + 1 || !affine_ok(A) : !map_ok(A)) break;
+            if (exact || !(constant || p.mixed) ? lev > c->levmin + 1 || !affine_ok(A) : !map_ok(A)) break;
             const size_t n3 = 3 * (size_t)A.g.nno;
             if (dev_alloc(c, &A.Ma, n3 * n3) || dev_alloc(c, &A.Mb, n3 * n3) || dev_alloc(c, &A.tmp, n3) ||
                 (p.mixed && (dev_alloc(c, &A.Maf, n3 * n3) || dev_alloc(c, &A.Mbf, n3 * n3))) ||

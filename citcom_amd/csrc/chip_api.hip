@@ -683,6 +683,8 @@ int rebuild(chip_ctx *c) {
         for (int lev = c->levmin; lev <= c->levmax; lev++) to_f32(q, c->L[lev].BIf, c->L[lev].BI, 3L * c->L[lev].g.nno);
     for (int lev = c->levmin; lev <= c->levmax; lev++)
         if (c->L[lev].Kh) scale_half(q, c->L[lev]);
+    for (int lev = c->levmin; lev <= c->levmax; lev++)
+        if (c->L[lev].planes.shape) rect_pack(q, c->L[lev]);
     for (int lev = c->levmin; lev <= c->levmax; lev++) box_tiles(q, c->L[lev]);
     CHIP_CHECK(hipGetLastError());
     return direct_factor(c);

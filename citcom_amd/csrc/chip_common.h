@@ -118,7 +118,9 @@ struct Level {
     // FP32 copies for the mixed-precision cycle
     float *velf = nullptr, *resf = nullptr, *flf = nullptr, *delf = nullptr, *AUf = nullptr;
     float *BIf = nullptr;
-    RectPart planes{};       // joined colour passes (k_gs_rect)
+    RectPart planes{};       // joined colour passes (k_gs_rect), and K and Kh packed for them
+    float *Kr = nullptr;
+    uint16_t *Krh = nullptr;
     // one-XCD smoother state (levels gs_xcd_ok accepts)
     XcdBar *xbar = nullptr;
     // box smoother of the FP32 cycles: the partition, and the cycle's

@@ -36,6 +36,8 @@ void gs_colour(hipStream_t s, const Level &L, const V *BI, int colour, V *d, con
 // the four colours of the planes of parity jpar, from dself (their nodes) and
 // dside (the planes between; null: zero) to dout
 RectPart rect_planes(const Geo &g);
+size_t rect_pack_elems(const Level &L, bool half);
+void rect_pack(hipStream_t s, const Level &L);
 template <typename V>
 void gs_rect(hipStream_t s, const Level &L, const V *BI, const V *F, int jpar, const V *dself, const V *dside, V *dout,
              hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);

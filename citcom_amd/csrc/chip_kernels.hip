@@ -647,23 +647,26 @@ template void gs_colour<float>(hipStream_t, const Level &, const float *, int, f
 // sweep's input (din); it writes its own nodes only, to dout.
 //
 // A lane forms one row of one node.  Its 81 coefficients are requested at the
-// start; the sums of the planes dy = -1 and +1, whose entries no colour of the
-// launch changes, are formed by all wavefronts at once; only the plane dy = 0
-// is left for the chain of colours, one workgroup barrier each.  A node's own
-// entries are kept in registers, so its three rows need no barrier between
-// reading and writing them.
+// start, packed for the launch (k_rect_pack; as nine-node pieces of the tiles'
+// lines they took 81 loads and a third of the time); the sums of the planes
+// dy = -1 and +1, whose entries no colour of the launch changes, are formed by
+// all wavefronts at once, as are the blocks of the plane dy = 0; in its turn a
+// colour only forms the blocks again whose entries have changed, one workgroup
+// barrier a colour.  A node's own entries are kept in registers, so its three
+// rows need no barrier between reading and writing them.
 //
-// Bound by the chain: launch, one load, four colours of LDS reads and sums.
-// FP64 vectors, a half sweep (four colours) against four launches of
-// k_gs_colour, without the gaps between launches: 4913 nodes (17x17x17) 8.1 us
-// against 18.4, 18513 (33x33x17) 9.8 against 18.5, 35937 (33x33x33) 11.0
-// against 18.9, 139425 (65x65x33) 31 against 30, 274625 (65x65x65) 73 against
-// 46: past one workgroup per CU the nodes computed twice and the LDS reads
-// cost more than the launches saved, and the level stays with k_gs_colour.
-// Shapes: narrow, a colour's 21 nodes in one wavefront, three lanes each
-// (four wavefronts, one a SIMD: 7.9 us where the wide shape takes 9.3); wide,
-// a colour's 64 nodes in three wavefronts, one a row (18513 nodes: 9.8 us
-// where narrow strips, two workgroups to some CUs, take 11.5).
+// Bound by latency (launch, one load, four colours of LDS reads and sums) and,
+// in the wide shape, by the coefficients' bytes, the nodes computed twice among
+// them.  FP64 vectors, a half sweep (four colours) against four launches of
+// k_gs_colour: 4913 nodes (17x17x17) 5.6 us against 18.4, 18513 (33x33x17) 7.6
+// against 18.5, 35937 (33x33x33) 9.6 against 18.9, 79233 (49x33x49) 19 against
+// 20, 139425 (65x65x33) 27 against 28, 194481 (81x49x49) 42 against 29: past one
+// workgroup per CU the nodes computed twice cost what the launches save, and
+// the level stays with k_gs_colour.
+// Shapes: narrow, a colour's 21 nodes in one wavefront, three lanes each (four
+// wavefronts, one a SIMD), while there are at most two workgroups to a CU
+// (18513 nodes: 7.6 us, wide 8.7; 35937 nodes, three to a CU: 14, wide 9.6);
+// wide, a colour's 64 nodes in three wavefronts, one a row.
 
 // row r of one plane's tree (absent neighbours have zero coefficients and
 // zero entries; adding the tree's empty slots changes no bit but a zero's sign)
@@ -674,6 +677,35 @@ __device__ __forceinline__ V plane_sum_row(const float kv[27], const V uv[27]) {
     for (int b = 0; b < 9; b++) t[b] = kv[3 * b] * uv[3 * b] + kv[3 * b + 1] * uv[3 * b + 1] + kv[3 * b + 2] * uv[3 * b + 2];
     return (((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) + t[8];
 }
+
+// Coefficients packed for the joined passes and the box smoother: a lane's 81
+// in 16-byte groups of G = 4 (FP32) or 8 (FP16), [cc / G][lane][cc % G], so
+// that a wavefront reads them in 21 or 11 coalesced loads per lane.  The
+// padding past cc = 80 (and the boxes' lanes without a node) hold zeros; in a
+// joined pass's run the lanes with a node come first and the others read the
+// last one's.
+template <typename KT>
+struct Pack {
+    static constexpr int G = 16 / (int)sizeof(KT);
+    static constexpr int NG = (81 + G - 1) / G;
+    static constexpr size_t WAVE = (size_t)NG * 64 * G;   // entries of a wavefront
+    uint4 q[NG];
+    __device__ __forceinline__ void load(const uint4 *__restrict__ p, int lanes = 64) {
+#pragma unroll
+        for (int t = 0; t < NG; t++) q[t] = p[t * lanes];
+    }
+    // the values as loaded up to here: widened earlier they would not fit the registers
+    __device__ __forceinline__ void hold() {
+#pragma unroll
+        for (int t = 0; t < NG; t++) asm volatile("" : "+v"(q[t].x), "+v"(q[t].y), "+v"(q[t].z), "+v"(q[t].w));
+    }
+    template <int FROM, int N>
+    __device__ __forceinline__ void widen(float kv[N]) const {
+        const KT *e = reinterpret_cast<const KT *>(q);
+#pragma unroll
+        for (int ci = 0; ci < N; ci++) kv[ci] = (float)e[FROM + ci];
+    }
+};
 
 // the shape of a workgroup: nodes of a colour, W lines, HZ entries of one k
 // parity in the staged region
@@ -686,29 +718,69 @@ struct RectShape {
     static constexpr int LINE = 3 * 2 * HZ;                 // [component][k parity][k/2]
 };
 
+// what a wavefront of a workgroup (seg, strip, plane j) and its lane take:
+// colour phase ph, row r of node (k, i) (act: if there is one), lines and
+// nodes stepping two, nodes past the segment that later colours read
+template <class S>
+struct RectLane {
+    int ph, r, k, i, lanes, slot;   // slot: the lane's place among the `lanes` with a node
+    bool act;
+    __device__ __forceinline__ RectLane(const Geo &g, const RectPart &rp, int seg, int strip, int w, int lane) {
+        ph = S::WIDE ? w / 3 : w;
+        const int i0 = strip * S::W, k0 = seg * rp.Wz, k1 = k0 + rp.Wz;
+        const int kp = ph & 1, ip = ph >> 1, grow = 2 - ph;
+        const int klo = max(kp, k0 - grow), khi = min(g.noz - 1, k1 + grow);
+        const int ilo = i0 + ip, ihi = min(g.nox - 1, i0 + S::W - ip);
+        const int nk = khi >= klo ? ((khi - klo) >> 1) + 1 : 0, ni = ihi >= ilo ? ((ihi - ilo) >> 1) + 1 : 0;
+        r = S::WIDE ? w - 3 * ph : lane / 21;
+        const int t = S::WIDE ? lane : lane - 21 * r;
+        act = r < 3 && t < nk * ni;
+        int ii = 0;   // t / nk, of at most W/2 + 1 lines
+#pragma unroll
+        for (int m = 1; m <= S::W / 2; m++) ii += t >= m * nk;
+        k = klo + 2 * (t - ii * nk);
+        i = ilo + 2 * ii;
+        lanes = (S::WIDE ? 1 : 3) * nk * ni;
+        slot = max(0, act ? (S::WIDE ? t : r * nk * ni + t) : lanes - 1);
+    }
+};
+
+// the packed coefficients of wavefront w of workgroup (seg, strip, j)
+template <class S>
+__device__ __forceinline__ size_t rect_wave(const RectPart &rp, int seg, int strip, int j, int w) {
+    return (((size_t)j * rp.nstrip + strip) * rp.ns + seg) * S::WAVES + w;
+}
+
+template <typename KT, class S>
+__global__ void __launch_bounds__(S::WAVES * 64) k_rect_pack(Geo g, RectPart rp, const KT *__restrict__ K,
+                                                             KT *__restrict__ Kr) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int seg = blockIdx.x, strip = blockIdx.y, j = blockIdx.z;
+    const RectLane<S> rl(g, rp, seg, strip, w, lane);
+    const KT *kq = K + (rl.act ? ktile(colour_index(g, rl.ph | (j & 1) << 2, rl.k, rl.i, j)) + 3 * 64 * rl.r : 0);
+    KT v[Pack<KT>::NG * Pack<KT>::G];
+#pragma unroll
+    for (int cc = 0; cc < Pack<KT>::NG * Pack<KT>::G; cc++)
+        v[cc] = rl.act && cc < 81 ? kq[(81 * (cc / 27) + 9 * (cc % 27 / 3) + cc % 3) * 64] : KT(0);
+    uint4 *dst = reinterpret_cast<uint4 *>(Kr) + rect_wave<S>(rp, seg, strip, j, w) * (Pack<KT>::NG * 64) + rl.slot;
+    if (!rl.act) return;
+#pragma unroll
+    for (int t = 0; t < Pack<KT>::NG; t++) dst[t * rl.lanes] = reinterpret_cast<const uint4 *>(v)[t];
+}
+
 template <typename V, typename KT, class S>
-__global__ void __launch_bounds__(S::WAVES * 64, sizeof(V) == 8 || sizeof(KT) == 2 ? 3 : 4) k_gs_rect(Geo g, RectPart rp, int jpar, const KT *__restrict__ K,
+__global__ void __launch_bounds__(S::WAVES * 64, sizeof(V) == 8 || sizeof(KT) == 2 ? 3 : 4) k_gs_rect(Geo g, RectPart rp, int jpar, const KT *__restrict__ Kr,
                                                            const V *__restrict__ BI, const V *__restrict__ F,
                                                            const V *__restrict__ dself, const V *__restrict__ dside,
                                                            V *__restrict__ dout) {
     constexpr int W = S::W, HZ = S::HZ, NL = S::NL, LINE = S::LINE;
     __shared__ __align__(16) V sd[3 * NL * LINE];   // [plane][line]
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ph = S::WIDE ? w / 3 : w;
     const int seg = blockIdx.x, strip = blockIdx.y, j = 2 * blockIdx.z + jpar;
     const int i0 = strip * W, k0 = seg * rp.Wz, k1 = k0 + rp.Wz;
-    // this wavefront's colour: its lines and nodes (step 2 each way)
-    const int kp = ph & 1, ip = ph >> 1, grow = 2 - ph;   // nodes past the segment that later colours read
-    const int klo = max(kp, k0 - grow), khi = min(g.noz - 1, k1 + grow);
-    const int ilo = i0 + ip, ihi = min(g.nox - 1, i0 + W - ip);
-    const int nk = khi >= klo ? ((khi - klo) >> 1) + 1 : 0, ni = ihi >= ilo ? ((ihi - ilo) >> 1) + 1 : 0;
-    const int r = S::WIDE ? w - 3 * ph : lane / 21, t = S::WIDE ? lane : lane - 21 * r;
-    const bool act = r < 3 && t < nk * ni;
-    int ii = 0;   // t / nk, of at most W/2 + 1 lines
-#pragma unroll
-    for (int m = 1; m <= W / 2; m++) ii += t >= m * nk;
-    const int k = klo + 2 * (t - ii * nk), i = ilo + 2 * ii;
-    const int c = kp | (ip << 1) | (jpar << 2);
+    const RectLane<S> rl(g, rp, seg, strip, w, lane);
+    const int ph = rl.ph, r = rl.r, k = rl.k, i = rl.i, kp = ph & 1;
+    const bool act = rl.act;
     const int fself = act ? 3 * nid(g, k, i, j) + r : 0;
     // staged region: lines i0-1 .. i0+W+1 of three planes, nodes kr0 .. (kr0
     // even), zero outside the mesh.  A wavefront takes whole lines, 21 nodes
@@ -726,18 +798,8 @@ __global__ void __launch_bounds__(S::WAVES * 64, sizeof(V) == 8 || sizeof(KT) ==
         stage[q] = (pl == 1 ? same : side)[3 * nid(g, gk, gi, gj) + comp];
     }
     const V Fr = F[fself], Br = BI[fself];
-    float kv[3][27];
-    {
-        const KT *kq = K + ktile(act ? colour_index(g, c, k, i, j) : g.cs[c]) + (r < 3 ? 3 * 64 * r : 0);
-#pragma unroll
-        for (int pp = 0; pp < 3; pp++) {   // in the order of their use
-            const int P = pp == 0 ? 0 : pp == 1 ? 2 : 1;
-#pragma unroll
-            for (int bb = 0; bb < 9; bb++)
-#pragma unroll
-                for (int cc = 0; cc < 3; cc++) kv[P][3 * bb + cc] = (float)kq[(81 * P + 9 * bb + cc) * 64];
-        }
-    }
+    Pack<KT> pk;
+    pk.load(reinterpret_cast<const uint4 *>(Kr) + rect_wave<S>(rp, seg, strip, j, w) * (Pack<KT>::NG * 64) + rl.slot, rl.lanes);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < S::BATCH; q++) {
@@ -751,12 +813,6 @@ __global__ void __launch_bounds__(S::WAVES * 64, sizeof(V) == 8 || sizeof(KT) ==
     // one), and its neighbours along k, which lie in the other parity's run
     const int own = act ? (NL + i - i0 + 1) * LINE + kp * HZ + ((k - kr0) >> 1) : (NL + 1) * LINE + kp * HZ + 1;
     const V *u0 = sd + own, *um = u0 + (kp ? -HZ : HZ - 1), *up = u0 + (kp ? 1 - HZ : HZ);
-    // the coefficients stay as loaded until here: widened earlier they would
-    // not fit the registers
-    auto hold = [](float kv[27]) {
-#pragma unroll
-        for (int e = 0; e < 27; e++) asm volatile("" : "+v"(kv[e]));
-    };
     auto gather = [&](int pl, V uv[27]) {
 #pragma unroll
         for (int dx = -1; dx <= 1; dx++)
@@ -769,27 +825,49 @@ __global__ void __launch_bounds__(S::WAVES * 64, sizeof(V) == 8 || sizeof(KT) ==
             }
     };
     V uv[27];
-    hold(kv[0]);
+    float kv[27];
+    pk.hold();
+    pk.template widen<0, 27>(kv);
     gather(-1, uv);
-    const V s0 = plane_sum_row<V>(kv[0], uv);
+    const V s0 = plane_sum_row<V>(kv, uv);
     __builtin_amdgcn_sched_barrier(0);   // one plane's entries live at a time
-    hold(kv[2]);
+    pk.hold();
+    pk.template widen<54, 27>(kv);
     gather(1, uv);
-    const V s2 = plane_sum_row<V>(kv[2], uv);
+    const V s2 = plane_sum_row<V>(kv, uv);
     __builtin_amdgcn_sched_barrier(0);
-    const V m0 = u0[0], m1 = u0[2 * HZ], m2 = u0[4 * HZ];
+    pk.hold();
+    pk.template widen<27, 27>(kv);
+    // the plane's nine blocks from the entries before the launch; in its turn a
+    // colour forms again those whose entries have changed: odd k the two along
+    // k, odd lines the six on the lines beside
+    V tb[9];
+    auto block = [&](int bb) {
+        const V *v = bb % 3 == 0 ? um : bb % 3 == 1 ? u0 : up;
+        const int p = (bb / 3 - 1) * LINE;
+        return kv[3 * bb] * v[p] + kv[3 * bb + 1] * v[p + 2 * HZ] + kv[3 * bb + 2] * v[p + 4 * HZ];
+    };
+#pragma unroll
+    for (int bb = 0; bb < 9; bb++) tb[bb] = block(bb);
+    const V dr = u0[r < 3 ? r * 2 * HZ : 0];
 #pragma unroll 1
     for (int p = 0; p < 4; p++) {
         __syncthreads();
         if (ph == p) {
-            gather(0, uv);
-            uv[12] = m0;
-            uv[13] = m1;
-            uv[14] = m2;
-            const V o = (s0 + plane_sum_row<V>(kv[1], uv)) + s2;
+            if (ph & 1) {
+                tb[3] = block(3);
+                tb[5] = block(5);
+            }
+            if (ph & 2) {
+#pragma unroll
+                for (int dz = 0; dz < 3; dz++) {
+                    tb[dz] = block(dz);
+                    tb[6 + dz] = block(6 + dz);
+                }
+            }
+            const V o = (s0 + ((((tb[0] + tb[1]) + (tb[2] + tb[3])) + ((tb[4] + tb[5]) + (tb[6] + tb[7]))) + tb[8])) + s2;
             // FP16 rows are stored scaled by BI: t = BI F - (BI K) d
             const float tt = sizeof(KT) == 2 ? (float)(Fr * Br - o) : (float)((Fr - o) * Br);
-            const V dr = r == 0 ? m0 : r == 1 ? m1 : m2;
             if (act) sd[own + r * 2 * HZ] = dr + tt;
         }
     }
@@ -824,29 +902,50 @@ static RectPart rect_part(const Geo &g, int shape) {
     return RectPart{};
 }
 
-// the narrow shape, else the wide one, while there is at most one workgroup
-// per CU (measured above); larger levels pass colour by colour
+// the narrow shape while there are at most two workgroups to a CU, else the
+// wide one with at most one (measured above); larger levels pass colour by colour
 RectPart rect_planes(const Geo &g) {
     constexpr long CUS = 256;
     for (const RectPart &rp : {rect_part<RectNarrow>(g, 1), rect_part<RectWide>(g, 2)})
-        if (rp.shape && (long)(g.noy + 1) / 2 * rp.nstrip * rp.ns <= CUS) return rp;
+        if (rp.shape && (long)(g.noy + 1) / 2 * rp.nstrip * rp.ns <= (rp.shape == 1 ? 2 : 1) * CUS) return rp;
     return RectPart{};
 }
 
 template <typename V, typename KT>
-static void rect_launch(hipStream_t s, const Level &L, const KT *K, const V *BI, const V *F, int jpar, const V *dself,
+static void rect_launch(hipStream_t s, const Level &L, const KT *Kr, const V *BI, const V *F, int jpar, const V *dself,
                         const V *dside, V *dout, hipEvent_t e0, hipEvent_t e1) {
     const RectPart &rp = L.planes;
     const dim3 grid(rp.ns, rp.nstrip, (L.g.noy - jpar + 1) / 2);
     if (grid.z == 0) return;
     auto launch = [&](auto kern, int waves) {
         if (e0)
-            hipExtLaunchKernelGGL(kern, grid, dim3(64 * waves), 0, s, e0, e1, 0, L.g, rp, jpar, K, BI, F, dself, dside, dout);
+            hipExtLaunchKernelGGL(kern, grid, dim3(64 * waves), 0, s, e0, e1, 0, L.g, rp, jpar, Kr, BI, F, dself, dside, dout);
         else
-            hipLaunchKernelGGL(kern, grid, dim3(64 * waves), 0, s, L.g, rp, jpar, K, BI, F, dself, dside, dout);
+            hipLaunchKernelGGL(kern, grid, dim3(64 * waves), 0, s, L.g, rp, jpar, Kr, BI, F, dself, dside, dout);
     };
     if (rp.shape == 1) launch(k_gs_rect<V, KT, RectNarrow>, RectNarrow::WAVES);
     else launch(k_gs_rect<V, KT, RectWide>, RectWide::WAVES);
+}
+
+size_t rect_pack_elems(const Level &L, bool half) {
+    const RectPart &rp = L.planes;
+    return (size_t)L.g.noy * rp.nstrip * rp.ns * (rp.shape == 1 ? RectNarrow::WAVES : RectWide::WAVES) *
+           (half ? Pack<_Float16>::WAVE : Pack<float>::WAVE);
+}
+
+// the levels' packed coefficients, after the stiffness (and its FP16 rows)
+void rect_pack(hipStream_t s, const Level &L) {
+    const RectPart &rp = L.planes;
+    const dim3 grid(rp.ns, rp.nstrip, L.g.noy);
+    auto launch = [&](auto *K, auto *Kr) {
+        using KT = std::remove_const_t<std::remove_pointer_t<decltype(Kr)>>;
+        if (rp.shape == 1)
+            hipLaunchKernelGGL((k_rect_pack<KT, RectNarrow>), grid, dim3(64 * RectNarrow::WAVES), 0, s, L.g, rp, K, Kr);
+        else
+            hipLaunchKernelGGL((k_rect_pack<KT, RectWide>), grid, dim3(64 * RectWide::WAVES), 0, s, L.g, rp, K, Kr);
+    };
+    if (L.Kr) launch((const float *)L.K, L.Kr);
+    if (L.Krh) launch((const _Float16 *)L.Kh, (_Float16 *)L.Krh);
 }
 
 template <typename V>
@@ -854,11 +953,11 @@ void gs_rect(hipStream_t s, const Level &L, const V *BI, const V *F, int jpar, c
              hipEvent_t e0, hipEvent_t e1) {
     if constexpr (sizeof(V) == 4) {
         if (L.Kh) {
-            rect_launch<V, _Float16>(s, L, (const _Float16 *)L.Kh, BI, F, jpar, dself, dside, dout, e0, e1);
+            rect_launch<V, _Float16>(s, L, (const _Float16 *)L.Krh, BI, F, jpar, dself, dside, dout, e0, e1);
             return;
         }
     }
-    rect_launch<V, float>(s, L, (const float *)L.K, BI, F, jpar, dself, dside, dout, e0, e1);
+    rect_launch<V, float>(s, L, (const float *)L.Kr, BI, F, jpar, dself, dside, dout, e0, e1);
 }
 template void gs_rect<double>(hipStream_t, const Level &, const double *, const double *, int, const double *,
                               const double *, double *, hipEvent_t, hipEvent_t);
@@ -1295,33 +1394,20 @@ __device__ __forceinline__ BoxColour box_colour(const BoxPart &bp, int bz, int b
     return r;
 }
 
-// Box tiles: for the (box, colour) tile b 8 + c and y-plane P, each node's
-// 81 coefficients of that plane (K[ktile(q)][81 P + cc]) contiguous in
-// 16-byte groups of G = 4 (FP32) or 8 (FP16): [tile][P][cc / G][lane][cc % G],
-// so a wavefront reads its plane in 21 or 11 coalesced 16-byte loads per
-// lane rather than 81 four- or two-byte ones (a wavefront can have at most
-// 63 vector loads in flight).  Lanes past the colour's count and the
-// padding past cc = 80 hold zeros.
-template <typename KT>
-struct BoxTile {
-    static constexpr int G = 16 / (int)sizeof(KT);
-    static constexpr int NG = (81 + G - 1) / G;
-    static constexpr size_t PLANE = (size_t)NG * 64 * G;
-    static constexpr size_t TILE = 3 * PLANE;
-};
-
+// Box tiles: for the (box, colour) tile b 8 + c and y-plane P, each node's 81
+// coefficients of that plane (K[ktile(q)][81 P + cc]) packed.
 size_t box_tile_elems(const Level &L) {
-    return (size_t)L.nbox * 8 * (L.Kbox_half ? BoxTile<_Float16>::TILE : BoxTile<float>::TILE);
+    return (size_t)L.nbox * 8 * 3 * (L.Kbox_half ? Pack<_Float16>::WAVE : Pack<float>::WAVE);
 }
 
 template <typename KT>
 __global__ void __launch_bounds__(64) k_box_tiles(Geo g, BoxPart bp, const KT *__restrict__ K, KT *__restrict__ Kb) {
-    using BT = BoxTile<KT>;
+    using BT = Pack<KT>;
     const int tile = blockIdx.x, lane = threadIdx.x;
     const int b = tile >> 3, c = tile & 7;
     const int bz = b % bp.n[0], bx = (b / bp.n[0]) % bp.n[1], by = b / (bp.n[0] * bp.n[1]);
     const BoxColour bc = box_colour(bp, bz, bx, by, c);
-    KT *dst = Kb + (size_t)tile * BT::TILE + lane * BT::G;
+    KT *dst = Kb + (size_t)tile * (3 * BT::WAVE) + lane * BT::G;
     const bool act = lane < bc.nz * bc.nx * bc.ny;
     const KT *src = K;
     if (act) {
@@ -1331,7 +1417,7 @@ __global__ void __launch_bounds__(64) k_box_tiles(Geo g, BoxPart bp, const KT *_
     }
     for (int P = 0; P < 3; P++)
         for (int cc = 0; cc < BT::NG * BT::G; cc++)
-            dst[P * BT::PLANE + (size_t)(cc / BT::G) * 64 * BT::G + cc % BT::G] =
+            dst[P * BT::WAVE + (size_t)(cc / BT::G) * 64 * BT::G + cc % BT::G] =
                 act && cc < 81 ? src[(81 * P + cc) * 64] : KT(0);
 }
 
@@ -1348,21 +1434,6 @@ void box_tiles(hipStream_t s, const Level &L) {
 constexpr int BOXH = BOX + 2;   // box side with its halo
 static_assert(BOX <= 8, "a box holds at most 64 nodes of one colour");
 
-// one plane's coefficients of one lane, as loaded (16-byte groups)
-template <typename KT>
-struct BoxCoefs {
-    uint4 q[BoxTile<KT>::NG];
-    __device__ __forceinline__ void load(const uint4 *__restrict__ p) {
-#pragma unroll
-        for (int t = 0; t < BoxTile<KT>::NG; t++) q[t] = p[t * 64];
-    }
-    __device__ __forceinline__ void widen(float kv[81]) const {
-        const KT *e = reinterpret_cast<const KT *>(q);
-#pragma unroll
-        for (int ci = 0; ci < 81; ci++) kv[ci] = (float)e[ci];
-    }
-};
-
 // One colour pass of a box: wavefront w forms y-plane w of the three rows
 // of the colour's (at most 64) nodes with the coefficients kc, then requests
 // the coefficients of the colour two ahead (kn) into kc before the workgroup
@@ -1371,7 +1442,7 @@ struct BoxCoefs {
 template <typename KT>
 __device__ __forceinline__ void box_pass(const Geo &g, const BoxPart &bp, int bz, int bx, int by, int c, int z0,
                                          int x0, int y0, int hz, int hx, int nz, int nx, float *sd,
-                                         const float *sF, const float *sB, float (*Ps)[3][64], BoxCoefs<KT> &kc,
+                                         const float *sF, const float *sB, float (*Ps)[3][64], Pack<KT> &kc,
                                          const uint4 *__restrict__ kn) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const BoxColour bc = box_colour(bp, bz, bx, by, c);
@@ -1405,7 +1476,7 @@ __device__ __forceinline__ void box_pass(const Geo &g, const BoxPart &bp, int bz
             }
         }
         float kv[81], out[3];
-        kc.widen(kv);
+        kc.template widen<0, 81>(kv);
         plane_sums<float>(kv, uv, okb, out);
         Ps[w][0][lane] = out[0];
         Ps[w][1][lane] = out[1];
@@ -1430,7 +1501,7 @@ template <typename KT, bool ZIN>
 __global__ void __launch_bounds__(192) k_gs_box(Geo g, BoxPart bp, const KT *__restrict__ Kb,
                                                 const float *__restrict__ BI, const float *__restrict__ F,
                                                 const float *__restrict__ din, float *__restrict__ dout) {
-    using BT = BoxTile<KT>;
+    using BT = Pack<KT>;
     __shared__ float sd[BOXH * BOXH * BOXH * 3];
     __shared__ float sF[BOX * BOX * BOX * 3], sB[BOX * BOX * BOX * 3];   // the box's own F and BI
     __shared__ float Ps[3][3][64];   // [plane][row][node]
@@ -1442,10 +1513,10 @@ __global__ void __launch_bounds__(192) k_gs_box(Geo g, BoxPart bp, const KT *__r
     const int nz = hz - 2, nx = hx - 2, ny = hy - 2;
     // this wavefront's plane of colour c's tile, lane's first group
     auto plane = [&](int c) {
-        return reinterpret_cast<const uint4 *>(Kb + ((size_t)b * 8 + c) * BT::TILE + w * BT::PLANE) + lane;
+        return reinterpret_cast<const uint4 *>(Kb + ((size_t)b * 8 + c) * (3 * BT::WAVE) + w * BT::WAVE) + lane;
     };
     // the first two colours' coefficients, in flight while the box loads
-    BoxCoefs<KT> ka, kb;
+    Pack<KT> ka, kb;
     ka.load(plane(0));
     kb.load(plane(1));
     for (int t = threadIdx.x; t < nz * nx * ny; t += 192) {

@@ -504,6 +504,7 @@ int build_mesh(chip_ctx *c) {
         Level &L = c->L[lev];
         L.planes = rect_planes(L.g);
         if (!L.planes.shape) continue;
+        if (dev_alloc(c, &L.Kr, rect_pack_elems(L, false)) || (L.Kh && dev_alloc(c, &L.Krh, rect_pack_elems(L, true)))) return -1;
         if (!L.tmp && dev_alloc(c, &L.tmp, 3 * (size_t)L.g.nno)) return -1;
         if (p.mixed && !L.tmpf && dev_alloc(c, &L.tmpf, 3 * (size_t)L.g.nno)) return -1;
     }

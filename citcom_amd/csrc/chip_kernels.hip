@@ -250,6 +250,16 @@ __device__ __forceinline__ V vload(const V *__restrict__ p) {
         return *p;
 }
 
+// a coefficient of a stream read once: kept out of the caches that hold the
+// vectors where the level's coefficients do not fit them anyway (streamed)
+template <bool STREAM, typename KT>
+__device__ __forceinline__ KT kload(const KT *__restrict__ p) {
+    if constexpr (STREAM)
+        return __builtin_nontemporal_load(p);
+    else
+        return *p;
+}
+
 // Plane P = dy+1 of the three rows of node (k, i, j), coefficients kp (its
 // tile column), into P[r]; arithmetic in the vector type V.
 // The three parts of plane_rows: the neighbours' vector entries (and which
@@ -275,10 +285,10 @@ __device__ __forceinline__ void plane_gather(const Geo &g, int k, int i, int j, 
     }
 }
 
-template <int P, typename KT>
+template <int P, bool STREAM, typename KT>
 __device__ __forceinline__ void plane_coefs(const KT *__restrict__ kp, float kv[81]) {
 #pragma unroll
-    for (int c = 0; c < 81; c++) kv[c] = (float)kp[(81 * P + c) * 64];
+    for (int c = 0; c < 81; c++) kv[c] = (float)kload<STREAM>(kp + (81 * P + c) * 64);
 }
 
 template <typename V>
@@ -309,14 +319,14 @@ __device__ __forceinline__ void plane_sums(const float kv[81], const V uv[27], c
     }
 }
 
-template <int P, typename V, typename KT>
+template <int P, bool STREAM, typename V, typename KT>
 __device__ __forceinline__ void plane_rows(const Geo &g, const KT *__restrict__ kp, int k, int i, int j, int self,
                                            const V *__restrict__ u, V out[3]) {
     float kv[81];
     V uv[27];
     bool okb[9];
     plane_gather<P, V, false>(g, k, i, j, self, u, uv, okb);
-    plane_coefs<P, KT>(kp, kv);
+    plane_coefs<P, STREAM, KT>(kp, kv);
     plane_sums<V>(kv, uv, okb, out);
 }
 
@@ -358,9 +368,10 @@ __global__ void __launch_bounds__(256) k_matvec(Geo g, const KT *__restrict__ K,
 // of row_product_t); planes 1 and 2 hand their terms to wavefront 0 through
 // LDS, which adds all 27 terms in row_product_t's sequential order, so the
 // result has the same bits as k_matvec's while three planes' loads are in
-// flight at once.
-template <typename V, typename KT>
-__global__ void __launch_bounds__(192) k_matvec3(Geo g, const KT *__restrict__ K, const unsigned *__restrict__ NODE,
+// flight at once.  Four wavefronts a SIMD: at most 128 registers (FP64 needs 129
+// left alone, and ran three).
+template <typename V, typename KT, bool STREAM>
+__global__ void __launch_bounds__(192, 4) k_matvec3(Geo g, const KT *__restrict__ K, const unsigned *__restrict__ NODE,
                                                  const V *__restrict__ u, V *__restrict__ Au,
                                                  const V *__restrict__ rhs, V *__restrict__ res,
                                                  const V *__restrict__ BIs, V *__restrict__ ucopy) {
@@ -392,7 +403,7 @@ __global__ void __launch_bounds__(192) k_matvec3(Geo g, const KT *__restrict__ K
             }
         }
 #pragma unroll
-        for (int c = 0; c < 81; c++) kv[c] = (float)kp[(81 * P + c) * 64];
+        for (int c = 0; c < 81; c++) kv[c] = (float)kload<STREAM>(kp + (81 * P + c) * 64);
 #pragma unroll
         for (int b = 0; b < 9; b++)
 #pragma unroll
@@ -483,6 +494,18 @@ __device__ __forceinline__ void row_product_all(const Geo &g, const float *__res
             }
 }
 
+// Levels whose coefficients are read past the caches: a sweep of a level of
+// more than the 256 MB of the Infinity Cache finds none of them there again,
+// and read plainly they put out the vectors, which the next colours read again
+// (129x129x65 nodes, 1042 MB: a colour pass in FP64 35.4 us -> 33.4, the FP64
+// residual 242 -> 232; 521 MB in FP16 19.1 -> 17.2; 65x65x65 nodes, 267 MB:
+// 11.6 -> 11.2).  The product after a sweep still finds a part of a level not
+// much larger (267 MB: 54 us, past the caches 60).  Levels that fit lose
+// (65x65x33 nodes, 136 MB: 7.4 -> 8.1 us, product 28 -> 33).
+constexpr double GS_STREAM = 256e6, MV_STREAM = 400e6;
+template <typename KT>
+static bool streamed(const Level &L, double limit) { return (double)L.g.pitch * KROW * sizeof(KT) > limit; }
+
 constexpr int MV_SMALL_NNO = 20000;   // levels up to this size use k_matvec_small
 
 template <typename V>
@@ -529,27 +552,24 @@ void matvec(hipStream_t s, const Level &L, const V *u, V *Au, const V *rhs, V *r
         return;
     }
     const int tiles = L.g.pitch / 64;   // the colour index space is whole 64-node tiles
+    auto launch = [&](auto kern, const auto *K, const V *BIs) {
+        if (e0)
+            hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, K, L.NODE, u, Au, rhs, res, BIs, ucopy);
+        else
+            hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, K, L.NODE, u, Au, rhs, res, BIs, ucopy);
+    };
     if constexpr (sizeof(V) == 4) {
         if (L.Kh) {
             const _Float16 *Kh = (const _Float16 *)L.Kh;
-            const V *BIs = (const V *)L.BIf;
-            auto kern = k_matvec3<V, _Float16>;
-            if (e0)
-                hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, Kh, L.NODE, u, Au, rhs, res,
-                                      BIs, ucopy);
-            else
-                hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, Kh, L.NODE, u, Au, rhs, res, BIs, ucopy);
+            if (streamed<_Float16>(L, MV_STREAM)) launch(k_matvec3<V, _Float16, true>, Kh, (const V *)L.BIf);
+            else launch(k_matvec3<V, _Float16, false>, Kh, (const V *)L.BIf);
             return;
         }
     }
     const V *none = nullptr;
     const float *K = L.K;
-    auto kern = k_matvec3<V, float>;
-    if (e0)
-        hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, K, L.NODE, u, Au, rhs, res, none,
-                              ucopy);
-    else
-        hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, K, L.NODE, u, Au, rhs, res, none, ucopy);
+    if (streamed<float>(L, MV_STREAM)) launch(k_matvec3<V, float, true>, K, none);
+    else launch(k_matvec3<V, float, false>, K, none);
 }
 template void matvec<double>(hipStream_t, const Level &, const double *, double *, const double *, double *,
                              hipEvent_t, hipEvent_t, double *);
@@ -564,7 +584,7 @@ template void matvec<float>(hipStream_t, const Level &, const float *, float *, 
 // together), the partial sums meet in LDS, and wavefront r updates row r.
 // Every row is formed before any unknown is written (workgroup barrier), as
 // the reference updates all three unknowns of a node from the same Ad.
-template <typename V, typename KT>
+template <typename V, typename KT, bool STREAM>
 __global__ void __launch_bounds__(192) k_gs_colour(Geo g, int c, const KT *__restrict__ K,
                                                    const V *__restrict__ BI, V *d, const V *__restrict__ F) {
     __shared__ V Ps[3][3][64];   // [plane][row][node]
@@ -586,11 +606,11 @@ __global__ void __launch_bounds__(192) k_gs_colour(Geo g, int c, const KT *__res
         V out[3];
         const KT *kp = K + ktile(q);
         if (w == 0)
-            plane_rows<0>(g, kp, k, i, j, self, (const V *)d, out);
+            plane_rows<0, STREAM>(g, kp, k, i, j, self, (const V *)d, out);
         else if (w == 1)
-            plane_rows<1>(g, kp, k, i, j, self, (const V *)d, out);
+            plane_rows<1, STREAM>(g, kp, k, i, j, self, (const V *)d, out);
         else
-            plane_rows<2>(g, kp, k, i, j, self, (const V *)d, out);
+            plane_rows<2, STREAM>(g, kp, k, i, j, self, (const V *)d, out);
         Ps[w][0][lane] = out[0];
         Ps[w][1][lane] = out[1];
         Ps[w][2][lane] = out[2];
@@ -608,23 +628,23 @@ __global__ void __launch_bounds__(192) k_gs_colour(Geo g, int c, const KT *__res
 template <typename V>
 void gs_colour(hipStream_t s, const Level &L, const V *BI, int colour, V *d, const V *F, hipEvent_t e0, hipEvent_t e1) {
     const int tiles = (L.g.cn[colour] + 63) / 64;
+    auto launch = [&](auto kern, const auto *K) {
+        if (e0)
+            hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, colour, K, BI, d, F);
+        else
+            hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, colour, K, BI, d, F);
+    };
     if constexpr (sizeof(V) == 4) {
         if (L.Kh) {
             const _Float16 *Kh = (const _Float16 *)L.Kh;
-            auto kern = k_gs_colour<V, _Float16>;
-            if (e0)
-                hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, colour, Kh, BI, d, F);
-            else
-                hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, colour, Kh, BI, d, F);
+            if (streamed<_Float16>(L, GS_STREAM)) launch(k_gs_colour<V, _Float16, true>, Kh);
+            else launch(k_gs_colour<V, _Float16, false>, Kh);
             return;
         }
     }
     const float *K = L.K;
-    auto kern = k_gs_colour<V, float>;
-    if (e0)
-        hipExtLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, e0, e1, 0, L.g, colour, K, BI, d, F);
-    else
-        hipLaunchKernelGGL(kern, dim3(tiles), dim3(192), 0, s, L.g, colour, K, BI, d, F);
+    if (streamed<float>(L, GS_STREAM)) launch(k_gs_colour<V, float, true>, K);
+    else launch(k_gs_colour<V, float, false>, K);
 }
 template void gs_colour<double>(hipStream_t, const Level &, const double *, int, double *, const double *, hipEvent_t,
                                 hipEvent_t);
@@ -1233,13 +1253,13 @@ __global__ void __launch_bounds__(192) k_gs_xcd(Geo g, const float *__restrict__
                     bool okb[9];
                     if (w == 0) {
                         plane_gather<0, V, true>(g, k, i, j, self, d, uv, okb);
-                        plane_coefs<0, float>(kp, kv);
+                        plane_coefs<0, false, float>(kp, kv);
                     } else if (w == 1) {
                         plane_gather<1, V, true>(g, k, i, j, self, d, uv, okb);
-                        plane_coefs<1, float>(kp, kv);
+                        plane_coefs<1, false, float>(kp, kv);
                     } else {
                         plane_gather<2, V, true>(g, k, i, j, self, d, uv, okb);
-                        plane_coefs<2, float>(kp, kv);
+                        plane_coefs<2, false, float>(kp, kv);
                     }
                     plane_sums<V>(kv, uv, okb, out);
                     Ps[w][0][lane] = out[0];

@@ -714,6 +714,17 @@ struct Pack {
 #pragma unroll
         for (int t = 0; t < NG; t++) q[t] = p[t * lanes];
     }
+    template <int P>
+    __device__ __forceinline__ void hold_plane() {
+#pragma unroll
+        for (int t = 27 * P / G; t <= (27 * P + 26) / G; t++)
+            asm volatile("" : "+v"(q[t].x), "+v"(q[t].y), "+v"(q[t].z), "+v"(q[t].w));
+    }
+    template <int FROM, int TO>
+    __device__ __forceinline__ void load_part(const uint4 *__restrict__ p) {
+#pragma unroll
+        for (int t = FROM; t < TO; t++) q[t] = p[t * 64];
+    }
     // the values as loaded up to here: widened earlier they would not fit the registers
     __device__ __forceinline__ void hold() {
 #pragma unroll
@@ -1414,8 +1425,8 @@ __device__ __forceinline__ BoxColour box_colour(const BoxPart &bp, int bz, int b
     return r;
 }
 
-// Box tiles: for the (box, colour) tile b 8 + c and y-plane P, each node's 81
-// coefficients of that plane (K[ktile(q)][81 P + cc]) packed.
+// Box tiles: for the (box, colour) tile b 8 + c and row r, each node's 81
+// coefficients of that row, plane by plane, packed.
 size_t box_tile_elems(const Level &L) {
     return (size_t)L.nbox * 8 * 3 * (L.Kbox_half ? Pack<_Float16>::WAVE : Pack<float>::WAVE);
 }
@@ -1435,10 +1446,10 @@ __global__ void __launch_bounds__(64) k_box_tiles(Geo g, BoxPart bp, const KT *_
         const int k = bc.k0 + 2 * kk, i = bc.i0 + 2 * (t % bc.nx), j = bc.j0 + 2 * (t / bc.nx);
         src = K + ktile(colour_index(g, c, k, i, j));
     }
-    for (int P = 0; P < 3; P++)
+    for (int r = 0; r < 3; r++)
         for (int cc = 0; cc < BT::NG * BT::G; cc++)
-            dst[P * BT::WAVE + (size_t)(cc / BT::G) * 64 * BT::G + cc % BT::G] =
-                act && cc < 81 ? src[(81 * P + cc) * 64] : KT(0);
+            dst[r * BT::WAVE + (size_t)(cc / BT::G) * 64 * BT::G + cc % BT::G] =
+                act && cc < 81 ? src[(81 * (cc / 27) + 9 * (cc % 27 / 3) + 3 * r + cc % 3) * 64] : KT(0);
 }
 
 void box_tiles(hipStream_t s, const Level &L) {
@@ -1453,136 +1464,153 @@ void box_tiles(hipStream_t s, const Level &L) {
 
 constexpr int BOXH = BOX + 2;   // box side with its halo
 static_assert(BOX <= 8, "a box holds at most 64 nodes of one colour");
-
-// One colour pass of a box: wavefront w forms y-plane w of the three rows
-// of the colour's (at most 64) nodes with the coefficients kc, then requests
-// the coefficients of the colour two ahead (kn) into kc before the workgroup
-// barriers, so their latency overlaps this colour's update and the next
-// colour's pass.
-template <typename KT>
-__device__ __forceinline__ void box_pass(const Geo &g, const BoxPart &bp, int bz, int bx, int by, int c, int z0,
-                                         int x0, int y0, int hz, int hx, int nz, int nx, float *sd,
-                                         const float *sF, const float *sB, float (*Ps)[3][64], Pack<KT> &kc,
-                                         const uint4 *__restrict__ kn) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const BoxColour bc = box_colour(bp, bz, bx, by, c);
-    const bool act = lane < bc.nz * bc.nx * bc.ny;
-    int k = 0, i = 0, j = 0;
-    if (act) {
-        const int kk = lane % bc.nz, t = lane / bc.nz;
-        k = bc.k0 + 2 * kk;
-        i = bc.i0 + 2 * (t % bc.nx);
-        j = bc.j0 + 2 * (t / bc.nx);
-    }
-    const int lself = (k - z0 + 1) + hz * ((i - x0 + 1) + hx * (j - y0 + 1));
-    const int lown = (k - z0) + nz * ((i - x0) + nx * (j - y0));
-    if (act) {
-        // plane w: the 9 neighbours (dz, dx) at dy = w - 1
-        float uv[27];
-        bool okb[9];
-        const int dy = w - 1;
-        const bool oy = (unsigned)(j + dy) < (unsigned)g.noy;
-#pragma unroll
-        for (int dx = -1; dx <= 1; dx++) {
-            const bool ox = oy && (unsigned)(i + dx) < (unsigned)g.nox;
-#pragma unroll
-            for (int dz = -1; dz <= 1; dz++) {
-                const int bb = (dz + 1) + 3 * (dx + 1);
-                okb[bb] = ox && (unsigned)(k + dz) < (unsigned)g.noz;
-                const int m = 3 * (lself + dz + hz * (dx + hx * dy));
-                uv[3 * bb] = sd[m];
-                uv[3 * bb + 1] = sd[m + 1];
-                uv[3 * bb + 2] = sd[m + 2];
-            }
-        }
-        float kv[81], out[3];
-        kc.template widen<0, 81>(kv);
-        plane_sums<float>(kv, uv, okb, out);
-        Ps[w][0][lane] = out[0];
-        Ps[w][1][lane] = out[1];
-        Ps[w][2][lane] = out[2];
-    }
-    // unconditional (the last colour's again near the end), so that no wait
-    // is placed on these loads before their use two passes later
-    kc.load(kn);
-    __syncthreads();
-    if (act) {
-        const float Fr = sF[3 * lown + w], Br = sB[3 * lown + w];
-        const float o = (Ps[0][w][lane] + Ps[1][w][lane]) + Ps[2][w][lane];
-        // FP16 rows are stored scaled by BI: t = BI F - (BI K) d
-        const float t = sizeof(KT) == 2 ? Fr * Br - o : (Fr - o) * Br;
-        sd[3 * lself + w] += t;
-    }
-    __syncthreads();
-}
+constexpr int BOX_TPB = 768;
 
 // One sweep, a workgroup per box.  ZIN: din is zero (not read).
+//
+// Twelve wavefronts: a row of a colour each, four colours (those of the even
+// or of the odd y-planes) at a time, as k_gs_rect: no colour of the four
+// changes the planes beside, so all wavefronts form these sums and the blocks
+// of the own plane at once, and in its turn a colour only forms the blocks
+// again whose entries have changed, one barrier a colour.  The coefficients of
+// the second four are requested when the first four's have been used but for
+// the own plane's (FP16: as many as 80 registers hold, two workgroups to a CU).
+// A sweep, before (a y-plane of the three rows to each of three wavefronts, two
+// barriers a colour) -> now: 33x33x17 nodes in FP32 16.7 us -> 13.8, 17x33x33 in
+// FP16 14.0 -> 9.8; 65x65x33 in FP16 24.9 -> 24.4.  Bound by latency, eight
+// colours in turn, on 75 or 45 boxes for 256 CUs; the last, two boxes to a CU,
+// by the LDS reads and arithmetic of three times the lanes.
 template <typename KT, bool ZIN>
-__global__ void __launch_bounds__(192) k_gs_box(Geo g, BoxPart bp, const KT *__restrict__ Kb,
-                                                const float *__restrict__ BI, const float *__restrict__ F,
-                                                const float *__restrict__ din, float *__restrict__ dout) {
+__global__ void __launch_bounds__(BOX_TPB, sizeof(KT) == 2 ? 6 : 3) k_gs_box(Geo g, BoxPart bp, const KT *__restrict__ Kb,
+                                                    const float *__restrict__ BI, const float *__restrict__ F,
+                                                    const float *__restrict__ din, float *__restrict__ dout) {
     using BT = Pack<KT>;
-    __shared__ float sd[BOXH * BOXH * BOXH * 3];
-    __shared__ float sF[BOX * BOX * BOX * 3], sB[BOX * BOX * BOX * 3];   // the box's own F and BI
-    __shared__ float Ps[3][3][64];   // [plane][row][node]
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int b = blockIdx.x;
+    // [component][y][x][parity of z][z / 2]: a colour's nodes 1, 20 and 260
+    // words apart, all but twelve in banks of their own
+    constexpr int EARLY = sizeof(KT) == 2 ? 6 : BT::NG;   // FP16: what 80 registers hold
+    constexpr int HS = BOXH / 2, XS = BOXH, YS = 130, CS = BOXH * YS;
+    __shared__ float sd[3 * CS];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ph = w / 3, r = w - 3 * ph, b = blockIdx.x;
     const int bz = b % bp.n[0], bx = (b / bp.n[0]) % bp.n[1], by = b / (bp.n[0] * bp.n[1]);
     const int z0 = bp.s[0][bz], x0 = bp.s[1][bx], y0 = bp.s[2][by];
     const int hz = bp.s[0][bz + 1] - z0 + 2, hx = bp.s[1][bx + 1] - x0 + 2, hy = bp.s[2][by + 1] - y0 + 2;
-    const int nz = hz - 2, nx = hx - 2, ny = hy - 2;
-    // this wavefront's plane of colour c's tile, lane's first group
-    auto plane = [&](int c) {
-        return reinterpret_cast<const uint4 *>(Kb + ((size_t)b * 8 + c) * (3 * BT::WAVE) + w * BT::WAVE) + lane;
+    auto place = [](int lz, int lx, int ly) { return ly * YS + lx * XS + (lz & 1) * HS + (lz >> 1); };
+    // this wavefront's colour of either half: the lane's node (an idle lane's: the box's first)
+    int own[2], fg[2];
+    bool act[2];
+    Pack<KT> pk;
+    auto tile = [&](int h) {
+        return reinterpret_cast<const uint4 *>(Kb + ((size_t)b * 8 + ph + 4 * h) * (3 * BT::WAVE) + r * BT::WAVE) + lane;
     };
-    // the first two colours' coefficients, in flight while the box loads
-    Pack<KT> ka, kb;
-    ka.load(plane(0));
-    kb.load(plane(1));
-    for (int t = threadIdx.x; t < nz * nx * ny; t += 192) {
-        const int lz = t % nz, r = t / nz, lx = r % nx, ly = r / nx;
-        const int n = nid(g, z0 + lz, x0 + lx, y0 + ly);
+    pk.load(tile(0));
 #pragma unroll
-        for (int e = 0; e < 3; e++) {
-            sF[3 * t + e] = F[3 * n + e];
-            sB[3 * t + e] = BI[3 * n + e];
-        }
+    for (int h = 0; h < 2; h++) {
+        const BoxColour bc = box_colour(bp, bz, bx, by, ph + 4 * h);
+        act[h] = lane < bc.nz * bc.nx * bc.ny;
+        const int nz = max(bc.nz, 1), nx = max(bc.nx, 1), kk = lane % nz, t = lane / nz;
+        const int k = act[h] ? bc.k0 + 2 * kk : z0, i = act[h] ? bc.i0 + 2 * (t % nx) : x0, j = act[h] ? bc.j0 + 2 * (t / nx) : y0;
+        own[h] = place(k - z0 + 1, i - x0 + 1, j - y0 + 1);
+        fg[h] = 3 * nid(g, k, i, j) + r;
     }
-    // the box and its halo; entries outside the mesh are zero and never read
-    for (int t = threadIdx.x; t < hz * hx * hy; t += 192) {
-        const int lz = t % hz, r = t / hz, lx = r % hx, ly = r / hx;
+    const float Fr[2] = {F[fg[0]], F[fg[1]]}, Br[2] = {BI[fg[0]], BI[fg[1]]};
+    // the box and its halo, zero outside the mesh
+    constexpr int BATCH = (BOXH * BOXH * BOXH + BOX_TPB - 1) / BOX_TPB;
+#pragma unroll
+    for (int q = 0; q < BATCH; q++) {
+        const int t = threadIdx.x + q * BOX_TPB;
+        const int lz = t % hz, u = t / hz, lx = u % hx, ly = u / hx;
         const int k = z0 - 1 + lz, i = x0 - 1 + lx, j = y0 - 1 + ly;
-        float v0 = 0.0f, v1 = 0.0f, v2 = 0.0f;
-        if (!ZIN && (unsigned)k < (unsigned)g.noz && (unsigned)i < (unsigned)g.nox && (unsigned)j < (unsigned)g.noy) {
+        float v[3] = {0.0f, 0.0f, 0.0f};
+        if (!ZIN && ly < hy && (unsigned)k < (unsigned)g.noz && (unsigned)i < (unsigned)g.nox && (unsigned)j < (unsigned)g.noy) {
             const int n = nid(g, k, i, j);
-            v0 = din[3 * n];
-            v1 = din[3 * n + 1];
-            v2 = din[3 * n + 2];
+#pragma unroll
+            for (int e = 0; e < 3; e++) v[e] = din[3 * n + e];
         }
-        sd[3 * t] = v0;
-        sd[3 * t + 1] = v1;
-        sd[3 * t + 2] = v2;
+        if (ly < hy)
+#pragma unroll
+            for (int e = 0; e < 3; e++) sd[e * CS + place(lz, lx, ly)] = v[e];
     }
     __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const bool odd = (((ph & 1) ^ z0) & 1) == 0;   // parity of the nodes' place along z
+        float *u0 = sd + own[h];
+        const float *um = u0 + (odd ? -HS : HS - 1), *up = u0 + (odd ? 1 - HS : HS);
+        auto block = [&](const Pack<KT> &c, int P, int bb) {
+            const KT *e = reinterpret_cast<const KT *>(c.q) + 27 * P + 3 * bb;
+            const float *v = (bb % 3 == 0 ? um : bb % 3 == 1 ? u0 : up) + (P - 1) * YS + (bb / 3 - 1) * XS;
+            return (float)e[0] * v[0] + (float)e[1] * v[CS] + (float)e[2] * v[2 * CS];
+        };
+        auto tree = [](const float t[9]) { return (((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) + t[8]; };
+        // FP16: two workgroups to a CU, for which a line's entries are live at a time
+        auto narrow = [](float &v, int bb) {
+            asm volatile("" : "+v"(v));
+            if (sizeof(KT) == 2 && bb % 3 == 2) __builtin_amdgcn_sched_barrier(0);
+        };
+        auto side = [&](int P) {
+            float t[9];
+#pragma unroll
+            for (int bb = 0; bb < 9; bb++) {
+                t[bb] = block(pk, P, bb);
+                narrow(t[bb], bb);
+            }
+            float v = tree(t);
+            asm volatile("" : "+v"(v));
+            __builtin_amdgcn_sched_barrier(0);   // one plane's entries live at a time
+            return v;
+        };
+        pk.template hold_plane<0>();
+        const float s0 = side(0);
+        pk.template hold_plane<2>();
+        const float s2 = side(2);
+        const Pack<KT> mid = pk;   // of which the own plane's are still needed
+        float tb[9];
+#pragma unroll
+        for (int bb = 0; bb < 9; bb++) {
+            tb[bb] = block(mid, 1, bb);
+            narrow(tb[bb], bb);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (h == 0) pk.template load_part<0, EARLY>(tile(1));
+        const float dr = u0[r * CS];
 #pragma unroll 1
-    for (int c = 0; c < 8; c += 2) {
-        box_pass<KT>(g, bp, bz, bx, by, c, z0, x0, y0, hz, hx, nz, nx, sd, sF, sB, Ps, ka, plane(min(c + 2, 7)));
-        box_pass<KT>(g, bp, bz, bx, by, c + 1, z0, x0, y0, hz, hx, nz, nx, sd, sF, sB, Ps, kb, plane(min(c + 3, 7)));
+        for (int p = 0; p < 4; p++) {
+            __syncthreads();
+            if (ph == p) {
+                if (ph & 1) {
+                    tb[3] = block(mid, 1, 3);
+                    tb[5] = block(mid, 1, 5);
+                }
+                if (ph & 2) {
+#pragma unroll
+                    for (int dz = 0; dz < 3; dz++) {
+                        tb[dz] = block(mid, 1, dz);
+                        tb[6 + dz] = block(mid, 1, 6 + dz);
+                    }
+                }
+                const float o = (s0 + tree(tb)) + s2;
+                // FP16 rows are stored scaled by BI: t = BI F - (BI K) d
+                const float t = sizeof(KT) == 2 ? Fr[h] * Br[h] - o : (Fr[h] - o) * Br[h];
+                if (act[h]) u0[r * CS] = dr + t;
+            }
+        }
+        if (h == 0) pk.template load_part<EARLY, BT::NG>(tile(1));
+        __syncthreads();
     }
     // the box's own nodes
-    for (int t = threadIdx.x; t < nz * nx * ny; t += 192) {
-        const int lz = t % nz, r = t / nz, lx = r % nx, ly = r / nx;
-        const int n = nid(g, z0 + lz, x0 + lx, y0 + ly);
-        const int m = 3 * ((lz + 1) + hz * ((lx + 1) + hx * (ly + 1)));
-        dout[3 * n] = sd[m];
-        dout[3 * n + 1] = sd[m + 1];
-        dout[3 * n + 2] = sd[m + 2];
+    const int nz = hz - 2, nx = hx - 2, ny = hy - 2;
+    if (const int t = threadIdx.x; t < nz * nx * ny) {
+        const int lz = t % nz, u = t / nz, lx = u % nx, ly = u / nx;
+        const int n = nid(g, z0 + lz, x0 + lx, y0 + ly), m = place(lz + 1, lx + 1, ly + 1);
+#pragma unroll
+        for (int e = 0; e < 3; e++) dout[3 * n + e] = sd[e * CS + m];
     }
 }
 
 void gs_box(hipStream_t s, const Level &L, const float *BI, const float *din, float *dout, const float *F,
             hipEvent_t e0, hipEvent_t e1) {
-    const dim3 grid(L.nbox), block(192);
+    const dim3 grid(L.nbox), block(BOX_TPB);
     auto launch = [&](auto kern, const auto *Kb) {
         if (e0)
             hipExtLaunchKernelGGL(kern, grid, block, 0, s, e0, e1, 0, L.g, L.bp, Kb, BI, F, din, dout);

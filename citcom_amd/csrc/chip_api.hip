@@ -577,7 +577,7 @@ int direct_take(chip_ctx *c, int *state) {
     *state = 2;
     if (info[0] != 0 || info[1] != 0) return 0;
     const size_t n = 3 * (size_t)c->L[c->dlev].g.nno;
-    CHIP_CHECK(hipMemcpyAsync(c->dAh, c->dAh_stage, n * n * sizeof(uint16_t), hipMemcpyDeviceToDevice, S(c)));
+    CHIP_CHECK(hipMemcpyAsync(c->dAh, c->dAh_stage, n * dense_pitch((int)n) * sizeof(uint16_t), hipMemcpyDeviceToDevice, S(c)));
     CHIP_CHECK(hipMemcpyAsync(c->dAs, c->dAs_stage, n * sizeof(float), hipMemcpyDeviceToDevice, S(c)));
     *state = 1;
     return 0;

@@ -85,6 +85,8 @@ void up_apply(hipStream_t s, const Level &L, const V *res, V *out);
 // entry, in FP16 (bits), and the scales; out = diag(sc) H F
 void dense_assemble(hipStream_t s, const Level &L, double *A);
 void sym_to_f32(hipStream_t s, const double *A, float *M, int n);
+// entries of a row of the scaled FP16 inverse: whole blocks of 256 columns
+__host__ __device__ inline int dense_pitch(int n) { return (n + 255) & ~255; }
 void rowscale_f16(hipStream_t s, const float *M, uint16_t *H, float *sc, int n);
 template <typename V>
 void dense_apply(hipStream_t s, const uint16_t *H, const float *sc, const V *F, V *out, int n);

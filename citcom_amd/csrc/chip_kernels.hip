@@ -1476,9 +1476,9 @@ constexpr int BOX_TPB = 768;
 // the second four are requested when the first four's have been used but for
 // the own plane's (FP16: as many as 80 registers hold, two workgroups to a CU).
 // A sweep, before (a y-plane of the three rows to each of three wavefronts, two
-// barriers a colour) -> now: 33x33x17 nodes in FP32 16.7 us -> 13.8, 17x33x33 in
+// barriers a colour) -> now: 33x33x17 nodes in FP32 16.7 us -> 13.8, 17x17x17 in
 // FP16 14.0 -> 9.8; 65x65x33 in FP16 24.9 -> 24.4.  Bound by latency, eight
-// colours in turn, on 75 or 45 boxes for 256 CUs; the last, two boxes to a CU,
+// colours in turn, on 75 or 27 boxes for 256 CUs; the last, two boxes to a CU,
 // by the LDS reads and arithmetic of three times the lanes.
 template <typename KT, bool ZIN>
 __global__ void __launch_bounds__(BOX_TPB, sizeof(KT) == 2 ? 6 : 3) k_gs_box(Geo g, BoxPart bp, const KT *__restrict__ Kb,
@@ -2292,7 +2292,26 @@ __global__ void __launch_bounds__(DOT_TPB) k_dots(int n, const V *__restrict__ a
 #pragma unroll
         for (int u = 0; u < 4; u++) w[m][u] = 0.0;
     const int stride = gridDim.x * blockDim.x;
-    for (int i0 = blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += 4 * stride) {
+    long i1 = blockIdx.x * blockDim.x + threadIdx.x;
+    // BATCH grid strides at a time with all their loads in flight, the sums in
+    // the same order (one pair of 3.2 M entries in FP64 21.6 us -> 14.3)
+    constexpr int BATCH = ND == 1 ? 16 : 8;
+    const V *const pa[4] = {a0, a1, a2, a3}, *const pb[4] = {b0, b1, b2, b3};
+    for (; i1 + (long)(BATCH - 1) * stride < n; i1 += (long)BATCH * stride) {
+        V x[ND][BATCH], y[ND][BATCH];
+#pragma unroll
+        for (int q = 0; q < BATCH; q++)
+#pragma unroll
+            for (int m = 0; m < ND; m++) {
+                x[m][q] = pa[m][i1 + (long)q * stride];
+                y[m][q] = pb[m][i1 + (long)q * stride];
+            }
+#pragma unroll
+        for (int q = 0; q < BATCH; q++)
+#pragma unroll
+            for (int m = 0; m < ND; m++) w[m][q & 3] += (double)x[m][q] * (double)y[m][q];
+    }
+    for (int i0 = (int)i1; i0 < n; i0 += 4 * stride) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int i = i0 + u * stride;

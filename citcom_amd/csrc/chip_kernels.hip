@@ -162,22 +162,6 @@ __device__ __forceinline__ void row_product_t(const Geo &g, KA kat, int k, int i
 }
 
 template <typename V>
-__device__ __forceinline__ void row_product(const Geo &g, const float *__restrict__ K, int q, int k, int i, int j,
-                                            const V *__restrict__ u, V out[3]) {
-    const float *kp = K + ktile(q);
-    row_product_t<V>(
-        g, [kp](int ci) { return kp[ci * 64]; }, k, i, j, [u](int idx) { return u[idx]; }, out);
-}
-
-// the same with the FP16 (row-scaled) coefficients, widened to FP32
-__device__ __forceinline__ void row_product(const Geo &g, const _Float16 *__restrict__ K, int q, int k, int i, int j,
-                                            const float *__restrict__ u, float out[3]) {
-    const _Float16 *kp = K + ktile(q);
-    row_product_t<float>(
-        g, [kp](int ci) { return (float)kp[ci * 64]; }, k, i, j, [u](int idx) { return u[idx]; }, out);
-}
-
-template <typename V>
 __device__ __forceinline__ void strip3(unsigned f, V v[3]) {
     if (f & VBX) v[0] = V(0);
     if (f & VBY) v[1] = V(0);
@@ -192,7 +176,7 @@ __device__ __forceinline__ void strip3(unsigned f, V v[3]) {
 // of 2w) into P[p], and the row sum is (P[0] + P[1]) + P[2].  A thread forms
 // a plane's tree in registers (PairSum16); a 16-lane row of a wavefront
 // forms the same tree with DPP row shifts (IEEE addition is commutative, so
-// both give the same bits).  The matvec keeps row_product's sequential order.
+// both give the same bits).  The matvec keeps row_product_t's sequential order.
 
 // tree over 16 slots formed term by term: push<B>(t[B]) for B = 0..15 keeps
 // one partial sum per tree level; after B = 15, total is t[0] of the tree
@@ -330,44 +314,13 @@ __device__ __forceinline__ void plane_rows(const Geo &g, const KT *__restrict__ 
     plane_sums<V>(kv, uv, okb, out);
 }
 
-// matvec: n_assemble_del2_u (Element_calculations.c:552-621) with strip;
-// optionally res = rhs - Au.  One thread per node: the three rows share the
-// 27 vector gathers.
-template <typename V, typename KT>
-__global__ void __launch_bounds__(256) k_matvec(Geo g, const KT *__restrict__ K, const unsigned *__restrict__ NODE,
-                                                const V *__restrict__ u, V *__restrict__ Au,
-                                                const V *__restrict__ rhs, V *__restrict__ res,
-                                                const V *__restrict__ BIs) {
-    const int q = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    const int col = colour_valid(g, q);
-    if (col < 0) return;
-    int k, i, j;
-    colour_kij(g, col, q, k, i, j);
-    V out[3];
-    row_product(g, K, q, k, i, j, u, out);
-    const int n = nid(g, k, i, j);
-    if (BIs) {  // rows stored scaled by BI: K d = (BI K) d / BI
-        out[0] = out[0] / BIs[3 * n];
-        out[1] = out[1] / BIs[3 * n + 1];
-        out[2] = out[2] / BIs[3 * n + 2];
-    }
-    strip3(NODE[n], out);
-    Au[3 * n] = out[0];
-    Au[3 * n + 1] = out[1];
-    Au[3 * n + 2] = out[2];
-    if (res) {
-        res[3 * n] = rhs[3 * n] - out[0];
-        res[3 * n + 1] = rhs[3 * n + 1] - out[1];
-        res[3 * n + 2] = rhs[3 * n + 2] - out[2];
-    }
-}
-
-// matvec of large levels with three wavefronts per 64-node tile: wavefront
+// matvec of large levels: n_assemble_del2_u (Element_calculations.c:552-621)
+// with strip, optionally res = rhs - Au; three wavefronts per 64-node tile: wavefront
 // p loads y-plane p's 81 coefficients (coalesced 256-byte runs over the
 // tile) and 27 vector entries and forms its 27 block terms (the expression
 // of row_product_t); planes 1 and 2 hand their terms to wavefront 0 through
 // LDS, which adds all 27 terms in row_product_t's sequential order, so the
-// result has the same bits as k_matvec's while three planes' loads are in
+// result has the reference's bits while three planes' loads are in
 // flight at once.  Four wavefronts a SIMD: at most 128 registers (FP64 needs 129
 // left alone, and ran three).
 template <typename V, typename KT, bool STREAM>
@@ -451,7 +404,7 @@ __global__ void __launch_bounds__(192, 4) k_matvec3(Geo g, const KT *__restrict_
 
 // The same product with all three planes' coefficients and vector entries
 // loaded before the first addition (one memory round trip instead of
-// three; the sums keep row_product's order).  For small levels, whose
+// three; the sums keep row_product_t's order).  For small levels, whose
 // matvec is latency-bound: 243 + 81 live values per thread, one wavefront
 // per workgroup.
 template <typename V>
@@ -1109,7 +1062,7 @@ __global__ void __launch_bounds__(SMALL_TPB) k_gs_lds(Geo g, const float *__rest
             __syncthreads();
         }
     }
-    // Ad = K d in row_product's sequential order, BC rows stripped
+    // Ad = K d in row_product_t's sequential order, BC rows stripped
     for (int cq = tid; Ad && cq < nno; cq += blockDim.x) {
         const int n = nb[cq * 27 + 13];
         double out[3] = {0.0, 0.0, 0.0};
@@ -1195,7 +1148,7 @@ void gs_small(hipStream_t s, const Level &L, double *d, const double *F, double 
 // register); if they do not, or a poll runs past its limit, the launch stops
 // early and writes a nonzero status (2: not on one XCD, 1: poll limit) for
 // the host, which reports the multigrid call as failed.  Then Ad = K d in
-// row_product's order (and res = rhs - Ad), as after the per-colour passes.
+// row_product_t's order (and res = rhs - Ad), as after the per-colour passes.
 
 __device__ __forceinline__ unsigned xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | 20); }
 

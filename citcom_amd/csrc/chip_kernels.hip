@@ -729,6 +729,23 @@ struct RectLane {
     }
 };
 
+// the plane staged for plane j beside a workgroup's own: past the mesh, where
+// its entries count as zero, the plane on the other side, since the own plane's
+// buffer may be the one being written (dout, in the odd planes' launch)
+__host__ __device__ constexpr int rect_side(int j, int noy) { return j < 0 ? 1 : j >= noy ? noy - 2 : j; }
+
+// no launch stages a plane that it writes, beside its own
+constexpr bool rect_side_clear(int most) {
+    for (int noy = 2; noy <= most; noy++)
+        for (int j = 0; j < noy; j++)
+            for (int d = -1; d <= 1; d += 2) {
+                const int s = rect_side(j + d, noy);
+                if (s < 0 || s >= noy || (s - j) % 2 == 0) return false;
+            }
+    return true;
+}
+static_assert(rect_side_clear(16), "the joined passes' side planes");
+
 // the packed coefficients of wavefront w of workgroup (seg, strip, j)
 template <class S>
 __device__ __forceinline__ size_t rect_wave(const RectPart &rp, int seg, int strip, int j, int w) {
@@ -777,7 +794,7 @@ __global__ void __launch_bounds__(S::WAVES * 64, sizeof(V) == 8 || sizeof(KT) ==
 #pragma unroll
     for (int q = 0; q < S::BATCH; q++) {
         const int ln = min(w + q / S::CH * S::WAVES, 3 * NL - 1), pl = ln / NL;
-        const int gi = min(max(i0 - 1 + ln - pl * NL, 0), g.nox - 1), gj = min(max(j + pl - 1, 0), g.noy - 1);
+        const int gi = min(max(i0 - 1 + ln - pl * NL, 0), g.nox - 1), gj = rect_side(j + pl - 1, g.noy);
         const int gk = min(max(kr0 + q % S::CH * 21 + l3, 0), g.noz - 1);
         stage[q] = (pl == 1 ? same : side)[3 * nid(g, gk, gi, gj) + comp];
     }

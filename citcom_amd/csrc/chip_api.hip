@@ -1142,6 +1142,21 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
         CHIP_CHECK(up(b, in2, nv));
         affine_apply(q, L, guess ? (const double *)a : nullptr, (const double *)b, L.tmp);
         CHIP_CHECK(down(out, L.tmp, nv));
+    } else if (o == "up" || o == "up_f32") {
+        if (!L.Mu || (o == "up_f32" && !L.velf)) {
+            set_error(o + ": the level above the coarsest, where its way up is a matrix (\"up_f32\": in the FP32 cycles of a mixed form)");
+            return -1;
+        }
+        CHIP_CHECK(up(b, in2, nv));
+        if (o == "up") {
+            up_apply(q, L, (const double *)b, a);
+        } else {
+            to_f32(q, L.resf, b, nv);
+            up_apply(q, L, (const float *)L.resf, L.delf);
+            fill(q, a, 0.0, nv);
+            add_f32(q, a, L.delf, nv);
+        }
+        CHIP_CHECK(down(out, a, nv));
     } else if (o == "direct") {
         if (lev != c->dlev || !c->direct_ok) {
             set_error("direct: the level solved exactly by the FP32 cycles, after a rebuild");

@@ -74,7 +74,7 @@ struct XcdBar {
     unsigned pad;
 };
 
-// the maps of a level, in the order Ma, Mb, Mu
+// the maps of a level, in the order Ma, Mb, Mu, and the first two's FP32 copies
 struct MapSet {
     double *m[3];
     float *f[3];
@@ -111,7 +111,7 @@ struct Level {
     // coarsest also the way up from a residual, Mu; scratch vectors for the
     // result in both precisions
     double *Ma = nullptr, *Mb = nullptr, *Mu = nullptr;
-    float *Maf = nullptr, *Mbf = nullptr, *Muf = nullptr;   // FP32 copies for the FP32 cycles (mixed forms)
+    float *Maf = nullptr, *Mbf = nullptr;   // FP32 copies for the FP32 cycles (mixed forms); Mu, which holds the FP64 Mc, has none
     int affine_sweeps = 0;
     double *tmp = nullptr;
     float *tmpf = nullptr;

@@ -1941,7 +1941,7 @@ int coarse_build(hipStream_t s, const Level &L, int sweeps) {
 }
 
 int affine_build(hipStream_t s, const Level &L, const Level &coarse) {
-    const MapSet ms{{L.Ma, L.Mb, L.Mu}, {L.Maf, L.Mbf, L.Muf}};
+    const MapSet ms{{L.Ma, L.Mb, L.Mu}, {L.Maf, L.Mbf, nullptr}};
     if (L.Mu)
         hipLaunchKernelGGL(k_map_restrict, dim3(nblk(3L * L.g.nno), std::min(3 * coarse.g.nno, 64)), dim3(256), 0, s, L.g,
                            coarse.g, coarse.TWW, coarse.MASS, coarse.NODE, coarse.Mc, L.Mu);
@@ -2004,14 +2004,11 @@ void affine_apply(hipStream_t s, const Level &L, const V *din, const V *F, V *ou
 template void affine_apply<double>(hipStream_t, const Level &, const double *, const double *, double *);
 template void affine_apply<float>(hipStream_t, const Level &, const float *, const float *, float *);
 
-// the way up to the level above the coarsest: out = Mu res
+// the way up to the level above the coarsest: out = Mu res.  FP64 in the FP32
+// cycles too: its sums hold the coarsest level's call, whose matrix is FP64.
 template <typename V>
 void up_apply(hipStream_t s, const Level &L, const V *res, V *out) {
-    const int n3 = 3 * L.g.nno;
-    if (sizeof(V) == 4 && L.Muf)
-        map_apply<V, float>(s, nullptr, L.Muf, nullptr, res, out, n3);
-    else
-        map_apply<V, double>(s, nullptr, L.Mu, nullptr, res, out, n3);
+    map_apply<V, double>(s, nullptr, L.Mu, nullptr, res, out, 3 * L.g.nno);
 }
 template void up_apply<double>(hipStream_t, const Level &, const double *, double *);
 template void up_apply<float>(hipStream_t, const Level &, const float *, float *);

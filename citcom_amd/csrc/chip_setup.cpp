@@ -467,9 +467,7 @@ int build_mesh(chip_ctx *c) {
                 (p.mixed && (dev_alloc(c, &A.Maf, n3 * n3) || dev_alloc(c, &A.Mbf, n3 * n3))) ||
                 dev_alloc(c, &A.tmpf, n3))
                 return -1;
-            if (!exact && lev == c->levmin + 1 &&
-                (dev_alloc(c, &A.Mu, n3 * n3) || (p.mixed && dev_alloc(c, &A.Muf, n3 * n3))))
-                return -1;
+            if (!exact && lev == c->levmin + 1 && dev_alloc(c, &A.Mu, n3 * n3)) return -1;
             A.affine_sweeps = p.down_heavy;
         }
     }

@@ -285,7 +285,7 @@ class Citcom:
         """Single operator on host arrays (see chip_apply in include/citcom_hip.h)."""
         n3, ne = 3 * self.nno(lev), self.nel(lev)
         out_n = {"matvec": n3, "gs0": n3, "gs1": n3, "box0": n3, "box1": n3, "coarse": n3, "direct": n3,
-                 "affine0": n3, "affine1": n3,
+                 "affine0": n3, "affine1": n3, "up": n3, "up_f32": n3,
                  "div": ne, "grad": n3,
                  "strip": n3, "cnet": n3,
                  "project": 3 * self.nno(lev - 1) if lev > 0 else 0, "interp": n3}[op]
@@ -294,7 +294,7 @@ class Citcom:
         n_in = {"matvec": n3, "gs1": n3, "box1": n3, "affine1": n3, "div": n3, "grad": ne, "strip": n3,
                 "project": n3, "interp": 3 * self.nno(lev - 1) if lev > 0 else 0}.get(op, 0)
         n_in2 = {"gs0": n3, "gs1": n3, "box0": n3, "box1": n3, "coarse": n3, "direct": n3, "affine0": n3, "affine1": n3,
-                 "cnet": n3}.get(op, 0)
+                 "up": n3, "up_f32": n3, "cnet": n3}.get(op, 0)
         for name, arr, need in (("x", x, n_in), ("x2", x2, n_in2)):
             if need and (arr is None or np.size(arr) != need):
                 raise ChipError(f"apply {op}: {name} needs {need} values, got "

@@ -1095,6 +1095,23 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
     auto down = [&](double *dst, const double *src, long n) {
         return hipMemcpyAsync(dst, src, n * 8, hipMemcpyDeviceToHost, q);
     };
+    // the FP32 cycles' vectors of the level, from and to host doubles through a stage
+    float *af = L.delf, *bf = L.resf, *df = L.AUf;
+    auto up32 = [&](float *dst, double *stage, const double *src) {
+        const hipError_t e = up(stage, src, nv);
+        to_f32(q, dst, stage, nv);
+        return e;
+    };
+    auto down32 = [&](double *dst, double *stage, const float *src) {
+        fill(q, stage, 0.0, nv);
+        add_f32(q, stage, src, nv);
+        return down(dst, stage, nv);
+    };
+    const bool f32 = o.size() > 4 && o.compare(o.size() - 4, 4, "_f32") == 0;
+    if (f32 && !L.velf) {
+        set_error(o + ": the FP32 cycles of a mixed form");
+        return -1;
+    }
     if (o == "matvec") {
         CHIP_CHECK(up(a, in, nv));
         do_matvec(c, lev, a, b);
@@ -1107,6 +1124,18 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
         CHIP_CHECK(down(out, a, nv));
         CHIP_CHECK(down(out2, d, nv));
         if (sync_dots(c) || xcd_status(c)) return -1;
+    } else if (o == "matvec_f32") {
+        CHIP_CHECK(up32(af, a, in));
+        do_matvec(c, lev, (const float *)af, bf);
+        CHIP_CHECK(down32(out, b, bf));
+    } else if (o == "gs0_f32" || o == "gs1_f32") {   // as the FP32 cycles' sweeps, the options' kernels
+        const int guess = (o == "gs1_f32");
+        if (guess) CHIP_CHECK(up32(af, a, in));
+        CHIP_CHECK(up32(bf, b, in2));
+        do_gs(c, lev, af, (const float *)bf, df, arg, guess);
+        CHIP_CHECK(down32(out, a, af));
+        CHIP_CHECK(down32(out2, d, df));
+        if (sync_dots(c) || xcd_status(c)) return -1;
     } else if (o == "box0" || o == "box1") {   // FP32 box smoother call: arg sweeps, then Ad = K d
         if (!L.Kbox || !L.velf) {
             set_error("box: the level has no box smoother (FP32 cycles of a mixed form, levels between the "
@@ -1114,27 +1143,19 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
             return -1;
         }
         const int guess = (o == "box1");
-        float *af = L.delf, *bf = L.resf, *df = L.AUf;
-        if (guess) {
-            CHIP_CHECK(up(a, in, nv));
-            to_f32(q, af, a, nv);
-        }
-        CHIP_CHECK(up(b, in2, nv));
-        to_f32(q, bf, b, nv);
+        if (guess) CHIP_CHECK(up32(af, a, in));
+        CHIP_CHECK(up32(bf, b, in2));
         const bool keep = c->box_gs;
         c->box_gs = true;
         do_gs(c, lev, af, (const float *)bf, df, arg, guess);
         c->box_gs = keep;
-        fill(q, a, 0.0, nv);
-        add_f32(q, a, af, nv);
-        fill(q, d, 0.0, nv);
-        add_f32(q, d, df, nv);
-        CHIP_CHECK(down(out, a, nv));
-        CHIP_CHECK(down(out2, d, nv));
+        CHIP_CHECK(down32(out, a, af));
+        CHIP_CHECK(down32(out2, d, df));
         CHIP_CHECK(hipStreamSynchronize(q));
     } else if (o == "affine0" || o == "affine1") {
         if (!L.Ma || lev != c->levmin + 1 || !affine_ok(L)) {
-            set_error("affine: the level has no affine smoother form");
+            set_error("affine: the level right above the coarsest, of at most 1500 unknowns, where its smoother call is a "
+                      "matrix (\"map0\", \"map1\": any level whose call is one)");
             return -1;
         }
         const int guess = (o == "affine1");
@@ -1142,21 +1163,37 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
         CHIP_CHECK(up(b, in2, nv));
         affine_apply(q, L, guess ? (const double *)a : nullptr, (const double *)b, L.tmp);
         CHIP_CHECK(down(out, L.tmp, nv));
-    } else if (o == "up" || o == "up_f32") {
-        if (!L.Mu || (o == "up_f32" && !L.velf)) {
-            set_error(o + ": the level above the coarsest, where its way up is a matrix (\"up_f32\": in the FP32 cycles of a mixed form)");
+    } else if (o == "map0" || o == "map1" || o == "map0_f32" || o == "map1_f32") {
+        if (!L.Ma) {
+            set_error(o + ": the level's smoother call is not a matrix");
             return -1;
         }
-        CHIP_CHECK(up(b, in2, nv));
-        if (o == "up") {
-            up_apply(q, L, (const double *)b, a);
+        const int guess = o[3] == '1';
+        if (f32) {
+            if (guess) CHIP_CHECK(up32(af, a, in));
+            CHIP_CHECK(up32(bf, b, in2));
+            affine_apply(q, L, guess ? (const float *)af : nullptr, (const float *)bf, L.tmpf);
+            CHIP_CHECK(down32(out, a, L.tmpf));
         } else {
-            to_f32(q, L.resf, b, nv);
-            up_apply(q, L, (const float *)L.resf, L.delf);
-            fill(q, a, 0.0, nv);
-            add_f32(q, a, L.delf, nv);
+            if (guess) CHIP_CHECK(up(a, in, nv));
+            CHIP_CHECK(up(b, in2, nv));
+            affine_apply(q, L, guess ? (const double *)a : nullptr, (const double *)b, L.tmp);
+            CHIP_CHECK(down(out, L.tmp, nv));
         }
-        CHIP_CHECK(down(out, a, nv));
+    } else if (o == "up" || o == "up_f32") {
+        if (!L.Mu) {
+            set_error(o + ": the level above the coarsest, where its way up is a matrix");
+            return -1;
+        }
+        if (f32) {
+            CHIP_CHECK(up32(bf, b, in2));
+            up_apply(q, L, (const float *)bf, af);
+            CHIP_CHECK(down32(out, a, af));
+        } else {
+            CHIP_CHECK(up(b, in2, nv));
+            up_apply(q, L, (const double *)b, a);
+            CHIP_CHECK(down(out, a, nv));
+        }
     } else if (o == "direct") {
         if (lev != c->dlev || !c->direct_ok) {
             set_error("direct: the level solved exactly by the FP32 cycles, after a rebuild");

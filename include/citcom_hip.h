@@ -125,9 +125,13 @@ int chip_construct_stiffness_B_matrix(chip_ctx *c);
  *     "affine0"/"affine1" (the level above) its multigrid smoother call
  *         (down_heavy sweeps) as an affine map: out = Mb in2 (zero guess) or
  *         Ma in + Mb in2
+ *     "map0"/"map1" (levels whose multigrid smoother call is a matrix) the
+ *         same on any such level
  *     "up" (the level above the coarsest, where the multigrid's way up from
- *         the coarsest level to it is a matrix of its residual) out = Mu in2;
- *         "up_f32" (mixed forms) the same as the FP32 cycles apply it
+ *         the coarsest level to it is a matrix of its residual) out = Mu in2
+ *     "matvec_f32", "gs0_f32"/"gs1_f32", "map0_f32"/"map1_f32", "up_f32"
+ *         (mixed forms) these as the FP32 cycles apply them, vectors rounded
+ *         to FP32; the smoother under the options set
  *     "cnet" (coarsest level) the learned coarse-level correction for the
  *         right-hand side in2 (after chip_set_coarse_net)
  *     "direct" (the level the FP32 cycles solve exactly, mixed forms, after

@@ -1837,11 +1837,16 @@ __global__ void __launch_bounds__(256) k_map_restrict(Geo gf, Geo gc, const floa
 // Map blockIdx.y + kind0 (0: Ma, 1: Mb, 2: Mu, whose first rows hold X on
 // entry), columns blockIdx.x NC ..: a level of one colour pass after the
 // other, each thread the three rows of a (node, column), in the order of
-// k_gs_colour.
+// k_gs_colour.  The kinds below `rounded` take the increments rounded to FP32,
+// as the reference's sweeps do (Mc, and Ma and Mb of at most AFFINE_MAX_DOF
+// unknowns); the others are the call in FP64, since a map of columns with
+// rounded increments may be further from it than the sweeps are (729 nodes,
+// three sweeps from a random guess: 3.0e-8, the sweeps 2.0e-8).
 template <int NC>
 __global__ void __launch_bounds__(1024) k_map_columns(Geo g, Geo gc, const float *__restrict__ K,
                                                       const double *__restrict__ BI, const float *__restrict__ iw,
-                                                      const unsigned *__restrict__ NODE, int sweeps, int kind0, MapSet ms) {
+                                                      const unsigned *__restrict__ NODE, int sweeps, int kind0, int rounded,
+                                                      MapSet ms) {
     extern __shared__ __align__(16) unsigned char smem[];
     double *ds = (double *)smem;   // [nno][3][NC], a node's run MAP_PAD longer against bank conflicts
     constexpr int ST = 3 * NC + MAP_PAD;
@@ -1898,7 +1903,8 @@ __global__ void __launch_bounds__(1024) k_map_columns(Geo g, Geo gc, const float
 #pragma unroll
                 for (int r = 0; r < 3; r++) {
                     const double F = kind != 0 && 3 * self + r == j0 + col ? 1.0 : 0.0;
-                    u[r * NC] += (float)((F - o[r]) * BI[3 * self + r]);
+                    const double t = (F - o[r]) * BI[3 * self + r];
+                    u[r * NC] += kind < rounded ? (double)(float)t : t;
                 }
             }
             __syncthreads();
@@ -1914,7 +1920,8 @@ __global__ void __launch_bounds__(1024) k_map_columns(Geo g, Geo gc, const float
 }
 
 // as many columns a workgroup as its LDS takes
-static int map_columns(hipStream_t s, const Level &L, const Geo &gc, int sweeps, int kind0, int kinds, const MapSet &ms) {
+static int map_columns(hipStream_t s, const Level &L, const Geo &gc, int sweeps, int kind0, int kinds, int rounded,
+                       const MapSet &ms) {
     const int n3 = 3 * L.g.nno;
     auto launch = [&](auto kern, int nc) {
         const size_t lds = (size_t)L.g.nno * (3 * nc + MAP_PAD) * 8;
@@ -1922,7 +1929,7 @@ static int map_columns(hipStream_t s, const Level &L, const Geo &gc, int sweeps,
         if (lds > 65536 && hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
             return false;
         hipLaunchKernelGGL(kern, dim3((n3 + nc - 1) / nc, kinds), dim3(1024), lds, s, L.g, gc, L.K, L.BI, L.iw, L.NODE,
-                           sweeps, kind0, ms);
+                           sweeps, kind0, rounded, ms);
         return true;
     };
     if (launch(k_map_columns<8>, 8) || launch(k_map_columns<4>, 4) || launch(k_map_columns<1>, 1)) return 0;
@@ -1937,7 +1944,7 @@ int coarse_build(hipStream_t s, const Level &L, int sweeps) {
                            L.K, L.BI, L.NODE, L.Mc, nullptr, nullptr, sweeps, 0, 1);
         return 0;
     }
-    return map_columns(s, L, L.g, sweeps, 1, 1, MapSet{{nullptr, L.Mc, nullptr}, {}});
+    return map_columns(s, L, L.g, sweeps, 1, 1, 2, MapSet{{nullptr, L.Mc, nullptr}, {}});
 }
 
 int affine_build(hipStream_t s, const Level &L, const Level &coarse) {
@@ -1945,7 +1952,7 @@ int affine_build(hipStream_t s, const Level &L, const Level &coarse) {
     if (L.Mu)
         hipLaunchKernelGGL(k_map_restrict, dim3(nblk(3L * L.g.nno), std::min(3 * coarse.g.nno, 64)), dim3(256), 0, s, L.g,
                            coarse.g, coarse.TWW, coarse.MASS, coarse.NODE, coarse.Mc, L.Mu);
-    return map_columns(s, L, coarse.g, L.affine_sweeps, 0, L.Mu ? 3 : 2, ms);
+    return map_columns(s, L, coarse.g, L.affine_sweeps, 0, L.Mu ? 3 : 2, affine_ok(L) ? 2 : 0, ms);
 }
 
 // out = A din + B F (A may be null): LANES lanes a row; lane t sums A's terms

@@ -135,12 +135,17 @@ template <typename V>
 void do_gs(chip_ctx *c, int lev, V *d, const V *F, V *Ad, int sweeps, int guess, const V *rhs = nullptr,
            V *res = nullptr);
 
+// the level's smoother call of multi_grid is applied as a matrix
+bool has_map(const chip_ctx *c, const Level &L) {
+    return L.Ma && c->small_levels && (c->const_maps || !L.const_map);
+}
+
 // a smoother call of multi_grid: the affine form where the level has one
 template <typename V>
 void mg_gs(chip_ctx *c, int lev, V *d, const V *F, V *Ad, int sweeps, int guess, const V *rhs = nullptr,
            V *res = nullptr) {
     const Level &L = c->L[lev];
-    if (L.Ma && c->small_levels && sweeps == L.affine_sweeps) {
+    if (has_map(c, L) && sweeps == L.affine_sweeps) {
         V *out = d;
         if (guess == 1) {
             if constexpr (sizeof(V) == sizeof(double)) out = L.tmp;
@@ -255,7 +260,7 @@ void enqueue_cycles(chip_ctx *c, V *F) {
             coarse_smooth(c, vel, rhs);
     };
     // the way up to the level above the coarsest as one matrix of its residual
-    const bool joined = !direct && !c->cnet_on && c->small_levels && L[levmin + 1].Mu;
+    const bool joined = !direct && !c->cnet_on && L[levmin + 1].Mu && has_map(c, L[levmin + 1]);
     for (int lev = levmax; lev > levmin; lev--) project(S(c), L[lev], L[lev - 1], (const V *)fl(lev), fl(lev - 1));
     bottom(vecs<V>(L[levmin]).vel, (const V *)fl(levmin));
     for (int lev = levmin + 1; lev <= levmax; lev++) {
@@ -661,6 +666,12 @@ int direct_factor(chip_ctx *c) {
     return (c->direct_ok != was) ? drop_mg_graph(c) : 0;
 }
 
+// the finest viscosity from the context's law
+void system_viscosity(chip_ctx *c) {
+    visc_from_T(S(c), c, c->T, c->L[c->levmax].EVI);
+    c->evi_varies = false;
+}
+
 int rebuild(chip_ctx *c) {
     hipStream_t q = S(c);
     // a side-stream factorization still reading the stiffness finishes
@@ -677,8 +688,14 @@ int rebuild(chip_ctx *c) {
     for (int lev = c->levmax; lev >= c->levmin; lev--) build_bpi(q, c->L[lev], c->p.precond);
     if (c->cnet_w) cnet_logeta(q, c->L[c->levmin], c->cnet_logeta);
     if (c->L[c->levmin].Mc && coarse_build(q, c->L[c->levmin], c->p.v_steps_low)) return -1;
-    for (int lev = c->levmin; lev <= c->levmax; lev++)
-        if (c->L[lev].Ma && affine_build(q, c->L[lev], c->L[lev - 1])) return -1;
+    if (c->const_maps == c->evi_varies) {   // the captured kernel sequence changes
+        if (drop_mg_graph(c)) return -1;
+        c->const_maps = !c->evi_varies;
+    }
+    for (int lev = c->levmin; lev <= c->levmax; lev++) {
+        const Level &L = c->L[lev];
+        if (L.Ma && (c->const_maps || !L.const_map) && affine_build(q, L, c->L[lev - 1])) return -1;
+    }
     if (c->p.mixed)
         for (int lev = c->levmin; lev <= c->levmax; lev++) to_f32(q, c->L[lev].BIf, c->L[lev].BI, 3L * c->L[lev].g.nno);
     for (int lev = c->levmin; lev <= c->levmax; lev++)
@@ -844,7 +861,7 @@ int stokes_step(chip_ctx *c, chip_stokes_stats *st) {
     // get_system_viscosity + construct_stiffness_B_matrix (Drive_solvers.c:123-126);
     // the viscosity first, so that the warm start reads this step's
     const bool update = !c->built || c->p.visc_update;
-    if (update) visc_from_T(q, c, c->T, c->L[c->levmax].EVI);
+    if (update) system_viscosity(c);
     if (warm_start_guess(c)) return -1;
     conform_velocity(q, L, c->U);
     assemble_forces(q, c, c->buoy, c->F);
@@ -1004,6 +1021,10 @@ int chip_upload(chip_ctx *c, const char *which, int lev, const void *host, long 
     Level &L = c->L[lev < 0 ? c->levmax : lev];
     if (ptr == L.GNX || ptr == L.GDA || ptr == L.ECO) return check_brick(c, L);
     if (ptr == L.EG) L.eg_brick = false;
+    if (ptr == c->L[c->levmax].EVI) {   // for the next rebuild's choice of maps
+        const float *v = static_cast<const float *>(host);
+        c->evi_varies = std::any_of(v + 1, v + n, [v](float x) { return x != v[0]; });
+    }
     return 0;
 }
 
@@ -1059,7 +1080,7 @@ int chip_download(chip_ctx *c, const char *which, int lev, void *host, long coun
 
 int chip_get_system_viscosity(chip_ctx *c) {
     CHIP_NEED_CTX(c);
-    visc_from_T(c->stream, c, c->T, c->L[c->levmax].EVI);
+    system_viscosity(c);
     CHIP_CHECK(hipGetLastError());
     return 0;
 }
@@ -1164,7 +1185,7 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
         affine_apply(q, L, guess ? (const double *)a : nullptr, (const double *)b, L.tmp);
         CHIP_CHECK(down(out, L.tmp, nv));
     } else if (o == "map0" || o == "map1" || o == "map0_f32" || o == "map1_f32") {
-        if (!L.Ma) {
+        if (!L.Ma || (L.const_map && !c->const_maps)) {
             set_error(o + ": the level's smoother call is not a matrix");
             return -1;
         }
@@ -1181,7 +1202,7 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
             CHIP_CHECK(down(out, L.tmp, nv));
         }
     } else if (o == "up" || o == "up_f32") {
-        if (!L.Mu) {
+        if (!L.Mu || (L.const_map && !c->const_maps)) {
             set_error(o + ": the level above the coarsest, where its way up is a matrix");
             return -1;
         }

@@ -449,13 +449,13 @@ int build_mesh(chip_ctx *c) {
         // the levels above: affine form when their two smoother calls in
         // multi_grid use the same number of sweeps.  Cycles that stop at a
         // level solved exactly reach them only where that is switched off:
-        // there, the level above the coarsest only, and not its way up
         // there, the level above the coarsest only, and not its way up.  The
         // sweeps' FP32 increments, which the maps do not round, move the
         // solution by 2e-11 at constant viscosity (28 solves), but by up to
         // 1.5e-9 in the pressure at the 64^3 workload's contrast of 10^4 (one
         // solve in thirty; the median 1e-11): FP64 cycles with varying
-        // viscosity keep the sweeps above AFFINE_MAX_DOF
+        // viscosity keep the sweeps above AFFINE_MAX_DOF, by the law here and
+        // where a viscosity is uploaded by what it holds (const_map)
         bool constant = !p.tdepv;
         for (int m = 1; m < p.num_mat; m++) constant = constant && p.visc0[m] == p.visc0[0];
         const bool exact = p.mixed && c->levmin + 2 < c->levmax && 3L * c->L[c->levmin + 2].g.nno <= DIRECT_MAX_DOF;
@@ -469,6 +469,7 @@ int build_mesh(chip_ctx *c) {
                 return -1;
             if (!exact && lev == c->levmin + 1 && dev_alloc(c, &A.Mu, n3 * n3)) return -1;
             A.affine_sweeps = p.down_heavy;
+            A.const_map = !p.mixed && !affine_ok(A);
         }
     }
     // the FP32 cycles' exact coarsest-level solve: the largest level of at

@@ -137,7 +137,7 @@ void do_gs(chip_ctx *c, int lev, V *d, const V *F, V *Ad, int sweeps, int guess,
 
 // the level's smoother call of multi_grid is applied as a matrix
 bool has_map(const chip_ctx *c, const Level &L) {
-    return L.Ma && c->small_levels && (c->const_maps || !L.const_map);
+    return L.Ma && c->small_levels && (c->const_maps || !L.const_map) && !(c->maps_stale && L.wide);
 }
 
 // a smoother call of multi_grid: the affine form where the level has one
@@ -260,7 +260,7 @@ void enqueue_cycles(chip_ctx *c, V *F) {
             coarse_smooth(c, vel, rhs);
     };
     // the way up to the level above the coarsest as one matrix of its residual
-    const bool joined = !direct && !c->cnet_on && L[levmin + 1].Mu && has_map(c, L[levmin + 1]);
+    const bool joined = !direct && !c->cnet_on && L[levmin + 1].Mu && !c->maps_stale && has_map(c, L[levmin + 1]);
     for (int lev = levmax; lev > levmin; lev--) project(S(c), L[lev], L[lev - 1], (const V *)fl(lev), fl(lev - 1));
     bottom(vecs<V>(L[levmin]).vel, (const V *)fl(levmin));
     for (int lev = levmin + 1; lev <= levmax; lev++) {
@@ -688,8 +688,9 @@ int rebuild(chip_ctx *c) {
     for (int lev = c->levmax; lev >= c->levmin; lev--) build_bpi(q, c->L[lev], c->p.precond);
     if (c->cnet_w) cnet_logeta(q, c->L[c->levmin], c->cnet_logeta);
     if (c->L[c->levmin].Mc && coarse_build(q, c->L[c->levmin], c->p.v_steps_low)) return -1;
-    if (c->const_maps == c->evi_varies) {   // the captured kernel sequence changes
+    if (c->maps_stale || c->const_maps == c->evi_varies) {   // the captured kernel sequence changes
         if (drop_mg_graph(c)) return -1;
+        c->maps_stale = false;
         c->const_maps = !c->evi_varies;
     }
     for (int lev = c->levmin; lev <= c->levmax; lev++) {
@@ -1021,6 +1022,11 @@ int chip_upload(chip_ctx *c, const char *which, int lev, const void *host, long 
     Level &L = c->L[lev < 0 ? c->levmax : lev];
     if (ptr == L.GNX || ptr == L.GDA || ptr == L.ECO) return check_brick(c, L);
     if (ptr == L.EG) L.eg_brick = false;
+    // what the sweeps and transfers read as it is, the maps as the last rebuild found it
+    if (!c->maps_stale && (ptr == L.BI || ptr == L.NODE || ptr == L.MASS || ptr == L.TWW)) {
+        if (drop_mg_graph(c)) return -1;
+        c->maps_stale = true;
+    }
     if (ptr == c->L[c->levmax].EVI) {   // for the next rebuild's choice of maps
         const float *v = static_cast<const float *>(host);
         c->evi_varies = std::any_of(v + 1, v + n, [v](float x) { return x != v[0]; });
@@ -1185,7 +1191,7 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
         affine_apply(q, L, guess ? (const double *)a : nullptr, (const double *)b, L.tmp);
         CHIP_CHECK(down(out, L.tmp, nv));
     } else if (o == "map0" || o == "map1" || o == "map0_f32" || o == "map1_f32") {
-        if (!L.Ma || (L.const_map && !c->const_maps)) {
+        if (!L.Ma || (L.const_map && !c->const_maps) || (L.wide && c->maps_stale)) {
             set_error(o + ": the level's smoother call is not a matrix");
             return -1;
         }
@@ -1202,7 +1208,7 @@ int chip_apply(chip_ctx *c, const char *op, int lev, const double *in, const dou
             CHIP_CHECK(down(out, L.tmp, nv));
         }
     } else if (o == "up" || o == "up_f32") {
-        if (!L.Mu || (L.const_map && !c->const_maps)) {
+        if (!L.Mu || (L.const_map && !c->const_maps) || c->maps_stale) {
             set_error(o + ": the level above the coarsest, where its way up is a matrix");
             return -1;
         }

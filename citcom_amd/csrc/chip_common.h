@@ -113,6 +113,7 @@ struct Level {
     double *Ma = nullptr, *Mb = nullptr, *Mu = nullptr;
     float *Maf = nullptr, *Mbf = nullptr;   // FP32 copies for the FP32 cycles (mixed forms); Mu, which holds the FP64 Mc, has none
     int affine_sweeps = 0;
+    bool wide = false;       // a map of more than AFFINE_MAX_DOF unknowns, or of a level two above the coarsest or more
     bool const_map = false;  // only while the viscosity is one value (chip_ctx::const_maps)
     double *tmp = nullptr;
     float *tmpf = nullptr;
@@ -182,6 +183,7 @@ struct chip_ctx {
     bool built = false;      // operators constructed at least once
     bool evi_varies = false;  // the finest viscosity was uploaded and is not one value
     bool const_maps = true;   // levels with const_map use their maps: as the last rebuild found the viscosity
+    bool maps_stale = false;  // BI, NODE, MASS or TWW uploaded since the last rebuild: no wide map, no way up
     bool use_graphs = true;  // replay multi_grid as a captured HIP graph
     bool small_levels = true;  // small levels' own smoother kernels (k_gs_lds, k_gs_rect)
     bool gs_wg = true;         // joined colour passes on levels of at most SMALL_NNO nodes

@@ -469,6 +469,7 @@ int build_mesh(chip_ctx *c) {
                 return -1;
             if (!exact && lev == c->levmin + 1 && dev_alloc(c, &A.Mu, n3 * n3)) return -1;
             A.affine_sweeps = p.down_heavy;
+            A.wide = lev > c->levmin + 1 || !affine_ok(A);
             A.const_map = !p.mixed && !affine_ok(A);
         }
     }

@@ -2817,7 +2817,9 @@ __global__ void __launch_bounds__(64) k_brick(Geo g, const float *__restrict__ G
 #pragma unroll
         for (int q = 0; q < 4; q++) GB[(size_t)(BRICK_B + 4 * d + q) * g.nel + e] = b[q];
         // get_elt_g: -(derivative at the centre) x weight, rounded once
-        GB[(size_t)(BRICK_E + d) * g.nel + e] = (float)(gnx[192 + 8 * d + 6] * (double)(8.0f * gda[10]));
+        const float ed = (float)(gnx[192 + 8 * d + 6] * (double)(8.0f * gda[10]));
+        ok = ok && isfinite(ed);
+        GB[(size_t)(BRICK_E + d) * g.nel + e] = ed;
         GB[(size_t)(BRICK_SIZE + d) * g.nel + e] = eco[5 + d];
     }
 #pragma unroll

@@ -51,6 +51,11 @@ __device__ __forceinline__ bf16x4 load4(const uint16_t *p) {
     return a;
 }
 
+// 0, or -1 if HIP holds an error, which launch_error() then names (per thread);
+// the error is used up
+int ret();
+hipError_t launch_error();
+
 // 3x3x3 convolution of X[nb][nv][ci] with W[co][27][ci] (wtrans: W[ci][27][co]),
 // the tap's offset mirrored if asked (unet_kernels.hip); for operands that
 // conv_block_ok accepts, 0 or -1

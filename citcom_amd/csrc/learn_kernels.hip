@@ -145,7 +145,6 @@ __global__ void k_to_bf16(const float *__restrict__ a, uint16_t *__restrict__ b,
 }
 
 hipStream_t st(void *s) { return static_cast<hipStream_t>(s); }
-int ret() { return hipGetLastError() == hipSuccess ? 0 : -1; }
 
 // ---- the weight gradient's partial sums without a workspace argument: a
 // file-scope device array, one copy per GPU, held until the process ends.
@@ -250,8 +249,8 @@ int cl_conv3d_bwd_weight_noalloc(const uint16_t *x, const uint16_t *dy, int nb, 
     // every slot of partial sums that is summed is written in full before, so
     // nothing is cleared
     if (cl_conv3d_bwd_weight(x, dy, nb, nx, ny, nz, grad, part, stream) == 0) return 0;
-    const hipError_t e = hipGetLastError();
-    g_learn_err = std::string("cl_conv3d_bwd_weight_noalloc: ") + hipGetErrorString(e);
+    // sizes that fit the scratch array are refused by HIP only
+    g_learn_err = std::string("cl_conv3d_bwd_weight_noalloc: ") + hipGetErrorString(launch_error());
     return -1;
 }
 

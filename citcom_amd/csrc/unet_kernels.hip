@@ -286,6 +286,10 @@ bool aligned(const void *p, unsigned n) { return ((uintptr_t)p & (n - 1)) == 0; 
 
 namespace learn {
 
+thread_local hipError_t g_launch_err = hipSuccess;
+int ret() { return (g_launch_err = hipGetLastError()) == hipSuccess ? 0 : -1; }
+hipError_t launch_error() { return g_launch_err; }
+
 // the block kernel takes up to 64 input channels and pointers aligned to its
 // vector loads and stores
 bool conv_block_ok(int ci, const uint16_t *x, const uint16_t *w, const uint16_t *res, const uint16_t *y, const float *yf) {
@@ -766,7 +770,6 @@ __global__ void k_wmse(const float *__restrict__ Y, int ystride, const float *__
 }
 
 hipStream_t st(void *s) { return static_cast<hipStream_t>(s); }
-int ret() { return hipGetLastError() == hipSuccess ? 0 : -1; }
 unsigned nblk(long n) { return (unsigned)((n + 255) / 256); }
 bool chan_ok(int c) { return c >= 16 && c <= 256 && c % 16 == 0; }
 

@@ -1522,6 +1522,14 @@ int chip_set_option(chip_ctx *c, const char *name, int value) {
         return -1;
     }
     if (n == "coarse_net" && value) c->cnet_calibrated = false;   // the next solve calibrates it
+    if (n == "stream") {
+        if (value < -1 || value > 1) {
+            set_error("chip_set_option: stream is -1 (by size), 0 or 1");
+            return -1;
+        }
+        for (int lev = c->levmin; lev <= c->levmax; lev++) c->L[lev].stream = value;
+        return drop_mg_graph(c);
+    }
     if (n == "direct_async") {
         c->direct_async = value != 0;
         return 0;

@@ -123,6 +123,7 @@ struct Level {
     RectPart planes{};       // joined colour passes (k_gs_rect), and K and Kh packed for them
     float *Kr = nullptr;
     uint16_t *Krh = nullptr;
+    int stream = -1;         // coefficients read past the caches: 1, 0, or by their size (-1)
     // one-XCD smoother state (levels gs_xcd_ok accepts)
     XcdBar *xbar = nullptr;
     // box smoother of the FP32 cycles: the partition, and the cycle's

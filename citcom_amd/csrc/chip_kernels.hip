@@ -457,7 +457,9 @@ __device__ __forceinline__ void row_product_all(const Geo &g, const float *__res
 // (65x65x33 nodes, 136 MB: 7.4 -> 8.1 us, product 28 -> 33).
 constexpr double GS_STREAM = 256e6, MV_STREAM = 400e6;
 template <typename KT>
-static bool streamed(const Level &L, double limit) { return (double)L.g.pitch * KROW * sizeof(KT) > limit; }
+static bool streamed(const Level &L, double limit) {
+    return L.stream < 0 ? (double)L.g.pitch * KROW * sizeof(KT) > limit : L.stream != 0;
+}
 
 constexpr int MV_SMALL_NNO = 20000;   // levels up to this size use k_matvec_small
 

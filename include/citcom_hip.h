@@ -223,6 +223,9 @@ long chip_device_bytes(chip_ctx *c);
  * first on a side stream while the step's solve goes on with the previous
  * inverse (taken up at the next rebuild); 0 factors on the work stream and
  * uses the new inverse at once.
+ * "stream": -1 (default) reads the coefficients of levels of more than 256 MB
+ * of them (colour passes; products: 400 MB) past the caches, 1 of every
+ * level, 0 of none; results are identical.
  * "xcd_gs": 1 runs a whole gauss_seidel call on levels of 1025 to 6000
  * nodes as one launch of a few workgroups on one XCD, with barriers through
  * that XCD's L2 between the colour passes; 0 (default) launches one kernel

@@ -1450,8 +1450,10 @@ constexpr int BOX_TPB = 768;
 // A sweep, before (a y-plane of the three rows to each of three wavefronts, two
 // barriers a colour) -> now: 33x33x17 nodes in FP32 16.7 us -> 13.8, 17x17x17 in
 // FP16 14.0 -> 9.8; 65x65x33 in FP16 24.9 -> 24.4.  Bound by latency, eight
-// colours in turn, on 75 or 27 boxes for 256 CUs; the last, two boxes to a CU,
-// by the LDS reads and arithmetic of three times the lanes.
+// colours in turn, on 75 or 27 boxes for 256 CUs; on the last, 405 boxes of
+// which two share a CU, a wavefront waits for operands in 48 % of its cycles
+// and for its turn to issue in 38 % (vector instructions 37 % of the time, LDS
+// 29 %, of which 12 % bank conflicts).
 template <typename KT, bool ZIN>
 __global__ void __launch_bounds__(BOX_TPB, sizeof(KT) == 2 ? 6 : 3) k_gs_box(Geo g, BoxPart bp, const KT *__restrict__ Kb,
                                                     const float *__restrict__ BI, const float *__restrict__ F,
@@ -1778,7 +1780,10 @@ constexpr int MAP_PAD = 2;
 // Mb F from a zero guess; and on the level right above the coarsest the way up
 // (restriction, coarsest call, prolongation, call with that guess) is one
 // matrix of the residual, Mu = Ma (P Mc R) + Mb.  The columns are the smoother's
-// results for unit vectors, formed when the stiffness is rebuilt.
+// results for unit vectors, formed when the stiffness is rebuilt.  The FP32
+// cycles read Ma and Mb rounded to FP32, with FP64 sums: on 441 to 1089 nodes
+// 2.9e-8 to 4.5e-8 from the call in FP64, where FP32 sweeps are 4.6e-8 to
+// 7.4e-8; Mc and Mu, whose sums hold Mc's, stay FP64.
 //
 // A sweep of such a level is bound by latency (two launches of 8 us whatever
 // its size), a map by reading 8 n^2 bytes; the FP64 cycle, three sweeps: 405
@@ -2869,17 +2874,20 @@ struct ElemGeo {
 };
 
 // k_node_ks (below) from the compact geometry: three wavefronts per 64-node
-// tile, wavefront P the 81 coefficients of y-plane dy = P - 1 in registers,
-// through the two or four elements times two planes of elements that hold them
-// in ascending element order.  The same products and sums: with self the
+// tile, wavefront P the 81 coefficients of y-plane dy = P - 1, through the two or
+// four elements times two planes of elements that hold them in ascending element
+// order.  The same products and sums: with self the
 // node, m its neighbour, row r, column c, an element adds
 //   sum over the Gauss points of (W lo) hi, lo and hi the derivatives (self
 //   along c, m along r) of the node with the smaller and the larger local
 //   number, + the Laplacian term on the diagonal, + visc aug e e
 // (the reference forms one of each pair and transposes; a node's own block is
 // read transposed).  Elements outside the mesh have weight 0.
-// Bound by FP64 arithmetic (about 17000 operations a node); 128x128x64
-// elements, finest level 1.7 ms, from the arrays (one thread a node) 12 to 17.
+// Bound by waits: 256 registers, 148 more spilled (388 B of scratch a lane), two
+// wavefronts a SIMD that wait in 63 % of their cycles; vector instructions take
+// 47 % of the time, and the 17000 FP64 operations a node would take a seventh
+// at their full rate.  128x128x64 elements, finest level 1.7 ms, from the
+// arrays (one thread a node) 12 to 17.
 __global__ void __launch_bounds__(192, 2) k_node_ks_brick(Geo g, const float *__restrict__ GB, const float *__restrict__ EVI,
                                                           const unsigned *__restrict__ NODE, int aug_on, double aug,
                                                           float *__restrict__ K, double *__restrict__ BI) {

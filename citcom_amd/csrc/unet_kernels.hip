@@ -42,9 +42,13 @@ constexpr int TAPS = 27;
 // WREG: all 27 taps' weights in registers (one or two channel blocks), any
 // number of tiles per wavefront; else the weights of nine taps at a time in
 // LDS, the next nine in flight during the products, CONV_M tiles per wavefront.
-// Bound by the staging (a block's loads, then its products, two or four
-// workgroups to a CU) and, at 16 channels, by the LDS reads (512 B per MFMA
-// from four SIMDs).  129x129x65 nodes: 16 -> 16 channels 52 us (1.3 TB/s of
+// A workgroup stages, multiplies and stores in turn, two or four of them to a
+// CU.  At 16 -> 16 channels bound by the issue of vector instructions (indexes
+// of the staging and the outputs, rounding; an MFMA in seven): they take 65 %
+// of the time, LDS 39 % (18 % bank conflicts), MFMA 35 %.  At 32 -> 16 by waits
+// for the staged loads, two workgroups to a CU: 46 % of a wavefront's cycles
+// (vector instructions 40 %, LDS 31 %, MFMA 26 %).  129x129x65 nodes: 16 -> 16
+// channels 52 us (1.3 TB/s of
 // activations, 290 TFLOP/s), 32 -> 16 119 us; 65x65x33, 32 -> 32 25 us; with
 // 8-byte loads of both operands per MFMA and no staging (the general kernel
 // below) these took 228, 228 and 98 us.
@@ -392,8 +396,10 @@ __global__ void k_transpose_w(const uint16_t *__restrict__ W, int ci, int co, ui
 // the bias as a tap of ones, and writes them once into its slot.  A second
 // kernel sums the slots in a fixed order.
 //
-// Bound by the LDS reads (a tap's operand per MFMA, shared by the NOB output
-// blocks) and the staging.  65^3 nodes, batch 4: 16 x 16 channels 83 us and
+// Bound by waits for the staged loads, which few products hide: 55 % of a
+// wavefront's cycles at 16 x 16 channels, 59 % at 32 x 16 (vector instructions
+// 40 and 37 % of the time, LDS 18 and 22 %, MFMA 18 and 21 %).  65^3 nodes,
+// batch 4: 16 x 16 channels 83 us and
 // its slots' sum 8; with 2-byte loads of single voxels and a slot for 512
 // voxels these took 1715 and 502 us.
 typedef short s16x4 __attribute__((ext_vector_type(4)));

@@ -97,7 +97,11 @@ void *chip_get_stream(chip_ctx *c);
  * "F" double[3nno], "V" float[3*nno] (V[d*nno+n]), "buoyancy" float[nno],
  * "EVI" float[8*nel(lev)] (lev = -1: finest), "K" float[nno(lev)*243] row
  * layout [n][r*81 + slot*3 + c], slot = (dz+1)+3(dx+1)+9(dy+1),
- * "BI" double[3nno(lev)], "BPI" double[nel(lev)] */
+ * "BI" double[3nno(lev)], "BPI" double[nel(lev)].  An uploaded array counts
+ * from then on ("EVI" and the element arrays from the next rebuild): after an
+ * upload of "BI", "NODE", "MASS" or "TWW" the multigrid leaves out the
+ * matrices that hold them (option "small_levels"; those of at most 1500
+ * unknowns stand for the last rebuild) until the next rebuild. */
 int chip_upload(chip_ctx *c, const char *which, int lev, const void *host, long count);
 int chip_download(chip_ctx *c, const char *which, int lev, void *host, long count);
 
@@ -204,12 +208,16 @@ long chip_device_bytes(chip_ctx *c);
  * graph, 0 launches its kernels one by one; results are identical.
  * "small_levels": 1 (default) smooths levels whose stiffness fits in LDS in
  * one single-workgroup kernel per gauss_seidel call, and other levels of at
- * most about 36000 nodes in two launches per sweep (four colours each);
- * 0 launches one kernel per colour pass on every level; results are
- * identical.
+ * most about 36000 nodes in two launches per sweep (four colours each), with
+ * the bits of one launch per colour pass; and applies the multigrid's
+ * smoother calls of the coarsest level and of small levels above it (at most
+ * 1500 unknowns; 3300 in mixed forms without an exact level and, in the plain
+ * form, at a constant viscosity) as matrices, which differ from the sweeps by
+ * the FP32 rounding of the increments.  0 launches one kernel per colour pass
+ * on every level but those of "box_gs".
  * "gs_wg": 1 (default) joins the colour passes also on levels of at most
- * 1024 nodes; 0 launches one kernel per colour pass there; results are
- * identical.
+ * 1024 nodes (where the smoother's call is not a matrix); 0 launches one
+ * kernel per colour pass there; results are identical.
  * "coarse_direct": 1 (default) lets the FP32 cycles of the mixed forms
  * stop at the largest level below the finest with at most 8192 unknowns
  * and at least two levels below it (17x17x9 nodes at 128x128x64 elements)
@@ -228,16 +236,16 @@ long chip_device_bytes(chip_ctx *c);
  * level, 0 of none; results are identical.
  * "xcd_gs": 1 runs a whole gauss_seidel call on levels of 1025 to 6000
  * nodes as one launch of a few workgroups on one XCD, with barriers through
- * that XCD's L2 between the colour passes; 0 (default) launches one kernel
- * per colour pass there; results are identical.  Setting 1 first checks
+ * that XCD's L2 between the colour passes; 0 (default) smooths them as the
+ * other options say; results are identical.  Setting 1 first checks
  * that the device dispatches workgroups to its XCDs round-robin, and is
  * refused where it does not.
  * "box_gs": 1 (default) smooths the levels of the mixed forms' FP32 cycles
  * between the exact (or the affine) level and the finest, larger than 1024
  * nodes, by boxes of at most 8 nodes a side: one launch per sweep, a
  * workgroup per box running the 8 colour passes on its own nodes in LDS,
- * the other boxes' nodes as they were before the sweep; 0 launches one
- * kernel per colour pass there.  The iterates differ (a box's face sees its
+ * the other boxes' nodes as they were before the sweep; 0 smooths them by
+ * colour passes, as "small_levels" says.  The iterates differ (a box's face sees its
  * neighbour's values of the previous sweep); the solve still iterates to
  * the same criterion.
  * "profile_level": >= 0 restricts chip_profile_enable to that level's

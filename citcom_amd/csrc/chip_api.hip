@@ -1027,9 +1027,11 @@ int chip_upload(chip_ctx *c, const char *which, int lev, const void *host, long 
         if (drop_mg_graph(c)) return -1;
         c->maps_stale = true;
     }
-    if (ptr == c->L[c->levmax].EVI) {   // for the next rebuild's choice of maps
+    if (ptr == c->L[c->levmax].EVI) {   // for the next rebuild's choice of maps, where a level has the choice
         const float *v = static_cast<const float *>(host);
-        c->evi_varies = std::any_of(v + 1, v + n, [v](float x) { return x != v[0]; });
+        bool choice = false;
+        for (int l = c->levmin; l <= c->levmax; l++) choice = choice || c->L[l].const_map;
+        c->evi_varies = choice && std::any_of(v + 1, v + n, [v](float x) { return x != v[0]; });
     }
     return 0;
 }
